@@ -249,3 +249,33 @@ def test_decode_graph_replays(hip, be, orc, weights):
         d.dec.graph(P, False)
     finally:
         d.free()
+
+
+@pytest.mark.parametrize("oh,ow", [
+    (130, 517),   # three row chunks, three column chunks, odd row starts
+    (64, 256),    # exactly one workgroup
+    (65, 257),    # one row and one column into the next
+    (20, 30),     # downscaling: every row takes new source rows
+    (1, 3),       # no whole dword of mask bytes
+])
+def test_mask_post_tile_edges(hip, be, orc, weights, oh, ow):
+    """The resize kernel at the edges of its 256-column, 64-row tiles and at
+    unaligned row starts: masks and statistics bit-exact against the oracle,
+    a plane with NaN and infinite logits among them."""
+    G, P = 16, 1
+    d = Dec(hip, be, orc, weights, G, P, 50)
+    try:
+        L = 4 * G
+        low = np.random.default_rng(oh).standard_normal((P * 3, L, L)).astype(np.float32)
+        low[1] = np.abs(low[1]) * -1   # no pixel above zero: the empty box
+        low[2, 5, 7], low[2, 40, 3], low[2, 20, 60] = np.nan, np.inf, -np.inf
+        sel = np.array([2, 0, 1], np.int32)
+        be.write(d.dec.buf("lowres"), 0, low)
+        stats = d.dec.postprocess(sel, oh, ow, 0.3, False)
+        _, mask, want = orc.postprocess(low, sel, oh, ow, 0.3, False)
+        assert np.array_equal(stats, want), (stats, want)
+        for k in range(3):
+            got = d.dec.read_mask(k, oh, ow, 0, 0, ow - 1, oh - 1)
+            assert np.array_equal(got, mask[k])
+    finally:
+        d.free()
