@@ -363,6 +363,8 @@ void hipb_free(struct hipb_backend *b)
         hipStreamSynchronize((hipStream_t)b->stream);
     if (b->scratch)
         hipFree(b->scratch);
+    for (int i = 0; i < b->gemm_ws_count; i++)
+        hipFree(b->gemm_ws[i]);
     for (int i = 0; i < 2; i++) {
         if (b->stage[i])
             hipHostFree(b->stage[i]);
@@ -616,6 +618,42 @@ void *hipb_scratch(struct hipb_backend *b, size_t n)
     }
     b->scratch_bytes = n;
     return b->scratch;
+}
+
+/* Workspace of the exact path's GEMM (its split operands): at least n
+ * bytes, or NULL (the product then does without) when n is 0, when it cannot
+ * be had, or while the caller captures the stream: only the library's own
+ * graphs (b->capture), which run on this stream alone, may hold it, and they
+ * may not grow it. It grows to at least twice its size and an outgrown one is
+ * kept until hipb_free, since a graph may hold its address. */
+void *hipb_gemm_ws(struct hipb_backend *b, size_t n)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    const int cap = (int)(sizeof(b->gemm_ws) / sizeof(b->gemm_ws[0]));
+    size_t want = n;
+    void *p = NULL;
+
+    if (n == 0)
+        return NULL;
+    if (!b->capture &&
+        (hipStreamIsCapturing((hipStream_t)b->stream, &st) != hipSuccess ||
+         st != hipStreamCaptureStatusNone))
+        return NULL;
+    if (b->gemm_ws_count > 0 && n <= b->gemm_ws_bytes)
+        return b->gemm_ws[b->gemm_ws_count - 1];
+    if (b->capture || b->gemm_ws_count == cap)
+        return NULL;
+    if (want < 2 * b->gemm_ws_bytes)
+        want = 2 * b->gemm_ws_bytes;
+    if (want < ((size_t)32 << 20))
+        want = (size_t)32 << 20;
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return NULL;
+    }
+    b->gemm_ws[b->gemm_ws_count++] = p;
+    b->gemm_ws_bytes = want;
+    return p;
 }
 
 /* ------------------------------------------------------------ timer */

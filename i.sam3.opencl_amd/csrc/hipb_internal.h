@@ -25,6 +25,9 @@ void hipb_run_end(struct hipb_backend *b, int err, const char *what,
 /* Grow a backend-owned device scratch to at least n bytes. */
 void *hipb_scratch(struct hipb_backend *b, size_t n);
 
+/* Workspace of at least n bytes for the exact path's GEMM, or NULL. */
+void *hipb_gemm_ws(struct hipb_backend *b, size_t n);
+
 /* Elements of a buffer of its own type. */
 size_t hipb_count(hipb_mem m);
 

@@ -424,7 +424,7 @@ static int vec_ok(int dt, long off, long s0, long s1, int ld)
     return off % q == 0 && s0 % q == 0 && s1 % q == 0 && ld % q == 0;
 }
 
-extern "C" int launch_gemm(const gemm_desc *d, void *stream)
+extern "C" int launch_gemm(const gemm_desc *d, void *ws, size_t ws_bytes, void *stream)
 {
     const dim3 grid((d->N + 127) / 128, (d->M + 127) / 128, d->nb);
     const int avec = vec_ok(d->adt, d->aoff, d->sa0, d->sa1, d->lda);
@@ -441,6 +441,12 @@ extern "C" int launch_gemm(const gemm_desc *d, void *stream)
     }
     if (d->unpart_ws > 0)
         return hipErrorInvalidValue; /* row remap: NT kernel only */
+    {
+        const int r = launch_gemm_split(d, ws, ws_bytes, stream);
+
+        if (r != -1)
+            return r;
+    }
     if (d->mode == MODE_BF16 && d->transb && d->nb == 1 && d->K % 64 == 0 &&
         avec && bvec && (long)grid.x * grid.y <= 64 &&
         ((uintptr_t)d->A & 15) == 0 && ((uintptr_t)d->B & 15) == 0) {

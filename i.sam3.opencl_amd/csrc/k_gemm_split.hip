@@ -1,0 +1,872 @@
+/* SPDX-License-Identifier: Unlicense
+ *
+ * Exact-path (fp32 operand) GEMM on gfx950:
+ *   C = act(alpha * A * op(B) + bias) + R     (sam3_kernels.cl:57-69)
+ * with float A and C and float or half B: large products on the bf16 matrix
+ * cores from split operands (k_gemm_frag, k_gemm_split), small ones on the
+ * f32 MFMA with K spread over waves (k_gemm_small_f32). launch_gemm_split
+ * chooses; what it does not take (unaligned or bf16 operands, bf16 C) stays
+ * with k_gemm_f32.
+ *
+ * The split. The f32 MFMA peaks at 157 TFLOP/s, the bf16 MFMA at sixteen
+ * times that. A float is exactly the sum of three bf16 values (8 + 8 + 8
+ * mantissa bits, each piece the rounding of what is left): x = x0 + x1 + x2,
+ * |x1| <= 2^-8 |x|, |x2| <= 2^-16 |x|, roundings to nearest, so the pieces'
+ * signs are unbiased. Of the nine products of two split values the six of
+ * order 2^-16 and above are formed on the bf16 MFMA with f32 accumulation;
+ * the three dropped ones are below 2^-24 of the product (2^-27 in the mean),
+ * less than the rounding of one f32 fused multiply-add. A half is exactly
+ * two pieces (five products). The range is the float's: bf16 has its
+ * exponents. Rounding the accumulator six times per 16 k instead of once per
+ * two, the result is no further from the 64-bit product than the f32 MFMA's
+ * in k_gemm_f32: relative error 1.1e-7 against 1.4e-7 at K = 64, 2.4e-7
+ * against 2.9e-7 at 256, 4.9e-7 against 5.7e-7 at 1024, 1.0e-6 against 1.15e-6
+ * at 4096; the small kernel's split sums 1.5e-7 (256) and 2.9e-7 (2048, 8.1e-7
+ * before).
+ *
+ * A non-finite operand (or one that rounds past the largest bf16) makes its
+ * pieces, and so every output it enters, NaN; an output that comes out
+ * non-finite is formed again from the float operands by fused multiply-adds
+ * in k order, so infinities and NaN travel as in k_gemm_f32.
+ *
+ * LDS holds MFMA fragments: per 32 rows, 16 k and piece 1 KiB of 64 chunks
+ * of 16 bytes (8 k of one row), chunk 32 (k half) + row, so that a fragment
+ * read is linear in the lane.
+ */
+#include "k_common.h"
+
+#include <type_traits>
+
+#define GS_K 16   /* K per step */
+/* Steps of a packed operand: K rounded up to 64 (zeros). */
+#define GS_STEPS(K) (((K) + 63) / 64 * 4)
+#define GS_NXCD 8 /* XCDs (L2 domains) of an MI355X */
+#define GS_BAND 8 /* tile rows walked together */
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+/* Four floats as NP bf16 pieces of four. */
+template <int NP> __device__ __forceinline__ void split4(const f32x4 x, u32x2 (&p)[NP])
+{
+    f32x4 r = x;
+
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        p[i].x = pack_bf16x2(r[0], r[1]);
+        p[i].y = pack_bf16x2(r[2], r[3]);
+        if (i + 1 < NP) {
+            r[0] -= __builtin_bit_cast(float, p[i].x << 16);
+            r[1] -= __builtin_bit_cast(float, p[i].x & 0xffff0000u);
+            r[2] -= __builtin_bit_cast(float, p[i].y << 16);
+            r[3] -= __builtin_bit_cast(float, p[i].y & 0xffff0000u);
+        }
+    }
+}
+
+/* LDS byte offset, in its piece's 1 KiB, of k quad q (4 k, 0..3) of row r
+ * of a 32-row block. */
+__device__ __forceinline__ int frag_off(int r, int q)
+{
+    const int h = q >> 1;
+
+    return 16 * (32 * h + (r ^ (4 * h))) + 8 * (q & 1);
+}
+
+/* One output formed from the float operands (non-finite results): a row of
+ * A against elements of B bstep apart. */
+template <int BDT>
+__device__ __noinline__ float dot_seq(const float *a, const void *b, long bstep, int K)
+{
+    float s = 0.0f;
+
+    for (int k = 0; k < K; k++)
+        s = fmaf(a[k],
+                 BDT == DT_F32 ? ((const float *)b)[k * bstep]
+                               : h2f(((const uint16_t *)b)[k * bstep]),
+                 s);
+    return s;
+}
+
+/* Operands split while they are staged: a workgroup owns a BM x BN tile of
+ * C, each wave WM x WN of it as 32 x 32 accumulators. K moves in steps of
+ * 16: beside a step's MFMAs from one LDS slot, the next step's floats,
+ * loaded into registers a step earlier, are split and written to the other
+ * slot (k half 1's chunks at row ^ 4, which keeps the staging writes, 4 rows
+ * x 16 k per 16 lanes, off each other's banks), and the loads of the step
+ * after go out: one barrier per step.
+ *
+ * Bound by issue: a split costs 22 VALU instructions per four floats, and on
+ * this chip VALU and MFMA time add up rather than overlap (128 x 64 tiles:
+ * 31 % and 41 % of the SIMD cycles), so it is used where a float meets few
+ * columns and splitting it in a pass of its own would cost more: the decoder's
+ * image tokens, 331776 x 128 x 256, 215 us against 293 by k_gemm_f32; 165888
+ * rows 93 us, 165 with the pass. */
+template <int BM, int BN, int WM, int WN, int BDT, bool TRANSB>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(gemm_desc d)
+{
+    constexpr int NW = (BM / WM) * (BN / WN), T = NW * 64;
+    constexpr int NA = WM / 32, NB = WN / 32;
+    constexpr int NPB = BDT == DT_F32 ? 3 : 2; /* pieces of B */
+    constexpr int ABYTES = BM / 32 * 3 * 1024, BBYTES = BN / 32 * NPB * 1024;
+    constexpr int SLOT = ABYTES + BBYTES;
+    constexpr int LA = BM * 4 / T, LB = BN * 4 / T; /* k quads per thread */
+    static_assert(BM * 4 % T == 0 && BN * 4 % T == 0, "staging split");
+    __shared__ __attribute__((aligned(16))) char S[2 * SLOT];
+    const int t = threadIdx.x, l = t & 63, w = t >> 6, h = l >> 5, l32 = l & 31;
+    const int wm = w / (BN / WN), wn = w % (BN / WN);
+    const int tn = (d.N + BN - 1) / BN, tm = (d.M + BM - 1) / BM;
+    const int total = tn * tm, per = (total + GS_NXCD - 1) / GS_NXCD;
+    /* Workgroup g runs on XCD g % 8: contiguous tiles per XCD, in bands of
+     * GS_BAND tile rows, so that its L2 serves a window of A and B rows. */
+    const int tile = (int)(blockIdx.x % GS_NXCD) * per + blockIdx.x / GS_NXCD;
+
+    if (tile >= total)
+        return;
+    const int band = tile / (GS_BAND * tn), rem = tile - band * GS_BAND * tn;
+    const int brows = min(GS_BAND, tm - band * GS_BAND);
+    const int m0 = (band * GS_BAND + rem % brows) * BM, n0 = rem / brows * BN;
+    const long z0 = blockIdx.z / d.nb1, z1 = blockIdx.z % d.nb1;
+    const long abase = d.aoff + z0 * d.sa0 + z1 * d.sa1;
+    const long bbase = d.boff + z0 * d.sb0 + z1 * d.sb1;
+    const int nk = (d.K + GS_K - 1) / GS_K;
+    f32x16 acc[NA][NB];
+    f32x4 ra[LA], rb[LB];
+    const float *pa[LA];
+    long ob[LB];
+
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            acc[i][j] = (f32x16){};
+    /* Quad i of thread t: row (t + T i) / 4, k quad t % 4; four lanes read a
+     * row's 64 bytes. Rows past M or N read the last one (never stored). A
+     * K x N B is read with lanes along n: column (t + T i) % BN, quad
+     * (t + T i) / BN. */
+#pragma unroll
+    for (int i = 0; i < LA; i++)
+        pa[i] = (const float *)d.A + abase + (long)min(m0 + (t + T * i) / 4, d.M - 1) * d.lda +
+                4 * (t & 3);
+#pragma unroll
+    for (int i = 0; i < LB; i++)
+        ob[i] = TRANSB ? bbase + (long)min(n0 + (t + T * i) / 4, d.N - 1) * d.ldb + 4 * (t & 3)
+                       : bbase + min(n0 + (t + T * i) % BN, d.N - 1);
+
+    /* The floats of step ks; `last` (a constant): the step may be partial,
+     * its k past K are zero. */
+    auto load = [&](int ks, auto last) {
+        const int k0 = ks * GS_K;
+        const bool in = !decltype(last)::value || k0 + 4 * (t & 3) < d.K;
+
+#pragma unroll
+        for (int i = 0; i < LA; i++)
+            ra[i] = in ? *(const f32x4 *)(pa[i] + k0) : (f32x4){};
+#pragma unroll
+        for (int i = 0; i < LB; i++) {
+            if constexpr (TRANSB) {
+                if constexpr (BDT == DT_F32)
+                    rb[i] = in ? *(const f32x4 *)((const float *)d.B + ob[i] + k0) : (f32x4){};
+                else {
+                    const u32x2 v =
+                        in ? *(const u32x2 *)((const uint16_t *)d.B + ob[i] + k0) : (u32x2){};
+
+                    for (int e = 0; e < 2; e++) {
+                        rb[i][2 * e] = h2f((uint16_t)(v[e] & 0xffffu));
+                        rb[i][2 * e + 1] = h2f((uint16_t)(v[e] >> 16));
+                    }
+                }
+            }
+            else {
+                const int q = (t + T * i) / BN;
+
+                for (int e = 0; e < 4; e++) {
+                    const int k = k0 + 4 * q + e;
+                    const bool kin = !decltype(last)::value || k < d.K;
+                    const long bi = ob[i] + (long)(kin ? k : 0) * d.ldb;
+                    const float v = BDT == DT_F32 ? ((const float *)d.B)[bi]
+                                                  : h2f(((const uint16_t *)d.B)[bi]);
+
+                    rb[i][e] = kin ? v : 0.0f;
+                }
+            }
+        }
+    };
+    auto stage = [&](int slot) {
+        char *s = S + slot * SLOT;
+
+#pragma unroll
+        for (int i = 0; i < LA; i++) {
+            const int row = (t + T * i) / 4;
+            char *p = s + (row >> 5) * 3072 + frag_off(row & 31, t & 3);
+            u32x2 v[3];
+
+            split4<3>(ra[i], v);
+            for (int e = 0; e < 3; e++)
+                *(u32x2 *)(p + 1024 * e) = v[e];
+        }
+#pragma unroll
+        for (int i = 0; i < LB; i++) {
+            const int row = TRANSB ? (t + T * i) / 4 : (t + T * i) % BN;
+            const int q = TRANSB ? t & 3 : (t + T * i) / BN;
+            char *p = s + ABYTES + (row >> 5) * NPB * 1024 + frag_off(row & 31, q);
+            u32x2 v[NPB];
+
+            split4<NPB>(rb[i], v);
+            for (int e = 0; e < NPB; e++)
+                *(u32x2 *)(p + 1024 * e) = v[e];
+        }
+    };
+    const int fo = 16 * (32 * h + (l32 ^ (4 * h)));
+    auto products = [&](int slot) {
+        const char *sa = S + slot * SLOT + wm * NA * 3072 + fo;
+        const char *sb = S + slot * SLOT + ABYTES + wn * NB * NPB * 1024 + fo;
+        bf16x8 a[NA][3], b[NB][NPB];
+
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+                a[i][e] = *(const bf16x8 *)(sa + 3072 * i + 1024 * e);
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int e = 0; e < NPB; e++)
+                b[j][e] = *(const bf16x8 *)(sb + NPB * 1024 * j + 1024 * e);
+        /* Piece pairs (a, b) with a + b <= 2, in k_gemm_frag's order: the
+         * two kernels give the same bits. */
+        constexpr int pairs[6][2] = {{2, 0}, {1, 1}, {1, 0}, {0, 2}, {0, 1}, {0, 0}};
+
+#pragma unroll
+        for (int p = 0; p < 6; p++) {
+            if (pairs[p][1] >= NPB)
+                continue;
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        a[i][pairs[p][0]], b[j][pairs[p][1]], acc[i][j], 0, 0, 0);
+        }
+    };
+
+    const std::false_type whole;
+    const std::true_type last;
+    /* Step ks from slot ks % 2 beside the staging of step ks + 1 and the
+     * loads of step ks + 2, in one basic block. */
+    auto step = [&](int ks, auto slot) {
+        constexpr int s = decltype(slot)::value;
+
+        __syncthreads();
+        stage(s ^ 1);
+        load(ks + 2, whole);
+        products(s);
+    };
+
+    if (nk > 1)
+        load(0, whole);
+    else
+        load(0, last);
+    stage(0);
+    if (nk > 2)
+        load(1, whole);
+    else if (nk > 1)
+        load(1, last);
+    int ks = 0;
+
+    for (; ks + 4 < nk; ks += 2) {
+        step(ks, std::integral_constant<int, 0>());
+        step(ks + 1, std::integral_constant<int, 1>());
+    }
+    for (; ks < nk; ks++) {
+        __syncthreads();
+        if (ks + 1 < nk) {
+            stage((ks + 1) & 1);
+            if (ks + 2 < nk)
+                load(ks + 2, last);
+        }
+        products(ks & 1);
+    }
+
+    /* Epilogue (store_one, sam3_kernels.cl:306-319): 32 lanes store 128
+     * contiguous bytes of a row. */
+    {
+        const long cbase = d.coff + z0 * d.sc0 + z1 * d.sc1;
+        const long rbase = d.roff + z0 * d.sc0 + z1 * d.sc1;
+        float *C = (float *)d.C + cbase;
+        const float *R = d.R ? (const float *)d.R + rbase : nullptr;
+
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int n = n0 + wn * WN + 32 * j + l32;
+            const float bn = d.bias && n < d.N ? d.bias[n] : 0.0f;
+
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int m = m0 + wm * WM + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                    float v = acc[i][j][r];
+
+                    if (m >= d.M || n >= d.N)
+                        continue;
+                    if (!(fabsf(v) < __builtin_inff()))
+                        v = dot_seq<BDT>((const float *)d.A + abase + (long)m * d.lda,
+                                         (const char *)d.B +
+                                             (BDT == DT_F32 ? 4 : 2) *
+                                                 (bbase + (TRANSB ? (long)n * d.ldb : (long)n)),
+                                         TRANSB ? 1 : d.ldb, d.K);
+                    v = act_k(d.alpha * v + bn, d.act);
+                    if (R)
+                        v += R[(long)m * d.ldc + n];
+                    C[(long)m * d.ldc + n] = v;
+                }
+        }
+    }
+}
+
+/* ------------------------------------------------------------ packed */
+
+/* Large products split their operands in a pass of their own (k_split_pack:
+ * 10 bytes moved per element, 15-60 us for the trunk's), so that the K loop
+ * is MFMAs, fragment reads and asynchronous copies only (k_gemm_frag). At
+ * 5184 rows, pass included, against k_gemm_f32: 1024 -> 3072 168 against 311
+ * us (194 TFLOP/s), 1024 -> 4096 243 against 454, 4096 -> 1024 287 against 682,
+ * 1024 -> 1024 87 against 188; half weights 142, 202, 243 and 75 us. (On a
+ * slower machine against the split while staging: 190 / 251, 273 / 323, 295 /
+ * 324, 81 / 87 us.) What bounds it now is the MFMA rate under its own power:
+ * 186 TFLOP/s of six products are 1120 TFLOP/s of bf16, 77 % of what the
+ * platform's 8192^3 bf16 product reaches.
+ */
+
+/* An operand split once into MFMA fragments: [32-row block][16-k step]
+ * [piece][64 chunks of 16 bytes], chunk 32 (k half) + row % 32; rows and k
+ * past the matrix are zero. */
+struct frag_src {
+    const void *src; /* element 0 of the operand */
+    long ld;
+    int rows, K, kmajor; /* kmajor: element (r, k) at k ld + r, else r ld + k */
+    char *dst;
+};
+
+/* 32 rows x 64 k per 256-thread workgroup: eight lanes read 256 contiguous
+ * bytes of a row (or, k-major, 32 lanes 128 contiguous bytes of a k), the
+ * pieces go through LDS (chunk position xored with the k octet against bank
+ * conflicts) and leave as contiguous fragments. */
+template <int DT, int NP> __device__ __forceinline__ void pack_block(const frag_src &f, int blk, char *S)
+{
+    const int t = threadIdx.x, nks = GS_STEPS(f.K), nkc = nks / 4;
+    const int rb = blk / nkc, kc = blk % nkc;
+    const int r = f.kmajor ? t & 31 : t >> 3, k8 = f.kmajor ? t >> 5 : t & 7;
+    const int row = rb * 32 + r, k0 = kc * 64 + k8 * 8;
+    f32x4 x[2] = {};
+
+    if (row < f.rows) {
+        const long i0 = f.kmajor ? (long)k0 * f.ld + row : (long)row * f.ld + k0;
+
+        if (!f.kmajor && k0 + 8 <= f.K) {
+            if constexpr (DT == DT_F32) {
+                x[0] = ((const f32x4 *)((const float *)f.src + i0))[0];
+                x[1] = ((const f32x4 *)((const float *)f.src + i0))[1];
+            }
+            else {
+                const u32x2 *v = (const u32x2 *)((const uint16_t *)f.src + i0);
+
+                for (int j = 0; j < 2; j++)
+                    for (int e = 0; e < 4; e++)
+                        x[j][e] = h2f((uint16_t)(v[j][e >> 1] >> (16 * (e & 1))));
+            }
+        }
+        else
+            for (int e = 0; e < 8; e++)
+                if (k0 + e < f.K) {
+                    const long i = i0 + (f.kmajor ? e * f.ld : e);
+
+                    x[e >> 2][e & 3] = DT == DT_F32 ? ((const float *)f.src)[i]
+                                                    : h2f(((const uint16_t *)f.src)[i]);
+                }
+    }
+    u32x2 lo[NP], hi[NP];
+
+    split4<NP>(x[0], lo);
+    split4<NP>(x[1], hi);
+    for (int p = 0; p < NP; p++) {
+        const int c = (32 * (k8 & 1) + r) ^ k8;
+
+        *(u32x4 *)(S + ((k8 >> 1) * NP + p) * 1024 + 16 * c) =
+            (u32x4){lo[p].x, lo[p].y, hi[p].x, hi[p].y};
+    }
+    __syncthreads();
+    const int frags = NP * 4;
+    char *dst = f.dst + ((long)rb * nks + 4 * kc) * NP * 1024;
+
+    for (int i = t; i < frags * 64; i += 256) {
+        const int fr = i >> 6, c = i & 63, k = 2 * (fr / NP) + (c >> 5);
+
+        *(u32x4 *)(dst + 16L * i) = *(const u32x4 *)(S + fr * 1024 + 16 * (c ^ k));
+    }
+}
+
+template <int BDT>
+__global__ __launch_bounds__(256) void k_split_pack(frag_src a, frag_src b, int ablocks)
+{
+    __shared__ __attribute__((aligned(16))) char S[4 * 3 * 1024];
+
+    if ((int)blockIdx.x < ablocks)
+        pack_block<DT_F32, 3>(a, blockIdx.x, S);
+    else
+        pack_block<BDT, BDT == DT_F32 ? 3 : 2>(b, blockIdx.x - ablocks, S);
+}
+
+/* Asynchronous 16-byte global -> LDS copy: lane i reads base + voff_i and
+ * writes lds + 16 i (base and lds wave-uniform). The kernel waits for it
+ * itself before the barrier that publishes the slot. */
+__device__ __forceinline__ void gs_g2lds16(const void *base, unsigned voff, unsigned lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "global_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(base)
+                 : "memory", "m0");
+}
+
+__device__ __forceinline__ void gs_vmwait0()
+{
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+}
+
+/* A workgroup owns a BM x BN tile, each wave WM x WN; per step of 16 k the
+ * fragments of the tile's rows and columns go HBM -> LDS asynchronously into
+ * one of two slots, a step ahead. The loop is one basic block (the step count
+ * is even; copies past the end repeat the last step into a slot that no one
+ * reads): with a branch in it the compiler kept a second copy of the
+ * accumulators, 128 moves per step (145 against 180 TFLOP/s). */
+template <int BM, int BN, int WM, int WN, int BDT>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void
+k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
+{
+    constexpr int NW = (BM / WM) * (BN / WN), NSLOT = 2;
+    constexpr int NA = WM / 32, NB = WN / 32;
+    constexpr int NPB = BDT == DT_F32 ? 3 : 2;
+    constexpr int AFR = BM / 32 * 3, FR = AFR + BN / 32 * NPB; /* fragments per step */
+    constexpr int CPW = (FR + NW - 1) / NW;                    /* copies per wave */
+    constexpr int SLOT = FR * 1024;
+    __shared__ __attribute__((aligned(16))) char S[NSLOT * SLOT];
+    const int t = threadIdx.x, l = t & 63, h = l >> 5, l32 = l & 31;
+    const int wu = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wu / (BN / WN), wn = wu % (BN / WN);
+    const int tn = (d.N + BN - 1) / BN, tm = (d.M + BM - 1) / BM;
+    const int total = tn * tm, per = (total + GS_NXCD - 1) / GS_NXCD;
+    const int tile = (int)(blockIdx.x % GS_NXCD) * per + blockIdx.x / GS_NXCD;
+
+    if (tile >= total)
+        return;
+    constexpr int GR = 4;
+    const int band = tile / (GR * tn), rem = tile - band * GR * tn;
+    const int brows = min(GR, tm - band * GR);
+    const int m0 = (band * GR + rem % brows) * BM, n0 = rem / brows * BN;
+    const int nk = GS_STEPS(d.K);
+    const int amax = (d.M - 1) / 32, bmax = (d.N - 1) / 32;
+    const char *src[CPW];
+    unsigned step[CPW], lds[CPW];
+
+    /* Copy i of wave w: fragment w + NW i of the step (the last ones may
+     * repeat fragment FR - 1); row blocks past the matrix read the last
+     * (never stored). */
+#pragma unroll
+    for (int i = 0; i < CPW; i++) {
+        const int f = min(wu + NW * i, FR - 1);
+        const bool isa = f < AFR;
+        const int np = isa ? 3 : NPB, g = isa ? f : f - AFR;
+        const int rb = isa ? min(m0 / 32 + g / 3, amax) : min(n0 / 32 + g / NPB, bmax);
+
+        src[i] = (isa ? pa : pb) + ((long)rb * nk * np + g % np) * 1024;
+        step[i] = np * 1024u;
+        lds[i] = (unsigned)(uintptr_t)S + 1024u * f;
+    }
+    const unsigned voff = 16u * l;
+    /* Copies of step ks (past the last: the last again, into a slot that no
+     * one reads any more, so that the loop has no branch). */
+    auto load = [&](int ks, int slot) {
+        const long kc = min(ks, nk - 1);
+
+#pragma unroll
+        for (int i = 0; i < CPW; i++)
+            gs_g2lds16(src[i] + kc * step[i], voff, lds[i] + (unsigned)SLOT * slot);
+    };
+    f32x16 acc[NA][NB];
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            acc[i][j] = (f32x16){};
+    const char *sa = S + wm * NA * 3072 + 16 * l;
+    const char *sb = S + AFR * 1024 + wn * NB * NPB * 1024 + 16 * l;
+    bf16x8 a[3][NA], b[NPB][NB];
+    auto rda = [&](int slot, int p) {
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+            a[p][i] = *(const bf16x8 *)(sa + SLOT * slot + 3072 * i + 1024 * p);
+    };
+    auto rdb = [&](int slot, int p) {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            b[p][j] = *(const bf16x8 *)(sb + SLOT * slot + NPB * 1024 * j + 1024 * p);
+    };
+    auto mm = [&](int p, int q) {
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p][i], b[q][j], acc[i][j],
+                                                                    0, 0, 0);
+    };
+
+    /* Step ks from slot `sl`: its first fragments (a[2], b[0]) are in
+     * registers. Once the others are too, the slot goes to the copies of
+     * step ks + 2 and the next step's first fragments are read under the
+     * last products. */
+    auto body = [&](int ks, auto slot) {
+        constexpr int sl = decltype(slot)::value, sn = (sl + 1) % NSLOT;
+
+        rda(sl, 1);
+        rdb(sl, 1);
+        mm(2, 0);
+        rda(sl, 0);
+        if constexpr (NPB == 3)
+            rdb(sl, 2);
+        mm(1, 1);
+        mm(1, 0);
+        if constexpr (NPB == 3)
+            mm(0, 2);
+        mm(0, 1);
+        gs_vmwait0();
+        __syncthreads();
+        load(ks + NSLOT, sl);
+        rda(sn, 2);
+        mm(0, 0);
+        rdb(sn, 0);
+    };
+
+    load(0, 0);
+    gs_vmwait0();
+    __syncthreads();
+    load(1, 1);
+    rda(0, 2);
+    rdb(0, 0);
+    for (int ks = 0; ks < nk; ks += NSLOT) {
+        body(ks, std::integral_constant<int, 0>());
+        body(ks + 1, std::integral_constant<int, 1>());
+    }
+    /* No copy may land after the workgroup's LDS is given back. */
+    gs_vmwait0();
+    {
+        float *C = (float *)d.C + d.coff;
+        const float *R = d.R ? (const float *)d.R + d.roff : nullptr;
+
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int n = n0 + wn * WN + 32 * j + l32;
+            const float bn = d.bias && n < d.N ? d.bias[n] : 0.0f;
+
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int m = m0 + wm * WM + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                    float v = acc[i][j][r];
+
+                    if (m >= d.M || n >= d.N)
+                        continue;
+                    if (!(fabsf(v) < __builtin_inff()))
+                        v = dot_seq<BDT>((const float *)d.A + d.aoff + (long)m * d.lda,
+                                         (const char *)d.B +
+                                             (BDT == DT_F32 ? 4 : 2) *
+                                                 (d.boff + (d.transb ? (long)n * d.ldb : (long)n)),
+                                         d.transb ? 1 : d.ldb, d.K);
+                    v = act_k(d.alpha * v + bn, d.act);
+                    if (R)
+                        v += R[(long)m * d.ldc + n];
+                    C[(long)m * d.ldc + n] = v;
+                }
+        }
+    }
+}
+
+/* ------------------------------------------------------------ small */
+
+/* Small GEMMs of the exact path : a workgroup per tile of
+ * 16 MT rows x 16 columns whose NW waves split K; no operand staging: each
+ * lane loads four consecutive k of its row of A and its row of B (the Linear
+ * weight, float or half) straight from memory, 16 k of 16 rows per load, as
+ * the operands of four v_mfma_f32_16x16x4_f32, and the partial tiles are
+ * summed through LDS in wave order.
+ *
+ * Bound by latency: a 128 x 128 tile of k_gemm_f32 walks K in steps of 16
+ * with the loads of each exposed (32 x 4096 x 1024: 112 us on 32 of 256
+ * CUs). Here a wave's loads for SMALLF_BATCH steps are in flight at once and
+ * K is spread over the waves: that product 8.4 us, the decoder's token
+ * products 3.1 us (8 x 256 x 256) to 7.9 us (8 x 256 x 2048).
+ *
+ * MFMA 16x16x4 lane layouts: A lane l holds A[l % 16][l / 16], B lane l
+ * B[l / 16][l % 16], D register r of lane l D[4 (l / 16) + r][l % 16]. The
+ * k a lane half holds may be any permutation as long as A and B agree. */
+#define SMALLF_BATCH 4
+
+template <int BDT, int MT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_small_f32(gemm_desc d)
+{
+    __shared__ float red[NW][MT][4][64];
+    const int t = threadIdx.x, l = t & 63, w = t >> 6, q = l >> 4, l16 = l & 15;
+    const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16;
+    const long z0 = blockIdx.z / d.nb1, z1 = blockIdx.z % d.nb1;
+    const long cz = z0 * d.sc0 + z1 * d.sc1;
+    const int ksteps = (d.K + 15) / 16, per = (ksteps + NW - 1) / NW;
+    const int s0 = w * per, s1 = min(s0 + per, ksteps);
+    const int n = min(n0 + l16, d.N - 1);
+    const float *pa[MT];
+    const long ao = d.aoff + z0 * d.sa0 + z1 * d.sa1 + 4 * q;
+    const long bo = d.boff + z0 * d.sb0 + z1 * d.sb1 + (long)n * d.ldb + 4 * q;
+    f32x4 acc[MT];
+
+    for (int i = 0; i < MT; i++) {
+        pa[i] = (const float *)d.A + ao + (long)min(m0 + 16 * i + l16, d.M - 1) * d.lda;
+        acc[i] = (f32x4){};
+    }
+    for (int s = s0; s < s1; s += SMALLF_BATCH) {
+        f32x4 a[SMALLF_BATCH][MT], b[SMALLF_BATCH];
+
+#pragma unroll
+        for (int u = 0; u < SMALLF_BATCH; u++) {
+            /* K % 4 == 0: a lane's four k are in or out together. */
+            const int k = 16 * (s + u);
+            const bool in = s + u < s1 && k + 4 * q < d.K;
+
+            for (int i = 0; i < MT; i++)
+                a[u][i] = in ? *(const f32x4 *)(pa[i] + k) : (f32x4){};
+            if constexpr (BDT == DT_F32)
+                b[u] = in ? *(const f32x4 *)((const float *)d.B + bo + k) : (f32x4){};
+            else {
+                const uint2 v = in ? *(const uint2 *)((const uint16_t *)d.B + bo + k)
+                                   : make_uint2(0, 0);
+
+                b[u][0] = h2f((uint16_t)(v.x & 0xffffu));
+                b[u][1] = h2f((uint16_t)(v.x >> 16));
+                b[u][2] = h2f((uint16_t)(v.y & 0xffffu));
+                b[u][3] = h2f((uint16_t)(v.y >> 16));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SMALLF_BATCH; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i][e], b[u][e], acc[i], 0,
+                                                                  0, 0);
+    }
+    for (int i = 0; i < MT; i++)
+        for (int r = 0; r < 4; r++)
+            red[w][i][r][l] = acc[i][r];
+    __syncthreads();
+    for (int x = t; x < MT * 256; x += 64 * NW) {
+        const int i = x >> 8, r = (x >> 6) & 3, ll = x & 63;
+        const int mr = m0 + 16 * i + 4 * (ll >> 4) + r, nc = n0 + (ll & 15);
+        const long idx = (long)mr * d.ldc + nc;
+        float v = red[0][i][r][ll];
+
+        for (int p = 1; p < NW; p++)
+            v += red[p][i][r][ll];
+        if (mr >= d.M || nc >= d.N)
+            continue;
+        v = act_k(d.alpha * v + (d.bias ? d.bias[nc] : 0.0f), d.act);
+        if (d.R)
+            v += ((const float *)d.R)[d.roff + cz + idx];
+        ((float *)d.C)[d.coff + cz + idx] = v;
+    }
+}
+
+/* ------------------------------------------------------------ launch */
+
+static int gs_aligned(const gemm_desc *d)
+{
+    const long a = d->aoff | d->sa0 | d->sa1 | d->lda, b = d->boff | d->sb0 | d->sb1 | d->ldb;
+
+    if (d->mode != MODE_F32 || d->adt != DT_F32 || d->cdt != DT_F32 || d->bdt == DT_BF16 ||
+        d->unpart_ws > 0 || d->pack_N > 0 || d->K < 4 || d->K % 4 || a % 4 ||
+        ((uintptr_t)d->A & 15))
+        return 0;
+    /* A K x N operand is read element by element. */
+    return !d->transb || (b % 4 == 0 && ((uintptr_t)d->B & 15) == 0);
+}
+
+static long gs_tiles(const gemm_desc *d, int bm, int bn)
+{
+    return (long)((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn);
+}
+
+/* Small: at most one 64 x 64 tile per two CUs (of one batch: the kernel, and
+ * so the bits, do not depend on how many are in a call), where a staged tile's K loop
+ * is all latency (400 x 1024 x 1024, 112 tiles: 25 us against 30; 1000 x 1024
+ * x 1024, 256 tiles: 49 against 31; 1000 x 300 x 4096, 80 tiles: 73 against
+ * 137). */
+static int gs_small(const gemm_desc *d)
+{
+    return d->transb && gs_tiles(d, 64, 64) * 2 <= dev_cu_count();
+}
+
+/* Rows of A per packed chunk: at most 512 MiB of pieces. */
+static int gs_chunk(const gemm_desc *d)
+{
+    const long row = GS_STEPS((long)d->K) * 96, rows = (512L << 20) / row / 256 * 256;
+
+    return rows < 256 ? 256 : rows < d->M ? (int)rows : d->M;
+}
+
+/* Packing pays when what it saves, 4.6e-15 s per product (125 against 175
+ * TFLOP/s), exceeds its 2.2e-12 s per element and a launch: at equal sides
+ * about 1000 x 1000. */
+extern "C" size_t gemm_split_ws(const gemm_desc *d)
+{
+    const double M = d->M, N = d->N, K = d->K;
+
+    if (!gs_aligned(d) || d->nb != 1 || gs_small(d) ||
+        (M + N) * K * 2.2e-12 + 4e-6 > M * N * K * 4.6e-15)
+        return 0;
+    return (size_t)GS_STEPS((long)d->K) * 1024 *
+           (((size_t)gs_chunk(d) + 31) / 32 * 3 +
+            ((size_t)d->N + 31) / 32 * (d->bdt == DT_F32 ? 3 : 2));
+}
+
+/* Tile shape of k_gemm_frag. With every CU busy the chip runs at its power:
+ * a 64 x 64 unit of C costs 1.0 (256 x 256 tiles) to 1.17 (64 x 64, more
+ * operand traffic); a last round that fills only some CUs runs each of its
+ * tiles at the higher clock, `alone` per unit, unless the power is used up
+ * all the same. Measured (11 us per unit at K = 1024, 5184 x 1024 .. 4096 and
+ * 2500 x 1024); the model picks within 3 % of the best of the five. */
+static const struct {
+    int bm, bn;
+    double full, alone;
+} gs_cfg[5] = {{256, 256, 1.0, 0.62}, {256, 128, 1.05, 0.85}, {128, 128, 1.06, 0.95},
+               {128, 64, 1.13, 0.9}, {64, 64, 1.17, 1.0}};
+
+static int gs_pick(const gemm_desc *d)
+{
+    const long cus = dev_cu_count();
+    double best = 0.0;
+    int pick = 0;
+
+    for (int c = 0; c < 5; c++) {
+        const long tiles = gs_tiles(d, gs_cfg[c].bm, gs_cfg[c].bn), rem = tiles % cus;
+        const double unit = gs_cfg[c].bm * gs_cfg[c].bn / 4096.0;
+        const double part = gs_cfg[c].full * rem / cus;
+        const double cost = unit * (tiles / cus * gs_cfg[c].full +
+                                    (rem == 0 ? 0.0
+                                              : part > gs_cfg[c].alone ? part : gs_cfg[c].alone));
+
+        if (c == 0 || cost < best) {
+            best = cost;
+            pick = c;
+        }
+    }
+    return pick;
+}
+
+template <int BDT>
+static int launch_packed(const gemm_desc *d, void *ws, hipStream_t s)
+{
+    constexpr int NPB = BDT == DT_F32 ? 3 : 2;
+    const long nks = GS_STEPS((long)d->K);
+    const int chunk = gs_chunk(d), bblocks = (int)((d->N + 31L) / 32 * (nks / 4));
+    char *pb = (char *)ws, *pa = pb + (d->N + 31L) / 32 * nks * NPB * 1024;
+    const frag_src fb = {(const char *)d->B + (BDT == DT_F32 ? 4 : 2) * d->boff, d->ldb, d->N,
+                         d->K, !d->transb, pb};
+
+    for (int m0 = 0; m0 < d->M; m0 += chunk) {
+        gemm_desc c = *d;
+
+        c.M = d->M - m0 < chunk ? d->M - m0 : chunk;
+        c.aoff += (long)m0 * d->lda;
+        c.coff += (long)m0 * d->ldc;
+        c.roff += (long)m0 * d->ldc;
+        const frag_src fa = {(const float *)d->A + c.aoff, d->lda, c.M, d->K, 0, pa};
+        const long ablocks = (c.M + 31L) / 32 * (nks / 4);
+        const int cfg = gs_pick(&c);
+        const long grid = (gs_tiles(&c, gs_cfg[cfg].bm, gs_cfg[cfg].bn) + GS_NXCD - 1) /
+                          GS_NXCD * GS_NXCD;
+
+        if (ablocks + bblocks > 0x7fffffffL || grid > 0x7fffffffL)
+            return hipErrorInvalidConfiguration;
+        /* The weights are split once, with the first chunk. */
+        hipLaunchKernelGGL((k_split_pack<BDT>),
+                           dim3((unsigned)(ablocks + (m0 ? 0 : bblocks))), dim3(256), 0, s, fa,
+                           fb, (int)ablocks);
+#define GS_FRAG(I, BM, BN, WM, WN)                                                              \
+    if (cfg == I)                                                                              \
+    hipLaunchKernelGGL((k_gemm_frag<BM, BN, WM, WN, BDT>), dim3((unsigned)grid),               \
+                       dim3((BM / WM) * (BN / WN) * 64), 0, s, c, pa, pb)
+        GS_FRAG(0, 256, 256, 64, 64);
+        GS_FRAG(1, 256, 128, 64, 64);
+        GS_FRAG(2, 128, 128, 64, 32);
+        GS_FRAG(3, 128, 64, 64, 32);
+        GS_FRAG(4, 64, 64, 32, 32);
+#undef GS_FRAG
+    }
+    return hipGetLastError();
+}
+
+template <int BDT, bool TRANSB>
+static int launch_staged(const gemm_desc *d, hipStream_t s)
+{
+    /* 128 x 64 tiles when they give every CU two (165888 x 128 x 256: 93
+     * against 95 us; 5184 x 1024 x 1024: 87 against 94), else 64 x 64 (5184 x
+     * 128 x 256: 11 against 17 us). */
+    const bool big = gs_tiles(d, 128, 64) * d->nb >= 2L * dev_cu_count();
+    const long tiles = big ? gs_tiles(d, 128, 64) : gs_tiles(d, 64, 64);
+    const long grid = (tiles + GS_NXCD - 1) / GS_NXCD * GS_NXCD;
+
+    if (grid > 0x7fffffffL)
+        return hipErrorInvalidConfiguration;
+    if (big)
+        hipLaunchKernelGGL((k_gemm_split<128, 64, 64, 32, BDT, TRANSB>),
+                           dim3((unsigned)grid, 1, d->nb), dim3(256), 0, s, *d);
+    else
+        hipLaunchKernelGGL((k_gemm_split<64, 64, 32, 32, BDT, TRANSB>),
+                           dim3((unsigned)grid, 1, d->nb), dim3(256), 0, s, *d);
+    return hipGetLastError();
+}
+
+template <int BDT> static int launch_small(const gemm_desc *d, hipStream_t s)
+{
+    /* Two row tiles per workgroup once single ones would give every CU two;
+     * four waves' loads cover K <= 512, eight beyond. */
+    const long t16 = gs_tiles(d, 16, 16);
+    const int mt = t16 >= 2L * dev_cu_count() ? 2 : 1;
+    const dim3 grid((d->N + 15) / 16, (d->M + 16 * mt - 1) / (16 * mt), d->nb);
+
+    if (mt == 2 && d->K > 512)
+        hipLaunchKernelGGL((k_gemm_small_f32<BDT, 2, 8>), grid, dim3(512), 0, s, *d);
+    else if (mt == 2)
+        hipLaunchKernelGGL((k_gemm_small_f32<BDT, 2, 4>), grid, dim3(256), 0, s, *d);
+    else if (d->K > 512)
+        hipLaunchKernelGGL((k_gemm_small_f32<BDT, 1, 8>), grid, dim3(512), 0, s, *d);
+    else
+        hipLaunchKernelGGL((k_gemm_small_f32<BDT, 1, 4>), grid, dim3(256), 0, s, *d);
+    return hipGetLastError();
+}
+
+extern "C" int launch_gemm_split(const gemm_desc *d, void *ws, size_t ws_bytes, void *stream)
+{
+    hipStream_t s = (hipStream_t)stream;
+    const size_t need = gemm_split_ws(d);
+
+    if (!gs_aligned(d))
+        return -1;
+    if (gs_small(d))
+        return d->bdt == DT_F32 ? launch_small<DT_F32>(d, s) : launch_small<DT_F16>(d, s);
+    if (need && ws && ws_bytes >= need)
+        return d->bdt == DT_F32 ? launch_packed<DT_F32>(d, ws, s)
+                                : launch_packed<DT_F16>(d, ws, s);
+    if (d->bdt == DT_F32)
+        return d->transb ? launch_staged<DT_F32, true>(d, s) : launch_staged<DT_F32, false>(d, s);
+    return d->transb ? launch_staged<DT_F16, true>(d, s) : launch_staged<DT_F16, false>(d, s);
+}

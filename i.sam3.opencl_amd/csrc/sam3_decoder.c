@@ -589,7 +589,9 @@ void sam_dec_graph(struct sam_model *m, int P, int enable)
                    hipb_errstr(err), err);
         return;
     }
+    b->capture = 1;
     dec_kernels(m, P);
+    b->capture = 0;
     err = hipStreamEndCapture((hipStream_t)b->stream, &g);
     if (hipb_failed() || err != hipSuccess || !g || b->scratch != scratch) {
         if (g)

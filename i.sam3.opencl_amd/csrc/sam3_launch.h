@@ -67,7 +67,13 @@ struct gemm_desc {
     void *pack_q16, *pack_k16, *pack_vt16;
     float *pack_knorm;
 };
-int launch_gemm(const struct gemm_desc *d, void *stream);
+/* ws: device workspace of at least gemm_split_ws(d) bytes, or NULL (the
+ * product then splits its operands while staging them). */
+int launch_gemm(const struct gemm_desc *d, void *ws, size_t ws_bytes, void *stream);
+/* Workspace the exact path's product d uses (0: none). */
+size_t gemm_split_ws(const struct gemm_desc *d);
+/* The exact path on split operands; -1 if d is not of its form. */
+int launch_gemm_split(const struct gemm_desc *d, void *ws, size_t ws_bytes, void *stream);
 /* The bf16 x bf16 "NT" kernel (A [M][K], B [N][K], K % 64 == 0,
  * unbatched); -1 if d does not have that form, else a hipError_t. */
 int launch_gemm_nt(const struct gemm_desc *d, void *stream);

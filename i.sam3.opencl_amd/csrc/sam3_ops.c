@@ -106,6 +106,7 @@ void gemm(struct sam_model *m, int M, int N, int K, struct opnd A,
     struct gemm_desc d;
     struct opnd Ro;
     const char *what;
+    void *ws;
     int err;
 
     if (M < 0 || N < 0 || K < 0 || nb < 1 || nb1 < 1 || act < ACT_NONE ||
@@ -173,8 +174,9 @@ void gemm(struct sam_model *m, int M, int N, int K, struct opnd A,
     what = gemm_nt_ok(&d)           ? "gemm_nt_bf16"
            : d.mode == MODE_BF16 ? "gemm_bf16"
                                  : "gemm_f32";
+    ws = hipb_gemm_ws(b, gemm_split_ws(&d));
     hipb_run_begin(b);
-    err = launch_gemm(&d, b->stream);
+    err = launch_gemm(&d, ws, b->gemm_ws_bytes, b->stream);
     hipb_run_end(b, err, what, 2.0 * M * N * K * (double)nb);
 }
 
@@ -1389,7 +1391,9 @@ void sam_trunk_graph(struct sam_model *m, int enable)
                    hipb_errstr(err), err);
         return;
     }
+    b->capture = 1;
     trunk_kernels(m);
+    b->capture = 0;
     err = hipStreamEndCapture((hipStream_t)b->stream, &g);
     if (hipb_failed() || err != hipSuccess || !g || work_gen != gen) {
         if (g)

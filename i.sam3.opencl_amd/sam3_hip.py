@@ -72,7 +72,11 @@ class HipbBackend(ctypes.Structure):
                 ("scratch", ctypes.c_void_p),
                 ("scratch_bytes", ctypes.c_size_t),
                 ("stage", ctypes.c_void_p * 2), ("stage_ev", ctypes.c_void_p * 2),
-                ("stage_next", ctypes.c_int)]
+                ("stage_next", ctypes.c_int),
+                ("gemm_ws", ctypes.c_void_p * 20),
+                ("gemm_ws_count", ctypes.c_int),
+                ("gemm_ws_bytes", ctypes.c_size_t),
+                ("capture", ctypes.c_int)]
 
 
 class Opnd(ctypes.Structure):

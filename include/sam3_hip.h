@@ -92,6 +92,12 @@ struct hipb_backend {
     void *stage[2];
     void *stage_ev[2];
     int stage_next;
+    /* Workspaces of the exact path's GEMM, each at least twice the one
+     * before; the last is in use, of gemm_ws_bytes. */
+    void *gemm_ws[20];
+    int gemm_ws_count;
+    size_t gemm_ws_bytes;
+    int capture; /* the library is capturing a graph of its own */
 };
 
 /* Select a device and create its stream (ocl_init, ocl_backend.h:57-59).

@@ -377,3 +377,92 @@ def test_mha_rejects_wide_heads_with_many_keys(hip, be):
     d = be.alloc(100 * 256 * 4)
     with pytest.raises(hip.Sam3HipError, match="mha: unsupported shape"):
         hip.mha(m, 1, 4, 100, 256, d, 0, d, 0, d, 0, d)
+
+
+@pytest.fixture(scope="module")
+def be_half(hip):
+    b = hip.Backend(precision="fp16")
+    yield b
+    b.free()
+
+
+@pytest.mark.parametrize("M,N,K,transb", [
+    (1, 1, 4, 1), (8, 256, 2048, 1), (33, 70, 300, 1), (32, 4096, 520, 1),  # f32 MFMA
+    (5184, 128, 256, 1), (700, 1024, 68, 1),      # split while staged, 64 x 64 tiles
+    (33000, 100, 36, 1), (16500, 256, 256, 0),    # 128 x 64 tiles; K x N operand
+    (2500, 1030, 1024, 1),                        # packed, 64 x 64 tiles
+    (5184, 1024, 260, 1), (5100, 4096, 132, 1),   # 128 x 64 and 256 x 128
+    (5184, 3072, 512, 1), (9000, 1000, 516, 0),   # 256 x 256; K x N operand
+    (4600, 2050, 64, 1),
+])
+@pytest.mark.parametrize("half", [False, True])
+def test_gemm_split_paths(hip, be, be_half, M, N, K, transb, half):
+    """The exact path's product kernels (f32 MFMA over split K, operands split
+    while staged, operands packed) at ragged sizes against float64, float and
+    half B, with bias and residual. A sum of K products of N(0, 1) values
+    rounded at most K times to 2^-24 of its running size, errors of random
+    sign: below sqrt(K) 2^-24 of the result (and one rounding for the
+    epilogue)."""
+    b = be_half if half else be
+    m = model(hip, b)
+    g = rng(M + N + K)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    B = (g.standard_normal((N, K) if transb else (K, N), dtype=np.float32) * 0.05)
+    if half:
+        B = B.astype(np.float16).astype(np.float32)
+    bias = g.standard_normal(N, dtype=np.float32)
+    C0 = g.standard_normal((M, N), dtype=np.float32)
+    dA, dB, dv, dC = b.upload(A), b.upload_weight(B), b.upload(bias), b.upload(C0)
+    hip.gemm(m, M, N, K, hip.mat(dA, 0, K), hip.mat(dB, 0, K if transb else N),
+             transb, hip.mat(dC, 0, N), 1, 1, dv, dC, 0, 0.5, hip.ACT_RELU)
+    got = b.read(dC).reshape(M, N)
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), [M - 1],
+                                     g.integers(0, M, 60)]))
+    p = A[rows].astype(np.float64) @ (B.T if transb else B).astype(np.float64)
+    want = np.maximum(0.5 * p + bias, 0) + C0[rows]
+    assert rel_l2(got[rows], want) <= (np.sqrt(K) + 2) * 2.0 ** -24
+    for x in (dA, dB, dv, dC):
+        b.release(x)
+
+
+def test_gemm_split_packed_bits(hip, be):
+    """Packing the operands first or splitting them while they are staged
+    gives the same bits: the first 700 rows of a product that is packed, and
+    the product of those rows alone, which is not."""
+    m = model(hip, be)
+    g = rng(7)
+    A = g.standard_normal((5184, 1000), dtype=np.float32)
+    B = g.standard_normal((1024, 1000), dtype=np.float32)
+    dA, dB, dC = be.upload(A), be.upload(B), be.alloc(5184 * 1024 * 4)
+    out = []
+    for rows in (5184, 700):
+        hip.linear(m, rows, 1000, 1024, dA, 0, dB, None, dC, 0)
+        out.append(be.read(dC, 700 * 1024).copy())
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 1024, 68), (5184, 1024, 260), (40, 64, 64)])
+def test_gemm_split_non_finite(hip, be, orc, M, N, K):
+    """Infinities, NaN and values that round past the largest bf16: every
+    output is what the sequential float sum gives (finite rows untouched)."""
+    m = model(hip, be)
+    g = rng(M)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    B = g.standard_normal((N, K), dtype=np.float32)
+    A[3, 5], A[4, 6], A[5, 7] = np.inf, np.nan, np.float32(3.4e38)
+    A[6, 1], A[6, 2] = np.inf, -np.inf
+    B[9, 5] = 0.0
+    B[11, 3] = -np.inf
+    B[:, 7] = 0.25
+    dA, dB, dC = be.upload(A), be.upload(B), be.alloc(M * N * 4)
+    hip.gemm(m, M, N, K, hip.mat(dA, 0, K), hip.mat(dB, 0, K), 1,
+             hip.mat(dC, 0, N))
+    got = be.read(dC).reshape(M, N)
+    want = np.zeros((16, N), np.float32)
+    orc.gemm(orc.GEMM_SEQ, 16, N, K, A[:16].ravel().copy(), 0, K, 0, 0, B.ravel(), 0, K,
+             0, 0, 1, want, 0, N, 0, 0, 1, 1)
+    assert np.array_equal(np.isnan(got[:16]), np.isnan(want))
+    assert np.array_equal(got[:16][np.isinf(want)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got[:16]), fin)
+    assert np.all(np.abs(got[:16][fin] - want[fin]) <= 1e-5 * np.abs(want[fin]) + 2e-4)
