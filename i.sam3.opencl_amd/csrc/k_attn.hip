@@ -235,6 +235,153 @@ __device__ __forceinline__ void block_yx(int yb, int xb, int W, int off, int &y,
 
 /* ------------------------------------------------------------ fp32 path */
 
+/* Online-softmax state of one wave of the exact path: a lane's query (the
+ * same in lanes l and l ^ 32), O^T registers, reference point m (log2
+ * units) and the lane's share of the weights' sum. */
+struct exact_state {
+    f32x16 o0, o1;
+    float m, l;
+};
+
+/* Softmax weights of a 32-key block from its raw scores s: register r holds
+ * key kb 32 + 8 (r / 4) + 4 h + r % 4 of the lane's query qi. Scores in log2
+ * units relative to m: t = s scale log2(e) - m as one rounding, keys past Nk
+ * (last block), the causal mask or the bias (brow; added to the scaled
+ * score, natural units, as softmax_ext adds it) applied; the weights are
+ * exp2(t). m is the first block's max, then moves only when a score leaves
+ * [m - SAFE_SPAN, m + SAFE_SPAN]: up (O and l shrink) when the block max
+ * passes m + SAFE_SPAN, down while the query has no weight yet and its block
+ * max lies below m - SAFE_SPAN. After the first block a wave takes the exact
+ * max (its cross-lane exchange, the rescale of O and l) only for blocks
+ * whose in-lane maxima it cannot clear; O / l does not depend on m. */
+template <int HD, bool EXT>
+__device__ __forceinline__ f32x16 exact_softmax(const attn_desc &d, f32x16 s, int kb, bool first,
+                                                int qi, const float *brow, int bH,
+                                                exact_state &st)
+{
+    const int h = (threadIdx.x & 63) >> 5, Nk = d.Nk;
+    const float sc2 = d.scale * LOG2E_F;
+    float rs = 0.0f, mx = -INFINITY;
+
+    if (EXT && brow) {
+        for (int r = 0; r < 16; r++)
+            s[r] *= d.scale;
+        if (d.bW > 0) {
+            const int yb = kb * 32 / d.bW, xb = kb * 32 - yb * d.bW;
+
+            for (int g = 0; g < 4; g++) {
+                int y, x;
+
+                block_yx(yb, xb, d.bW, 8 * g + 4 * h, y, x);
+                box_add<4>(brow, bH, Nk, kb * 32 + 8 * g + 4 * h, y, x, s, 4 * g);
+            }
+        }
+        else
+            for (int g = 0; g < 4; g++) {
+                const f32x4 bv = *(const f32x4 *)(brow + kb * 32 + 8 * g + 4 * h);
+
+                for (int e = 0; e < 4; e++)
+                    s[4 * g + e] += bv[e];
+            }
+        for (int r = 0; r < 16; r++)
+            s[r] = fmaf(s[r], LOG2E_F, -st.m);
+    }
+    else
+        for (int r = 0; r < 16; r++)
+            s[r] = fmaf(s[r], sc2, -st.m);
+    if (kb * 32 + 32 > Nk)
+        for (int r = 0; r < 16; r++) {
+            const int key = kb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+
+            s[r] = key < Nk ? s[r] : -INFINITY;
+        }
+    if (EXT && d.causal)
+        for (int r = 0; r < 16; r++) {
+            const int key = kb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+
+            if (key > qi)
+                s[r] = -INFINITY;
+        }
+    for (int r = 0; r < 16; r++)
+        mx = fmaxf(mx, s[r]);
+    if (first || __ballot(mx > SAFE_SPAN || (st.l == 0.0f && mx < -SAFE_SPAN &&
+                                                mx != -INFINITY)) != 0) {
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const bool empty = st.l + __shfl_xor(st.l, 32, 64) == 0.0f;
+        /* The first block sets m to its max outright, as the reference's
+         * softmax does (that key's weight is then exactly 1: a query
+         * that sees one key gets its value row unchanged). */
+        const float mv = (first || mx > SAFE_SPAN || (empty && mx < -SAFE_SPAN)) &&
+                                 mx != -INFINITY
+                             ? mx
+                             : 0.0f;
+
+        if (!first) {
+            /* Moving down, the query has no weight to rescale. */
+            const float corr = __builtin_amdgcn_exp2f(-fmaxf(mv, 0.0f));
+
+            st.l *= corr;
+            for (int r = 0; r < 16; r++) {
+                st.o0[r] *= corr;
+                if (HD == 64)
+                    st.o1[r] *= corr;
+            }
+        }
+        for (int r = 0; r < 16; r++)
+            s[r] -= mv;
+        st.m += mv;
+    }
+    for (int r = 0; r < 16; r++) {
+        s[r] = __builtin_amdgcn_exp2f(s[r]);
+        rs += s[r];
+    }
+    st.l += rs;
+    return s;
+}
+
+/* Store of the lane's query row: O registers over the weights' sum l. */
+template <int HD>
+__device__ __forceinline__ void exact_store(const attn_desc &d, long orow, const f32x16 &o0,
+                                            const f32x16 &o1, float l)
+{
+    const int h = (threadIdx.x & 63) >> 5;
+    const float inv = 1.0f / l;
+
+    if (d.odt == DT_F32 && ((orow & 3) | ((uintptr_t)d.O & 15)) == 0) {
+        /* Registers 4 g .. 4 g + 3 are columns 8 g + 4 h .. + 3 of the
+         * lane's query row: one 16-byte store each. */
+        float *op = (float *)d.O + orow + 4 * h;
+
+        for (int g = 0; g < 4; g++) {
+            const f32x4 x0 = {o0[4 * g] * inv, o0[4 * g + 1] * inv, o0[4 * g + 2] * inv,
+                              o0[4 * g + 3] * inv};
+
+            *(f32x4 *)(op + 8 * g) = x0;
+            if (HD == 64) {
+                const f32x4 x1 = {o1[4 * g] * inv, o1[4 * g + 1] * inv,
+                                  o1[4 * g + 2] * inv, o1[4 * g + 3] * inv};
+
+                *(f32x4 *)(op + 32 + 8 * g) = x1;
+            }
+        }
+        return;
+    }
+    for (int r = 0; r < 16; r++) {
+        const int dd = 8 * (r >> 2) + 4 * h + (r & 3);
+
+        if (d.odt == DT_F32) {
+            ((float *)d.O)[orow + dd] = o0[r] * inv;
+            if (HD == 64)
+                ((float *)d.O)[orow + 32 + dd] = o1[r] * inv;
+        }
+        else {
+            ((uint16_t *)d.O)[orow + dd] = f2bf(o0[r] * inv);
+            if (HD == 64)
+                ((uint16_t *)d.O)[orow + 32 + dd] = f2bf(o1[r] * inv);
+        }
+    }
+}
+
 /* fp32 operands in the reference row layout (Q/K/V/O opnds of
  * sam3_model.c:1004-1011, or the Q, K, V, O rows of the text path's
  * attend, sam3_text.c:305-343), v_mfma_f32_32x32x2_f32, 32-key blocks:
@@ -303,9 +450,7 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
     const int kr = t / LPR, dc = (t % LPR) * 8;
     const bool loader = t < 32 * LPR;
     float qreg[HH], kpre[8], vpre[8];
-    f32x16 o0, o1;
-    float m_run = 0.0f, l_run = 0.0f;
-    const float sc2 = d.scale * LOG2E_F;
+    exact_state st;
 
     /* Q: lane holds channels HH h .. HH h + HH - 1 of query qi, rotated
      * and scaled. */
@@ -328,10 +473,8 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
             }
         }
     }
-    for (int r = 0; r < 16; r++) {
-        o0[r] = 0.0f;
-        o1[r] = 0.0f;
-    }
+    st.o0 = st.o1 = (f32x16){};
+    st.m = st.l = 0.0f;
 
     /* Global -> registers for block kb (RoPE on K), registers -> LDS. */
     auto fetch = [&](int kb) {
@@ -378,115 +521,30 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
         for (int r = 0; r < 16; r++)
             s[r] = 0.0f;
 #pragma unroll
-        for (int st = 0; st < HH; st++)
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(Kt[buf][st + HH * h][l32], qreg[st], s, 0,
-                                                     0, 0);
+        for (int i = 0; i < HH; i++)
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(Kt[buf][i + HH * h][l32], qreg[i], s, 0, 0,
+                                                     0);
         return s;
     };
-    /* Scores in log2 units relative to the lane's reference point m
-     * (m_run, log2 units, the same in lanes l and l ^ 32): t = s scale
-     * log2(e) - m as one rounding, keys past Nk (last block), the causal
-     * mask or the bias (added to the scaled score, natural units, as
-     * softmax_ext adds it) applied; then P = exp2(t), O^T += V^T P^T from
-     * buffer buf. Register r holds key kb 32 + 8 (r / 4) + 4 h + r % 4.
-     * m is the first block's max, then moves only when a score leaves
-     * [m - SAFE_SPAN, m + SAFE_SPAN]: up (O and l shrink) when the block
-     * max passes m + SAFE_SPAN, down while the query has no weight yet
-     * and its block max lies below m - SAFE_SPAN. After the first block a
-     * wave takes the exact max (its cross-lane exchange, the rescale of O
-     * and l) only for blocks whose in-lane maxima it cannot clear; O / l
-     * does not depend on m. */
+    /* The block's weights, then O^T += V^T P^T from buffer buf. */
     auto soft_pv = [&](f32x16 s, int kb, int buf) {
-        float rs = 0.0f, mx = -INFINITY;
-
-        if (EXT && brow) {
-            for (int r = 0; r < 16; r++)
-                s[r] *= d.scale;
-            if (d.bW > 0) {
-                const int yb = kb * 32 / d.bW, xb = kb * 32 - yb * d.bW;
-
-                for (int g = 0; g < 4; g++) {
-                    int y, x;
-
-                    block_yx(yb, xb, d.bW, 8 * g + 4 * h, y, x);
-                    box_add<4>(brow, bH, Nk, kb * 32 + 8 * g + 4 * h, y, x, s, 4 * g);
-                }
-            }
-            else
-                for (int g = 0; g < 4; g++) {
-                    const f32x4 bv = *(const f32x4 *)(brow + kb * 32 + 8 * g + 4 * h);
-
-                    for (int e = 0; e < 4; e++)
-                        s[4 * g + e] += bv[e];
-                }
-            for (int r = 0; r < 16; r++)
-                s[r] = fmaf(s[r], LOG2E_F, -m_run);
-        }
-        else
-            for (int r = 0; r < 16; r++)
-                s[r] = fmaf(s[r], sc2, -m_run);
-        if (kb * 32 + 32 > Nk)
-            for (int r = 0; r < 16; r++) {
-                const int key = kb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-
-                s[r] = key < Nk ? s[r] : -INFINITY;
-            }
-        if (EXT && d.causal)
-            for (int r = 0; r < 16; r++) {
-                const int key = kb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-
-                if (key > qi)
-                    s[r] = -INFINITY;
-            }
-        for (int r = 0; r < 16; r++)
-            mx = fmaxf(mx, s[r]);
-        if (kb == kb0 || __ballot(mx > SAFE_SPAN || (l_run == 0.0f && mx < -SAFE_SPAN &&
-                                                    mx != -INFINITY)) != 0) {
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const bool empty = l_run + __shfl_xor(l_run, 32, 64) == 0.0f;
-            /* The first block sets m to its max outright, as the reference's
-             * softmax does (that key's weight is then exactly 1: a query
-             * that sees one key gets its value row unchanged). */
-            const float mv = (kb == kb0 || mx > SAFE_SPAN || (empty && mx < -SAFE_SPAN)) &&
-                                     mx != -INFINITY
-                                 ? mx
-                                 : 0.0f;
-
-            if (kb != kb0) {
-                /* Moving down, the query has no weight to rescale. */
-                const float corr = __builtin_amdgcn_exp2f(-fmaxf(mv, 0.0f));
-
-                l_run *= corr;
-                for (int r = 0; r < 16; r++) {
-                    o0[r] *= corr;
-                    if (HD == 64)
-                        o1[r] *= corr;
-                }
-            }
-            for (int r = 0; r < 16; r++)
-                s[r] -= mv;
-            m_run += mv;
-        }
-        for (int r = 0; r < 16; r++) {
-            s[r] = __builtin_amdgcn_exp2f(s[r]);
-            rs += s[r];
-        }
-        l_run += rs;
+        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
         /* The exponentials issued before the P V MFMAs: left to the
          * scheduler, which weighs the code after the key loop too, each
          * MFMA could follow the exponential it reads and wait for it
          * (3 % on one 576-token window). */
         __builtin_amdgcn_sched_barrier(0);
-        /* O^T += V^T P^T: step st contracts key 8 (st / 4) + 4 h + st % 4,
-         * the key of this lane's score register st. */
+        /* Step i contracts key 8 (i / 4) + 4 h + i % 4, the key of this
+         * lane's weight register i. */
 #pragma unroll
-        for (int st = 0; st < 16; st++) {
-            const int key = 8 * (st >> 2) + 4 * h + (st & 3);
+        for (int i = 0; i < 16; i++) {
+            const int key = 8 * (i >> 2) + 4 * h + (i & 3);
 
-            o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[buf][key][l32], s[st], o0, 0, 0, 0);
+            st.o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[buf][key][l32], s[i], st.o0, 0, 0,
+                                                         0);
             if (HD == 64)
-                o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[buf][key][32 + l32], s[st], o1, 0,
-                                                          0, 0);
+                st.o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(Vs[buf][key][32 + l32], s[i],
+                                                             st.o1, 0, 0, 0);
         }
     };
 
@@ -510,50 +568,381 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
     }
     __builtin_amdgcn_s_setprio(0);
 
-    l_run += __shfl_xor(l_run, 32, 64);
+    st.l += __shfl_xor(st.l, 32, 64);
     if constexpr (SPLIT)
-        if (!split_merge<HD == 64>(part, cnt, item, nsplit, sp, !idle, o0, o1, m_run, l_run))
+        if (!split_merge<HD == 64>(part, cnt, item, nsplit, sp, !idle, st.o0, st.o1, st.m, st.l))
             return;
-    if (qi >= N)
-        return;
-    {
-        const float inv = 1.0f / l_run;
-        const long orow = d.ooff + b0 * d.so0 + b1 * d.so1 + (long)qi * d.ldo;
+    if (qi < N)
+        exact_store<HD>(d, d.ooff + b0 * d.so0 + b1 * d.so1 + (long)qi * d.ldo, st.o0, st.o1,
+                        st.l);
+}
 
-        if (d.odt == DT_F32 && ((orow & 3) | ((uintptr_t)d.O & 15)) == 0) {
-            /* Registers 4 g .. 4 g + 3 are columns 8 g + 4 h .. + 3 of the
-             * lane's query row: one 16-byte store each. */
-            float *op = (float *)d.O + orow + 4 * h;
+/* Asynchronous 16-byte global -> LDS copy (global_load_lds_dwordx4):
+ * lane i of the wave writes lds_base + 16 i (lds_base wave-uniform, via
+ * M0). Issued as inline assembly so that the compiler does not treat the
+ * copy as a store that later LDS reads of the other slot must wait for:
+ * the kernel waits for it itself (s_waitcnt vmcnt(0)) before the barrier
+ * that hands the slot to the readers. */
+__device__ __forceinline__ void g2lds16(const void *g, void *lds_base)
+{
+    /* The low 32 bits of a flat LDS address are the LDS offset. */
+    const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_base);
 
-            for (int g = 0; g < 4; g++) {
-                const f32x4 x0 = {o0[4 * g] * inv, o0[4 * g + 1] * inv, o0[4 * g + 2] * inv,
-                                  o0[4 * g + 3] * inv};
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "global_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(lds), "v"(g)
+                 : "memory", "m0");
+}
 
-                *(f32x4 *)(op + 8 * g) = x0;
-                if (HD == 64) {
-                    const f32x4 x1 = {o1[4 * g] * inv, o1[4 * g + 1] * inv,
-                                      o1[4 * g + 2] * inv, o1[4 * g + 3] * inv};
+/* The same copy with a wave-uniform 64-bit base in SGPRs and a 32-bit
+ * per-lane byte offset (the saddr form): no per-lane address arithmetic
+ * when only the base moves from block to block. `lds` must be
+ * wave-uniform. */
+__device__ __forceinline__ void g2lds16_s(const void *base, unsigned voff, unsigned lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "global_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(base)
+                 : "memory", "m0");
+}
 
-                    *(f32x4 *)(op + 32 + 8 * g) = x1;
+/* ------------------------------------------------------------ fp32 path, split operands */
+
+/* The exact path of larger problems: K, V and Q, and the weights P, as three
+ * bf16 pieces each (exactly the float, split4), six piece products per
+ * product on v_mfma_f32_32x32x16_bf16 with f32 accumulation, the three below
+ * 2^-24 of it dropped: what the f32 MFMA of k_attn_f32 forms at a sixteenth
+ * of the rate. K (rotated) and V^T are split once per call by
+ * k_kv_split into MFMA fragments, which this kernel copies HBM -> LDS
+ * asynchronously, a 32-key block ahead; Q is split into registers; the
+ * weights come out of exact_softmax, k_attn_f32's, and meet V^T from the
+ * registers they are in (its keys permuted to match).
+ *
+ * Bound by the sum of its MFMA time (48 per 32-key block and wave at head
+ * width 64, 1536 cycles) and its VALU time (about 210 instructions, 88 of
+ * them splitting the weights), which do not overlap on this chip; three waves
+ * per SIMD. 16 heads x 64, packing included, against k_attn_f32: 5184 x 5184
+ * 979 -> 519 us (212 TFLOP/s), 2600 x 2600 257 -> 150, 800 x 800 45 -> 37; 8 x
+ * 32: 5184 x 5184 276 -> 163. The error against 64 bits is lower at every size
+ * measured (5184 keys: 1.15e-6 against 1.34e-6).
+ *
+ * A non-finite operand makes every result it enters NaN; a query whose
+ * result comes out non-finite is formed again from the float operands
+ * (exact_row_seq), so infinities and NaN travel as in k_attn_f32. */
+
+/* Bytes of a key block's fragments: K [HD / 16][3], then V^T [HD / 32][2]
+ * [3], 1 KiB each. */
+#define KVS_BLOCK(HD) ((HD) * 384)
+
+/* Fragments of 32-key block blockIdx.x of unit blockIdx.y: K chunk (row r,
+ * k half h) 8 channels at 32 h + r; V^T chunk (channel c, k half h of step s)
+ * the keys 16 s + 4 h + {0..3, 8..11}, the keys of weight registers 8 s ..
+ * 8 s + 7. Keys past Nk are zero. Through LDS so that both the row reads and
+ * the fragment writes are contiguous. Bound by memory: 4 bytes read and 6
+ * written per element. */
+template <int HD>
+__global__ __launch_bounds__(256) void k_kv_split(attn_desc d, char *__restrict__ out)
+{
+    __shared__ __attribute__((aligned(16))) float Ks[32][HD + 4], Vs[32][HD + 4];
+    constexpr int LPR = HD / 8;
+    const int t = threadIdx.x, Nk = d.Nk, kb = blockIdx.x;
+    const long unit = blockIdx.y, b0 = unit / d.nb1, b1 = unit % d.nb1;
+    const int kr = t / LPR, dc = (t % LPR) * 8, key = kb * 32 + kr;
+    char *o = out + (unit * gridDim.x + kb) * KVS_BLOCK(HD);
+
+    if (kr < 32) {
+        float k[8] = {}, v[8] = {};
+
+        if (key < Nk) {
+            const float *kp = (const float *)d.K + d.koff + b0 * d.sk0 + b1 * d.sk1 +
+                              (long)key * d.ldk + dc;
+            const float *vp = (const float *)d.V + d.voff + b0 * d.sv0 + b1 * d.sv1 +
+                              (long)key * d.ldv + dc;
+
+            for (int e = 0; e < 8; e++) {
+                k[e] = kp[e];
+                v[e] = vp[e];
+            }
+            if (HD == 64 && d.rope) {
+                const float2 *rot = (const float2 *)d.rope + (long)(key % d.npos) * 32 + dc / 2;
+
+                for (int j = 0; j < 4; j++) {
+                    const float a = k[2 * j], b = k[2 * j + 1];
+                    const float2 r = rot[j];
+
+                    k[2 * j] = fmaf(a, r.x, -(b * r.y));
+                    k[2 * j + 1] = fmaf(a, r.y, b * r.x);
                 }
             }
-            return;
         }
-        for (int r = 0; r < 16; r++) {
-            const int dd = 8 * (r >> 2) + 4 * h + (r & 3);
-
-            if (d.odt == DT_F32) {
-                ((float *)d.O)[orow + dd] = o0[r] * inv;
-                if (HD == 64)
-                    ((float *)d.O)[orow + 32 + dd] = o1[r] * inv;
-            }
-            else {
-                ((uint16_t *)d.O)[orow + dd] = f2bf(o0[r] * inv);
-                if (HD == 64)
-                    ((uint16_t *)d.O)[orow + 32 + dd] = f2bf(o1[r] * inv);
-            }
+        for (int e = 0; e < 8; e++) {
+            Ks[kr][dc + e] = k[e];
+            Vs[kr][dc + e] = v[e];
         }
     }
+    __syncthreads();
+    for (int i = t; i < HD * 4; i += 256) {
+        /* Chunk i of K: octet i / 32 of row i % 32. */
+        const int r = i & 31, c8 = i >> 5;
+        u32x2 x[3], y[3];
+        char *p = o + (c8 >> 1) * 3072 + 16 * (32 * (c8 & 1) + r);
+
+        split4<3>(*(const f32x4 *)&Ks[r][8 * c8], x);
+        split4<3>(*(const f32x4 *)&Ks[r][8 * c8 + 4], y);
+        for (int e = 0; e < 3; e++)
+            *(u32x4 *)(p + 1024 * e) = (u32x4){x[e].x, x[e].y, y[e].x, y[e].y};
+    }
+    for (int i = t; i < HD * 4; i += 256) {
+        /* Chunk i of V^T: channel i % HD, step and half i / HD. */
+        const int c = i % HD, q = i / HD, k0 = 16 * (q >> 1) + 4 * (q & 1);
+        f32x4 lo, hi;
+        u32x2 x[3], y[3];
+        char *p = o + HD * 192 + ((c >> 5) * 2 + (q >> 1)) * 3072 + 16 * (32 * (q & 1) + (c & 31));
+
+        for (int e = 0; e < 4; e++) {
+            lo[e] = Vs[k0 + e][c];
+            hi[e] = Vs[k0 + 8 + e][c];
+        }
+        split4<3>(lo, x);
+        split4<3>(hi, y);
+        for (int e = 0; e < 3; e++)
+            *(u32x4 *)(p + 1024 * e) = (u32x4){x[e].x, x[e].y, y[e].x, y[e].y};
+    }
+}
+
+/* Columns 8 g + 4 h .. + 3 (g < HD / 8) of query qi's result from the float
+ * operands, one key after another (non-finite results). */
+template <int HD, bool EXT>
+__device__ __noinline__ void exact_row_seq(attn_desc d, long unit, int qi, const float *brow,
+                                           int bH, float *o)
+{
+    /* A score is the same number in both passes, however large. */
+#pragma clang fp contract(off)
+    const int h = (threadIdx.x & 63) >> 5;
+    const long b0 = unit / d.nb1, b1 = unit % d.nb1;
+    const float *q = (const float *)d.Q + d.qoff + b0 * d.sq0 + b1 * d.sq1 + (long)qi * d.ldq;
+    const float *K = (const float *)d.K + d.koff + b0 * d.sk0 + b1 * d.sk1;
+    const float *V = (const float *)d.V + d.voff + b0 * d.sv0 + b1 * d.sv1;
+    const float2 *cs = HD == 64 ? (const float2 *)d.rope : nullptr;
+    float mx = -INFINITY, l = 0.0f;
+
+    for (int e = 0; e < HD / 2; e++)
+        o[e] = 0.0f;
+    for (int pass = 0; pass < 2; pass++)
+        for (int key = 0; key < d.Nk; key++) {
+            const float *k = K + (long)key * d.ldk;
+            float s = 0.0f;
+
+            for (int j = 0; j < HD / 2; j++) {
+                float qa = q[2 * j], qb = q[2 * j + 1], ka = k[2 * j], kb = k[2 * j + 1];
+
+                if (cs) {
+                    const float2 rq = cs[(long)(qi % d.npos) * 32 + j];
+                    const float2 rk = cs[(long)(key % d.npos) * 32 + j];
+                    const float a = qa, c = ka;
+
+                    qa = fmaf(a, rq.x, -(qb * rq.y));
+                    qb = fmaf(a, rq.y, qb * rq.x);
+                    ka = fmaf(c, rk.x, -(kb * rk.y));
+                    kb = fmaf(c, rk.y, kb * rk.x);
+                }
+                s = fmaf(qb, kb, fmaf(qa, ka, s));
+            }
+            if (EXT && brow) {
+                const float b = d.bW > 0 ? brow[key / d.bW] + brow[bH + key % d.bW] : brow[key];
+
+                s = (s * d.scale + b) * LOG2E_F;
+            }
+            else
+                s *= d.scale * LOG2E_F;
+            if (EXT && d.causal && key > qi)
+                s = -INFINITY;
+            if (pass == 0)
+                mx = fmaxf(mx, s);
+            else {
+                const float p = __builtin_amdgcn_exp2f(s - (mx == -INFINITY ? 0.0f : mx));
+
+                l += p;
+                for (int e = 0; e < HD / 2; e++)
+                    o[e] = fmaf(p, V[(long)key * d.ldv + 8 * (e >> 2) + 4 * h + (e & 3)], o[e]);
+            }
+        }
+    o[HD / 2] = l;
+}
+
+template <int HD, bool EXT, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void k_attn_split(attn_desc d, const char *__restrict__ kv,
+                                                       float *__restrict__ part,
+                                                       unsigned *__restrict__ cnt, int nsplit)
+{
+    constexpr int NS = HD / 16, BLK = KVS_BLOCK(HD), CPW = BLK / 4096;
+    __shared__ __attribute__((aligned(16))) char S[2 * BLK];
+    const int t = threadIdx.x, l = t & 63, h = l >> 5, l32 = l & 31;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int N = d.N, Nk = d.Nk;
+    /* As k_attn_f32: (unit, tile, split) triples in NXCD contiguous ranges. */
+    const int ntiles = (N + 127) / 128;
+    const long total = (long)d.nb * ntiles * nsplit, per = (total + NXCD - 1) / NXCD;
+    const long pos = (long)(blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
+
+    if (pos >= total)
+        return;
+    /* (readfirstlane: the divisions leave their results in VGPRs.) */
+    const int item = __builtin_amdgcn_readfirstlane((int)(pos / nsplit));
+    const int unit = __builtin_amdgcn_readfirstlane(item / ntiles);
+    const int sp = (int)pos - item * nsplit, tile = item - unit * ntiles;
+    const long b0 = unit / d.nb1, b1 = unit % d.nb1;
+    const int qi = tile * 128 + w * 32 + l32;
+    const bool idle = tile * 128 + w * 32 >= N;
+    const int nblk = (Nk + 31) / 32;
+    const int kb0 = __builtin_amdgcn_readfirstlane((int)((long)sp * nblk / nsplit));
+    const int kb1 = __builtin_amdgcn_readfirstlane((int)((long)(sp + 1) * nblk / nsplit));
+    const int bH = d.bW > 0 ? Nk / d.bW : 0;
+    const float *brow = EXT && d.bias
+                            ? d.bias + ((long)unit * N + (qi < N ? qi : N - 1)) *
+                                           (d.bW > 0 ? bH + d.bW : (Nk + 63) / 64 * 64)
+                            : nullptr;
+    const char *src = kv + ((long)unit * nblk) * BLK + 1024 * CPW * w;
+    const unsigned lds = (unsigned)(uintptr_t)S + 1024u * CPW * w, voff = 16u * l;
+    auto load = [&](int kb, int buf) {
+        const uint64_t a = (uint64_t)(uintptr_t)src + (uint64_t)kb * BLK;
+        const char *b = (const char *)(uintptr_t)(
+            (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a) |
+            (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)) << 32);
+        const unsigned to = __builtin_amdgcn_readfirstlane(lds + BLK * buf);
+
+        for (int i = 0; i < CPW; i++)
+            g2lds16_s(b + 1024 * i, voff, to + 1024u * i);
+    };
+    bf16x8 q[NS][3];
+    exact_state st;
+
+    load(kb0, 0);
+    /* Q: the lane's channels 16 s + 8 h .. + 7 of query qi, rotated, split. */
+    for (int s = 0; s < NS; s++) {
+        float x[8] = {};
+
+        if (qi < N) {
+            const int c0 = 16 * s + 8 * h;
+            const float *qr = (const float *)d.Q + d.qoff + b0 * d.sq0 + b1 * d.sq1 +
+                              (long)qi * d.ldq + c0;
+
+            for (int e = 0; e < 8; e++)
+                x[e] = qr[e];
+            if (HD == 64 && d.rope) {
+                const float2 *rot = (const float2 *)d.rope + (long)(qi % d.npos) * 32 + c0 / 2;
+
+                for (int j = 0; j < 4; j++) {
+                    const float a = x[2 * j], b = x[2 * j + 1];
+                    const float2 r = rot[j];
+
+                    x[2 * j] = fmaf(a, r.x, -(b * r.y));
+                    x[2 * j + 1] = fmaf(a, r.y, b * r.x);
+                }
+            }
+        }
+        u32x2 lo[3], hi[3];
+
+        split4<3>((f32x4){x[0], x[1], x[2], x[3]}, lo);
+        split4<3>((f32x4){x[4], x[5], x[6], x[7]}, hi);
+        for (int p = 0; p < 3; p++)
+            q[s][p] = __builtin_bit_cast(bf16x8, (u32x4){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
+    }
+    st.o0 = st.o1 = (f32x16){};
+    st.m = st.l = 0.0f;
+
+    int lvl = -1;
+
+    for (int kb = kb0; kb < kb1; kb++) {
+        const int buf = (kb - kb0) & 1;
+        const char *kf = S + BLK * buf + 16 * l, *vf = kf + NS * 3072;
+        f32x16 s = {};
+
+        prio_by_progress(kb - kb0, kb1 - kb0, lvl);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (kb + 1 < kb1)
+            load(kb + 1, buf ^ 1);
+        /* Piece pairs (K or V, Q or P) of a product, smallest first. */
+        constexpr int pairs[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            bf16x8 k[3];
+
+            for (int p = 0; p < 3; p++)
+                k[p] = *(const bf16x8 *)(kf + i * 3072 + p * 1024);
+            for (int p = 0; p < 6; p++)
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[pairs[p][0]], q[i][pairs[p][1]], s,
+                                                            0, 0, 0);
+        }
+        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
+        bf16x8 pf[2][3];
+
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            u32x2 lo[3], hi[3];
+
+            split4<3>((f32x4){s[8 * i], s[8 * i + 1], s[8 * i + 2], s[8 * i + 3]}, lo);
+            split4<3>((f32x4){s[8 * i + 4], s[8 * i + 5], s[8 * i + 6], s[8 * i + 7]}, hi);
+            for (int p = 0; p < 3; p++)
+                pf[i][p] =
+                    __builtin_bit_cast(bf16x8, (u32x4){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
+        }
+        auto pv = [&](f32x16 o, int c) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                bf16x8 v[3];
+
+                for (int p = 0; p < 3; p++)
+                    v[p] = *(const bf16x8 *)(vf + (c * 2 + i) * 3072 + p * 1024);
+                for (int p = 0; p < 6; p++)
+                    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[pairs[p][0]], pf[i][pairs[p][1]],
+                                                                o, 0, 0, 0);
+            }
+            return o;
+        };
+
+        st.o0 = pv(st.o0, 0);
+        if (HD == 64)
+            st.o1 = pv(st.o1, 1);
+    }
+    __builtin_amdgcn_s_setprio(0);
+
+    st.l += __shfl_xor(st.l, 32, 64);
+    auto finite = [&]() {
+        float sum = st.l;
+
+        for (int r = 0; r < 16; r++)
+            sum += (st.o0[r] - st.o0[r]) + (HD == 64 ? st.o1[r] - st.o1[r] : 0.0f);
+        return fabsf(sum) < INFINITY;
+    };
+
+    if constexpr (SPLIT) {
+        /* A split that is not finite outweighs the others in the merge. */
+        if (!finite()) {
+            st.m = 1e30f;
+            st.l = INFINITY;
+        }
+        if (!split_merge<HD == 64>(part, cnt, item, nsplit, sp, !idle, st.o0, st.o1, st.m, st.l))
+            return;
+    }
+    if (qi >= N)
+        return;
+    if (!finite()) {
+        float o[HD / 2 + 1];
+
+        exact_row_seq<HD, EXT>(d, unit, qi, brow, bH, o);
+        st.l = o[HD / 2];
+        for (int r = 0; r < 16; r++) {
+            st.o0[r] = o[r];
+            if (HD == 64)
+                st.o1[r] = o[HD / 4 + r];
+        }
+    }
+    exact_store<HD>(d, d.ooff + b0 * d.so0 + b1 * d.so1 + (long)qi * d.ldo, st.o0, st.o1, st.l);
 }
 
 /* ------------------------------------------------------------ packing */
@@ -846,37 +1235,6 @@ struct SoftState {
     f32x16 o0, o1;
     float m, l;
 };
-
-/* Asynchronous 16-byte global -> LDS copy (global_load_lds_dwordx4):
- * lane i of the wave writes lds_base + 16 i (lds_base wave-uniform, via
- * M0). Issued as inline assembly so that the compiler does not treat the
- * copy as a store that later LDS reads of the other slot must wait for:
- * the kernel waits for it itself (s_waitcnt vmcnt(0)) before the barrier
- * that hands the slot to the readers. */
-__device__ __forceinline__ void g2lds16(const void *g, void *lds_base)
-{
-    /* The low 32 bits of a flat LDS address are the LDS offset. */
-    const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_base);
-
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(lds), "v"(g)
-                 : "memory", "m0");
-}
-
-/* The same copy with a wave-uniform 64-bit base in SGPRs and a 32-bit
- * per-lane byte offset (the saddr form): no per-lane address arithmetic
- * when only the base moves from block to block. `lds` must be
- * wave-uniform. */
-__device__ __forceinline__ void g2lds16_s(const void *base, unsigned voff, unsigned lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory", "m0");
-}
 
 /* Balanced launch of k_attn_bf16 when the tiles fill between two and
  * three workgroups per CU (the global ViT block: 82 tiles per XCD on 32
@@ -1980,8 +2338,23 @@ extern "C" int launch_attn_bf16(const attn_desc *d, const void *q16,
     return hipGetLastError();
 }
 
-extern "C" int launch_attn_f32(const attn_desc *d, float *part, unsigned *cnt, int nsplit,
-                               void *stream)
+extern "C" size_t attn_split_ws(const attn_desc *d)
+{
+    /* The pieces save about 4e-15 s per operation (100 against 165-210
+     * TFLOP/s), packing costs a launch and 20 bytes moved per channel of a
+     * key. Measured, 8 heads x 32: 1200 x 1200 31 us either way, 600 x 5184 46
+     * -> 41, 201 x 5184 30 -> 32; 16 x 64: 576 x 576 24 -> 25, 800 x 800 45 ->
+     * 37. (Units past the pass's grid take the other kernel.) */
+    const double ops = 4.0 * d->nb * (double)d->N * d->Nk * d->hd;
+    const double keys = (double)d->nb * d->Nk * d->hd;
+
+    if (d->nb > 65535 || ops * 4.0e-15 < keys * 5.0e-12 + 5e-6)
+        return 0;
+    return (size_t)d->nb * (((size_t)d->Nk + 31) / 32) * KVS_BLOCK((size_t)d->hd);
+}
+
+extern "C" int launch_attn_f32(const attn_desc *d, void *ws, float *part, unsigned *cnt,
+                               int nsplit, void *stream)
 {
     const int nblk = (d->Nk + 31) / 32;
     const long total = (long)d->nb * ((d->N + 127) / 128) * nsplit;
@@ -1992,6 +2365,27 @@ extern "C" int launch_attn_f32(const attn_desc *d, float *part, unsigned *cnt, i
         nsplit > nblk || (nsplit > 1 && (!part || !cnt)) || (d->hd != 64 && d->hd != 32) ||
         (d->hd == 32 && d->rope))
         return hipErrorInvalidConfiguration;
+    if (ws) {
+        const dim3 g((unsigned)nblk, (unsigned)d->nb);
+        auto kern = nsplit > 1 ? (d->hd == 32 ? (ext ? k_attn_split<32, true, true>
+                                                     : k_attn_split<32, false, true>)
+                                              : (ext ? k_attn_split<64, true, true>
+                                                     : k_attn_split<64, false, true>))
+                               : (d->hd == 32 ? (ext ? k_attn_split<32, true, false>
+                                                     : k_attn_split<32, false, false>)
+                                              : (ext ? k_attn_split<64, true, false>
+                                                     : k_attn_split<64, false, false>));
+
+        if (d->hd == 32)
+            hipLaunchKernelGGL(k_kv_split<32>, g, dim3(256), 0, (hipStream_t)stream, *d,
+                               (char *)ws);
+        else
+            hipLaunchKernelGGL(k_kv_split<64>, g, dim3(256), 0, (hipStream_t)stream, *d,
+                               (char *)ws);
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, *d,
+                           (const char *)ws, part, cnt, nsplit);
+        return hipGetLastError();
+    }
     {
         auto kern = nsplit > 1 ? (d->hd == 32 ? (ext ? k_attn_f32<32, true, true>
                                                      : k_attn_f32<32, false, true>)

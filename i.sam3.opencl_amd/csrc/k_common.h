@@ -17,6 +17,7 @@ typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define LOG2E_F 1.4426950408889634f
 
@@ -60,6 +61,25 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
     p.x = (__bf16)lo;
     p.y = (__bf16)hi;
     return __builtin_bit_cast(uint32_t, p);
+}
+
+/* Four floats as NP bf16 pieces of four, each the rounding (to nearest) of
+ * what the pieces before it leave: three are exactly the float. */
+template <int NP> __device__ __forceinline__ void split4(const f32x4 x, u32x2 (&p)[NP])
+{
+    f32x4 r = x;
+
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        p[i].x = pack_bf16x2(r[0], r[1]);
+        p[i].y = pack_bf16x2(r[2], r[3]);
+        if (i + 1 < NP) {
+            r[0] -= __builtin_bit_cast(float, p[i].x << 16);
+            r[1] -= __builtin_bit_cast(float, p[i].x & 0xffff0000u);
+            r[2] -= __builtin_bit_cast(float, p[i].y << 16);
+            r[3] -= __builtin_bit_cast(float, p[i].y & 0xffff0000u);
+        }
+    }
 }
 
 /* Element load of any storage type as float. */

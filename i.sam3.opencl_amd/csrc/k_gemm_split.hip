@@ -43,26 +43,6 @@
 #define GS_NXCD 8 /* XCDs (L2 domains) of an MI355X */
 #define GS_BAND 8 /* tile rows walked together */
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-/* Four floats as NP bf16 pieces of four. */
-template <int NP> __device__ __forceinline__ void split4(const f32x4 x, u32x2 (&p)[NP])
-{
-    f32x4 r = x;
-
-#pragma unroll
-    for (int i = 0; i < NP; i++) {
-        p[i].x = pack_bf16x2(r[0], r[1]);
-        p[i].y = pack_bf16x2(r[2], r[3]);
-        if (i + 1 < NP) {
-            r[0] -= __builtin_bit_cast(float, p[i].x << 16);
-            r[1] -= __builtin_bit_cast(float, p[i].x & 0xffff0000u);
-            r[2] -= __builtin_bit_cast(float, p[i].y << 16);
-            r[3] -= __builtin_bit_cast(float, p[i].y & 0xffff0000u);
-        }
-    }
-}
-
 /* LDS byte offset, in its piece's 1 KiB, of k quad q (4 k, 0..3) of row r
  * of a 32-row block. */
 __device__ __forceinline__ int frag_off(int r, int q)

@@ -155,8 +155,11 @@ struct attn_desc {
  * are split nsplit ways in the same launch: `part` (nb ceil(N / 128)
  * SPLIT_RECS(nsplit) 9216 floats) holds the records and `cnt` (nb
  * ceil(N / 128) SPLIT_CNT counts) the arrival counts. */
-int launch_attn_f32(const struct attn_desc *d, float *part, unsigned *cnt, int nsplit,
-                    void *stream);
+int launch_attn_f32(const struct attn_desc *d, void *ws, float *part, unsigned *cnt,
+                    int nsplit, void *stream);
+/* Workspace with which launch_attn_f32 splits its operands (0: it does not
+ * pay, or the shape does not take it); ws NULL: the f32 MFMA kernel. */
+size_t attn_split_ws(const struct attn_desc *d);
 
 /* Packed bf16 staging of the fast path, Np = N rounded up to 64:
  * q16/k16 [nb][Np][64] (RoPE applied, q scaled), vt16 [nb][64][Np],

@@ -749,13 +749,15 @@ static void attn_fused_hd(struct sam_model *m, const char *who, int hd, int N,
                 n32 = 64;
             ns = n32 > 1 ? (int)n32 : 1;
         }
+        void *ws;
         float *part = attn_part(m, N, nb, ns);
         unsigned *cnt = ns > 1 ? attn_cnt(m, (long)nb * ((N + 127) / 128) * SPLIT_CNT) : NULL;
 
         if (ns > 1 && (!part || !cnt))
             return;
+        ws = hipb_gemm_ws(b, attn_split_ws(&d));
         hipb_run_begin(b);
-        err = launch_attn_f32(&d, part, cnt, ns, b->stream);
+        err = launch_attn_f32(&d, ws, part, cnt, ns, b->stream);
         hipb_run_end(b, err, "attn_f32", 4.0 * N * (double)Nk * hd * nb);
     }
 }

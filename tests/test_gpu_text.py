@@ -222,3 +222,51 @@ def test_box_bias_grids(hip, be, orc, Nq, H, W, hd):
     want = orc.attend(Q, K, V, heads, hd, dy=dy, dx=dx, W=W)
     assert report("box grid H=%d W=%d hd=%d %s" % (H, W, hd, be.precision), got,
                   want) <= TOL[be.precision]
+
+
+@pytest.mark.parametrize("nq,nk,heads,hd,form", [
+    (1000, 2000, 6, 64, "plain"),     # key splits, ragged query tile and key block
+    (1601, 1601, 16, 64, "plain"),    # one split, a one-query tile and a one-key block
+    (1300, 1300, 16, 32, "plain"),
+    (1500, 1500, 12, 64, "causal"),
+    (1100, 1100, 16, 32, "causal"),
+    (900, 72 * 40, 8, 32, "box"),     # bias rows
+    (700, 50 * 45, 8, 64, "box"),     # bias table
+])
+@pytest.mark.parametrize("bad", [False, True])
+def test_split_operands(hip, be, orc, nq, nk, heads, hd, form, bad):
+    """Sizes at which the exact path splits its operands (and the same calls
+    on bf16), sampled queries against the oracle. `bad`: infinities and NaN in
+    K and V of a head; the exact path's results are finite, infinite or NaN as
+    the oracle's, the other heads' untouched."""
+    g = np.random.default_rng(nq + nk)
+    Q = g.standard_normal((nq, heads * hd)).astype(np.float32)
+    K, V = (g.standard_normal((nk, heads * hd)).astype(np.float32) for _ in range(2))
+    kw = {"causal": form == "causal"}
+    if form == "box":
+        W = 72 if nk % 72 == 0 else 50
+        kw.update(dy=(2 * g.standard_normal((nq, nk // W, heads))).astype(np.float32),
+                  dx=(2 * g.standard_normal((nq, W, heads))).astype(np.float32), W=W)
+    if bad:
+        if be.precision == "bf16":
+            pytest.skip("the bf16 path's operands are rounded, not split")
+        V[3, 5], V[7, 9] = np.inf, np.nan   # head 0
+        K[11, hd + 2] = 3.4e38              # head 1: scores of +-inf
+    got = _run(hip, be, Q, K, V, heads, hd, **kw)
+    rows = np.unique(np.concatenate([[0, 1, 31, 32, 127, 128, nq - 2, nq - 1],
+                                     g.choice(nq, 40, replace=False)]))
+    if form == "causal":
+        want = orc.attend(Q, K, V, heads, hd, **kw)[rows]
+    else:
+        if form == "box":
+            kw.update(dy=kw["dy"][rows], dx=kw["dx"][rows])
+        want = orc.attend(Q[rows], K, V, heads, hd, **kw)
+    got = got[rows]
+    if bad:
+        cols = slice(2 * hd, None)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        fin = np.isfinite(want[:, :2 * hd])
+        assert np.allclose(got[:, :2 * hd][fin], want[:, :2 * hd][fin], rtol=1e-4, atol=1e-4)
+        got, want = got[:, cols], want[:, cols]
+    assert report("split operands %s %s" % (form, be.precision), got, want) <= TOL[be.precision]
