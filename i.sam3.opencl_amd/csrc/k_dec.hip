@@ -179,11 +179,11 @@ __global__ __launch_bounds__(256) void k_mha_fewkeys(
     }
 }
 
-/* Few keys (<= 8), head width 32, for precision=bf16: four lanes per
- * (prompt, query, head), each holding 8 of the 32 channels; the partial
- * dot products close over the four lanes, the softmax runs on the exp2
- * domain, and each lane writes its 8 output channels. Rows are read as
- * float4 (16-byte aligned strides, checked by the launcher). */
+/* Few keys (<= 8), head width 32 (the token self-attention): four lanes per
+ * (prompt, query, head), each holding 8 of the 32 channels; the partial dot
+ * products close over the four lanes, the softmax runs on the exp2 domain,
+ * and each lane writes its 8 output channels. Rows are read as float4
+ * (16-byte aligned strides, checked by the launcher). */
 __global__ __launch_bounds__(256) void k_mha_few32x4(
     const float *__restrict__ Q, long sq, const float *__restrict__ K,
     long sk, const float *__restrict__ V, long sv, float *__restrict__ O,
@@ -240,22 +240,6 @@ __global__ __launch_bounds__(256) void k_mha_few32x4(
     *(f32x4 *)(out + 4) = o1 * inv;
 }
 
-extern "C" int launch_mha_few32x4(const float *Q, long sq, const float *K,
-                                  long sk, const float *V, long sv, float *O,
-                                  int P, int Nq, int Nk, int dint, float scale,
-                                  void *stream)
-{
-    const long total = (long)P * Nq * 32;
-
-    if (dint != 256 || Nk < 1 || Nk > 8 || ((sq | sk | sv) & 3) ||
-        (((uintptr_t)Q | (uintptr_t)K | (uintptr_t)V | (uintptr_t)O) & 15))
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mha_few32x4, dim3((unsigned)((total + 255) / 256)),
-                       dim3(256), 0, (hipStream_t)stream, Q, sq, K, sk, V, sv,
-                       O, Nq, Nk, dint, scale * LOG2E_F, total);
-    return hipGetLastError();
-}
-
 static bool aligned16(long sq, long sk, long sv)
 {
     return sq % 4 == 0 && sk % 4 == 0 && sv % 4 == 0;
@@ -290,6 +274,19 @@ extern "C" int launch_mha_fewkeys(const float *Q, long sq, const float *K,
             FEW(1) FEW(2) FEW(3) FEW(4) FEW(5) FEW(6) FEW(7) FEW(8)
         }
 #undef FEW
+        return hipGetLastError();
+    }
+    /* Four lanes per (query, head) where rows are float4s, against one lane
+     * that walks keys and channels serially: 8 x 8 tokens, 1 to 32 prompts,
+     * 48 us, 7 with four lanes. */
+    if (dint == 256 && Nk <= 8 && aligned16(sq, sk, sv) &&
+        (((uintptr_t)Q | (uintptr_t)K | (uintptr_t)V | (uintptr_t)O) & 15) == 0) {
+        const long total = (long)P * Nq * 32;
+
+        if ((total + 255) / 256 > 0x7fffffffL)
+            return hipErrorInvalidConfiguration;
+        hipLaunchKernelGGL(k_mha_few32x4, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
+                           Q, sq, K, sk, V, sv, O, Nq, Nk, dint, scale * LOG2E_F, total);
         return hipGetLastError();
     }
     {

@@ -429,13 +429,6 @@ static void mha_run(struct sam_model *m, const char *who, int noalloc, int P,
                                   be->stream);
         what = "attn_manykeys";
     }
-    else if (be->bf16 && c == 32 && Nk <= 8 && (sq | sk | sv) % 4 == 0) {
-        /* precision=bf16: the decoder's token self-attention, four lanes
-         * per (query, head) instead of the reference's one. */
-        err = launch_mha_few32x4(qp->ptr, sq, kp->ptr, sk, vp->ptr, sv,
-                                 o->ptr, P, Nq, Nk, dint, scale, be->stream);
-        what = "attn_fewkeys";
-    }
     else {
         err = launch_mha_fewkeys(qp->ptr, sq, kp->ptr, sk, vp->ptr, sv,
                                  o->ptr, P, Nq, Nk, dint, scale, be->stream);
