@@ -424,6 +424,25 @@ void convt_scatter(struct sam_model *m, hipb_mem G, hipb_mem out,
     hipb_run_end(be, err, "convt_scatter", 0.0);
 }
 
+/* The heads' weights and biases are there, of one element type, large
+ * enough and 16-byte aligned: what k_dec_heads reads. */
+static int dec_heads_ok(const struct sam_decoder *d)
+{
+    int i, j;
+
+    for (i = 0; i <= 3; i++)
+        for (j = 0; j < 3; j++) {
+            const hipb_mem W = i ? d->hyper_w[i][j] : d->iou_w[j];
+            const hipb_mem B = i ? d->hyper_b[i][j] : d->iou_b[j];
+            const size_t n = j < 2 ? SAM_DIM : i ? 32 : 4;
+
+            if (!W || !B || W->dtype != d->iou_w[0]->dtype || B->dtype != HIPB_F32 ||
+                hipb_count(W) < n * SAM_DIM || hipb_count(B) < n || ((uintptr_t)W->ptr & 15))
+                return 0;
+        }
+    return 1;
+}
+
 /* The device part of sam_decode for P prompts whose tokens are in qpe /
  * qry: the two-way transformer, the hypernetwork and IoU heads (raw IoU
  * outputs in sv), the upscaling and the logits. Host-synchronisation
@@ -469,10 +488,11 @@ static void dec_kernels(struct sam_model *m, int P)
               ACT_NONE);
 
     /* Hypernetwork MLPs of mask tokens 1..3 (into d->hyper [P][3][32])
-     * and the IoU head (4 raw outputs into d->sv): on the bf16 path one
-     * kernel for all four; else GEMMs over the P prompts' token rows (row
-     * stride NTOK x 256) with the hidden layers in d->sq / d->sk. */
-    if (d->fold_w && d->iou_w[0]->dtype == d->hyper_w[1][0]->dtype) {
+     * and the IoU head (4 raw outputs into d->sv): one kernel for all four
+     * when their weights are as it takes them; else GEMMs over the P prompts'
+     * token rows (row stride NTOK x 256) with the hidden layers in d->sq /
+     * d->sk. */
+    if (dec_heads_ok(d)) {
         const void *w0[4], *w1[4], *w2[4];
         const float *b0[4], *b1[4], *b2[4];
 

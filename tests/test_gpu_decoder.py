@@ -279,3 +279,22 @@ def test_mask_post_tile_edges(hip, be, orc, weights, oh, ow):
             assert np.array_equal(got, mask[k])
     finally:
         d.free()
+
+
+def test_decode_half_weights(hip, orc, weights):
+    """precision=fp16: the decode (its heads' kernel on half rows among it)
+    against the oracle on the same weights rounded to half."""
+    G, P = 16, 3
+    w = {k: a.astype(np.float16).astype(np.float32) if k.endswith("w") and a.ndim == 2
+         else a for k, a in weights.items()}
+    b = hip.Backend(precision="fp16")
+    d = Dec(hip, b, orc, w, G, P, 52)
+    try:
+        pts = np.random.default_rng(53).uniform(0, 14 * G, (P, 2)).astype(np.float32)
+        iou = d.dec.decode(pts)
+        oiou, olow, _, _ = orc.sam_decode(d.dw, pts, d.prep, d.s0, d.s1)
+        assert report("decode lowres half", d.dec.lowres(P), olow) <= TOL["fp32"]
+        assert np.abs(iou - oiou).max() <= TOL["fp32"]
+    finally:
+        d.free()
+        b.free()
