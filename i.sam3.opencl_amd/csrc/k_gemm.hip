@@ -406,15 +406,115 @@ __global__ __launch_bounds__(256) void k_gemm_small(gemm_desc d)
     }
 }
 
-template <int ADT>
-static void launch_small_b(const gemm_desc *d, dim3 grid, hipStream_t s)
+/* The smallest of them: a workgroup per tile of 16 MT rows x 16 columns
+ * whose NW waves split K; no operand staging: each lane loads its
+ * MFMA fragments straight from memory (A row and B row, the Linear weight, l
+ * % 16, eight consecutive k at 8 (l / 16)), v_mfma_f32_16x16x32_bf16 with f32
+ * accumulation; the partial tiles are summed through LDS in wave order, then
+ * the usual epilogue, a thread per element. Bound by latency: 4.7 us for
+ * 512 x 256 x 256 (k_gemm_small: 6.7, its tiles leave CUs idle there), 12 for
+ * 512 x 256 x 2048 (17). The same operands as
+ * k_gemm_small. */
+/* K steps of 32 whose loads a wave has in flight at once. */
+#define SMALL16_BATCH 4
+
+template <int ADT, int BDT, int MT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_small16(gemm_desc d)
+{
+    __shared__ float red[NW][MT][4][64];
+    const int t = threadIdx.x, l = t & 63, w = t >> 6, q = l >> 4, l16 = l & 15;
+    const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16;
+    const int ksteps = d.K / 32, per = (ksteps + NW - 1) / NW;
+    const int s0 = w * per, s1 = min(s0 + per, ksteps);
+    const long brow = d.boff + (long)min(n0 + l16, d.N - 1) * d.ldb + 8 * q;
+    long arow[MT];
+    f32x4 acc[MT];
+
+    for (int i = 0; i < MT; i++) {
+        arow[i] = d.aoff + (long)min(m0 + 16 * i + l16, d.M - 1) * d.lda + 8 * q;
+        acc[i] = (f32x4){};
+    }
+    for (int s = s0; s < s1; s += SMALL16_BATCH) {
+        bf16x8 a[SMALL16_BATCH][MT], b[SMALL16_BATCH];
+
+#pragma unroll
+        for (int u = 0; u < SMALL16_BATCH; u++)
+            if (s + u < s1) {
+                b[u] = frag8<BDT>(d.B, brow + 32L * (s + u));
+                for (int i = 0; i < MT; i++)
+                    a[u][i] = frag8<ADT>(d.A, arow[i] + 32L * (s + u));
+            }
+#pragma unroll
+        for (int u = 0; u < SMALL16_BATCH; u++)
+            if (s + u < s1)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i], b[u], acc[i], 0, 0,
+                                                                     0);
+    }
+    for (int i = 0; i < MT; i++)
+        for (int r = 0; r < 4; r++)
+            red[w][i][r][l] = acc[i][r];
+    __syncthreads();
+    for (int x = t; x < MT * 256; x += 64 * NW) {
+        const int i = x >> 8, r = (x >> 6) & 3, ll = x & 63;
+        const int mr = m0 + 16 * i + 4 * (ll >> 4) + r, nc = n0 + (ll & 15);
+        const long idx = (long)mr * d.ldc + nc;
+        float v = red[0][i][r][ll];
+
+        for (int p = 1; p < NW; p++)
+            v += red[p][i][r][ll];
+        if (mr >= d.M || nc >= d.N)
+            continue;
+        v = act_k(d.alpha * v + (d.bias ? d.bias[nc] : 0.0f), d.act);
+        if (d.cdt == DT_F32) {
+            if (d.R)
+                v += ((const float *)d.R)[d.roff + idx];
+            ((float *)d.C)[d.coff + idx] = v;
+        }
+        else {
+            if (d.R)
+                v += bf2f(((const uint16_t *)d.R)[d.roff + idx]);
+            ((uint16_t *)d.C)[d.coff + idx] = f2bf(v);
+        }
+    }
+}
+
+template <int ADT, int BDT> static void launch_small_ab(const gemm_desc *d, hipStream_t s)
+{
+    /* Two row tiles per workgroup once single ones would give every CU two;
+     * eight waves where four would have more than four steps each. */
+    const long t16 = (long)((d->N + 15) / 16) * ((d->M + 15) / 16);
+    const long t32 = (long)((d->N + 31) / 32) * ((d->M + 31) / 32);
+    const int mt = t16 >= 2L * dev_cu_count() ? 2 : 1;
+    const dim3 grid((d->N + 15) / 16, (d->M + 16 * mt - 1) / (16 * mt));
+
+    /* 32 x 32 tiles once they give every CU one (1024^3: 27 us against 38;
+     * 512 x 2048 x 256 11 against 14; 512 x 256 x 2048, 128 tiles, 17 against
+     * 12; 32 x 4096 x 1024 10 against 7). */
+    if (t32 > dev_cu_count()) {
+        hipLaunchKernelGGL((k_gemm_small<ADT, BDT>), dim3((d->N + 31) / 32, (d->M + 31) / 32),
+                           dim3(256), 0, s, *d);
+        return;
+    }
+    if (mt == 2 && d->K > 512)
+        hipLaunchKernelGGL((k_gemm_small16<ADT, BDT, 2, 8>), grid, dim3(512), 0, s, *d);
+    else if (mt == 2)
+        hipLaunchKernelGGL((k_gemm_small16<ADT, BDT, 2, 4>), grid, dim3(256), 0, s, *d);
+    else if (d->K > 512)
+        hipLaunchKernelGGL((k_gemm_small16<ADT, BDT, 1, 8>), grid, dim3(512), 0, s, *d);
+    else
+        hipLaunchKernelGGL((k_gemm_small16<ADT, BDT, 1, 4>), grid, dim3(256), 0, s, *d);
+}
+
+template <int ADT> static void launch_small_b(const gemm_desc *d, hipStream_t s)
 {
     if (d->bdt == DT_F32)
-        hipLaunchKernelGGL((k_gemm_small<ADT, DT_F32>), grid, dim3(256), 0, s, *d);
+        launch_small_ab<ADT, DT_F32>(d, s);
     else if (d->bdt == DT_BF16)
-        hipLaunchKernelGGL((k_gemm_small<ADT, DT_BF16>), grid, dim3(256), 0, s, *d);
+        launch_small_ab<ADT, DT_BF16>(d, s);
     else
-        hipLaunchKernelGGL((k_gemm_small<ADT, DT_F16>), grid, dim3(256), 0, s, *d);
+        launch_small_ab<ADT, DT_F16>(d, s);
 }
 
 static int vec_ok(int dt, long off, long s0, long s1, int ld)
@@ -450,13 +550,11 @@ extern "C" int launch_gemm(const gemm_desc *d, void *ws, size_t ws_bytes, void *
     if (d->mode == MODE_BF16 && d->transb && d->nb == 1 && d->K % 64 == 0 &&
         avec && bvec && (long)grid.x * grid.y <= 64 &&
         ((uintptr_t)d->A & 15) == 0 && ((uintptr_t)d->B & 15) == 0) {
-        const dim3 sg((d->N + 31) / 32, (d->M + 31) / 32);
-
         /* A is never half (the gemm wrapper rejects it). */
         if (d->adt == DT_F32)
-            launch_small_b<DT_F32>(d, sg, s);
+            launch_small_b<DT_F32>(d, s);
         else
-            launch_small_b<DT_BF16>(d, sg, s);
+            launch_small_b<DT_BF16>(d, s);
         return hipGetLastError();
     }
     if (d->mode == MODE_BF16) {

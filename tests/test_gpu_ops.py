@@ -466,3 +466,38 @@ def test_gemm_split_non_finite(hip, be, orc, M, N, K):
     fin = np.isfinite(want)
     assert np.array_equal(np.isfinite(got[:16]), fin)
     assert np.all(np.abs(got[:16][fin] - want[fin]) <= 1e-5 * np.abs(want[fin]) + 2e-4)
+
+
+@pytest.mark.parametrize("M,N,K,act,abf,cbf", [
+    (8, 256, 256, 0, False, False), (1, 4, 64, 1, False, False),
+    (17, 33, 128, 2, True, True), (512, 256, 2048, 0, False, False),
+    (512, 300, 576, 1, True, False), (40, 4000, 1088, 0, False, True),
+])
+def test_gemm_small_bf16(hip, be16, orc, M, N, K, act, abf, cbf):
+    """The bf16 path's smallest products (16-column tiles, K over the waves),
+    with bias and residual, against float64 of the bf16 operands: each element
+    within one rounding of the f32 sum (K 2^-24 of the operands' magnitude)
+    and, stored as bf16, one of the result (2^-9)."""
+    m = model(hip, be16)
+    g = rng(M + N + K + 5)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    A16 = from_bf16(to_bf16(A))
+    W = to_bf16(g.uniform(-0.06, 0.06, (N, K)).astype(np.float32))
+    bias = g.standard_normal(N, dtype=np.float32)
+    C0 = from_bf16(to_bf16(g.standard_normal((M, N), dtype=np.float32)))
+    dA = be16.upload_typed(to_bf16(A), hip.BF16) if abf else be16.upload(A)
+    dW, dv = be16.upload_typed(W, hip.BF16), be16.upload(bias)
+    dC = be16.upload_typed(to_bf16(C0), hip.BF16) if cbf else be16.upload(C0)
+    hip.linear(m, M, K, N, dA, 0, dW, dv, dC, 0, act, 1)
+    got = be16.read_f32(dC, M * N).reshape(M, N).astype(np.float64)
+    p = A16.astype(np.float64) @ from_bf16(W).T.astype(np.float64) + bias
+    if act == 1:
+        from scipy.special import erf
+        p = 0.5 * p * (1 + erf(p / np.sqrt(2)))
+    elif act == 2:
+        p = np.maximum(p, 0)
+    want = p + C0
+    tol = K * 2.0 ** -24 * np.abs(A16).max() * 0.06 * 8 + 1e-6
+    if cbf:
+        tol = tol + 2.0 ** -8 * np.abs(want)
+    assert np.all(np.abs(got - want) <= tol)
