@@ -1243,3 +1243,155 @@ extern "C" int launch_dec_heads(const float *qry, const void *const w0[4],
                            qry, hw, hyper, iou);
     return hipGetLastError();
 }
+
+/* ------------------------------------------------------------------ */
+/* Exact path: second transposed convolution                           */
+/* ------------------------------------------------------------------ */
+
+/* u2 [P][4 G2^2][32] from u1 [P][G2^2][64] on the fp32 and fp16 paths: ConvT
+ * 64 -> 32 (up3w [64][32 co][4 dd], dd = 2 dy + dx), + up3b + feat_s0, GELU,
+ * so that the product is not written and read again before its scatter (0.68
+ * GB of it for 32 prompts at 72 x 72, and a launch).
+ *
+ * Product on operands split into bf16 pieces (k_gemm_split.hip: three per
+ * float, two per half weight, piece pairs down to 2^-16), transposed: weight
+ * rows are the A operand, tokens the B operand, so a lane holds one token,
+ * and with the weight rows of a 32-row block in the order row 8 a + 4 b + e =
+ * channel 16 b + 4 a + e (block = dd) it holds 16 consecutive channels of
+ * each of the token's four output pixels, 64 contiguous bytes of u2 and of
+ * the map. A workgroup splits
+ * the weights into LDS once (48 KiB) and takes `tiles` 32-token tiles of one
+ * prompt per wave; the tokens go from memory to registers.
+ *
+ * Bound by VALU: 64 exact GELUs per lane and tile (erff, ~45 instructions)
+ * against 96 MFMAs. 32 prompts at 72 x 72: 209 us against 346 for the product
+ * and its scatter.
+ *
+ * Non-finite tokens or weights make their products NaN; such a product is
+ * formed again from the floats in k order. */
+template <int DT>
+__global__ __launch_bounds__(256, 3) void
+k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
+                 const float *__restrict__ b3, const float *__restrict__ feat,
+                 float *__restrict__ u2, int G2, int tiles)
+{
+    constexpr int NP = DT == DT_F32 ? 3 : 2;
+    constexpr int pairs[6][2] = {{2, 0}, {1, 1}, {1, 0}, {0, 2}, {0, 1}, {0, 0}};
+    __shared__ __attribute__((aligned(16))) char S[16 * NP * 1024];
+    __shared__ __attribute__((aligned(16))) float bs[32];
+    const int t = threadIdx.x, l = t & 63, w = t >> 6, h = l >> 5, l32 = l & 31;
+    const int p = blockIdx.y, T4 = G2 * G2;
+    auto weight = [&](int k, int n) {
+        return DT == DT_F32 ? ((const float *)W)[k * 128 + n]
+                            : h2f(((const uint16_t *)W)[k * 128 + n]);
+    };
+
+    for (int i = t; i < 1024; i += 256) {
+        /* Column n, k octet o: eight loads, lanes along n. */
+        const int n = i & 127, o = i >> 7, co = n >> 2, dd = n & 3;
+        const int row = 8 * ((co >> 2) & 3) + 4 * (co >> 4) + (co & 3);
+        u32x2 lo[NP], hi[NP];
+        f32x4 x, y;
+        char *q = S + (dd * 4 + (o >> 1)) * NP * 1024 + 16 * (32 * (o & 1) + row);
+
+        for (int e = 0; e < 4; e++) {
+            x[e] = weight(8 * o + e, n);
+            y[e] = weight(8 * o + 4 + e, n);
+        }
+        split4<NP>(x, lo);
+        split4<NP>(y, hi);
+        for (int e = 0; e < NP; e++)
+            *(u32x4 *)(q + 1024 * e) = (u32x4){lo[e].x, lo[e].y, hi[e].x, hi[e].y};
+    }
+    if (t < 32)
+        bs[t] = b3[t];
+    __syncthreads();
+
+    const int first = (blockIdx.x * 4 + w) * tiles;
+
+    for (int tile = first; tile < first + tiles && tile * 32 < T4; tile++) {
+        const int m = tile * 32 + l32, mc = min(m, T4 - 1);
+        const float *xr = u1 + ((long)p * T4 + mc) * 64 + 8 * h;
+        const int yy = mc / G2, xx = mc - yy * G2;
+        bf16x8 x[4][3];
+        f32x16 acc[4];
+
+        for (int s = 0; s < 4; s++) {
+            u32x2 lo[3], hi[3];
+
+            split4<3>(*(const f32x4 *)(xr + 16 * s), lo);
+            split4<3>(*(const f32x4 *)(xr + 16 * s + 4), hi);
+            for (int e = 0; e < 3; e++)
+                x[s][e] =
+                    __builtin_bit_cast(bf16x8, (u32x4){lo[e].x, lo[e].y, hi[e].x, hi[e].y});
+        }
+#pragma unroll
+        for (int dd = 0; dd < 4; dd++) {
+            acc[dd] = (f32x16){};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                bf16x8 wf[NP];
+
+                for (int e = 0; e < NP; e++)
+                    wf[e] = *(const bf16x8 *)(S + ((dd * 4 + s) * NP + e) * 1024 + 16 * l);
+#pragma unroll
+                for (int q = 0; q < 6; q++)
+                    if (pairs[q][1] < NP)
+                        acc[dd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            wf[pairs[q][1]], x[s][pairs[q][0]], acc[dd], 0, 0, 0);
+            }
+        }
+        if (m >= T4)
+            continue;
+#pragma unroll
+        for (int dd = 0; dd < 4; dd++) {
+            const long px = (long)(2 * yy + (dd >> 1)) * 2 * G2 + 2 * xx + (dd & 1);
+            const float *fs = feat + px * 32 + 16 * h;
+            float *o = u2 + ((long)p * 4 * T4 + px) * 32 + 16 * h;
+
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                const f32x4 f = *(const f32x4 *)(fs + 4 * a);
+                const f32x4 b = *(const f32x4 *)&bs[16 * h + 4 * a];
+                f32x4 v;
+
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float g = acc[dd][4 * a + e];
+
+                    if (!(fabsf(g) < INFINITY)) {
+                        g = 0.0f;
+                        for (int k = 0; k < 64; k++)
+                            g = fmaf(xr[k - 8 * h], weight(k, 4 * (16 * h + 4 * a + e) + dd), g);
+                    }
+                    v[e] = act_k(g + b[e] + f[e], ACT_GELU_K);
+                }
+                *(f32x4 *)(o + 4 * a) = v;
+            }
+        }
+    }
+}
+
+extern "C" int launch_upscale2_split(const float *u1, const void *W, int dt, const float *b3,
+                                     const float *feat, float *u2, int G2, int P, int cus,
+                                     void *stream)
+{
+    const long total = ((long)G2 * G2 + 31) / 32 * P;
+    /* Three workgroups of four waves per CU, each with as many tiles as that
+     * takes, at least two (the weights' split is about half a tile's work). */
+    long tiles = (total + 12L * cus - 1) / (12L * cus);
+    const long per = ((long)G2 * G2 + 31) / 32;
+
+    if (P < 1 || P > 65535 || G2 < 1 || G2 > 16384)
+        return hipErrorInvalidConfiguration;
+    tiles = tiles < 2 ? 2 : tiles > 64 ? 64 : tiles;
+    const dim3 g((unsigned)((per + 4 * tiles - 1) / (4 * tiles)), P);
+
+    if (dt == DT_F32)
+        hipLaunchKernelGGL(k_upscale2_split<DT_F32>, g, dim3(256), 0, (hipStream_t)stream, u1, W,
+                           b3, feat, u2, G2, (int)tiles);
+    else
+        hipLaunchKernelGGL(k_upscale2_split<DT_F16>, g, dim3(256), 0, (hipStream_t)stream, u1, W,
+                           b3, feat, u2, G2, (int)tiles);
+    return hipGetLastError();
+}

@@ -443,6 +443,19 @@ static int dec_heads_ok(const struct sam_decoder *d)
     return 1;
 }
 
+/* The second upscaling's operands are as launch_upscale2_split reads them
+ * (a caller's may not be: the operators then report or take them). */
+static int upscale2_ok(const struct sam_model *m, const struct sam_decoder *d)
+{
+    const size_t pix = (size_t)16 * m->grid * m->grid;
+
+    return d->up3w && d->up3b && d->feat_s0 &&
+           (d->up3w->dtype == HIPB_F32 || d->up3w->dtype == HIPB_F16) &&
+           d->up3b->dtype == HIPB_F32 && d->feat_s0->dtype == HIPB_F32 &&
+           hipb_count(d->up3w) >= 64 * 128 && hipb_count(d->up3b) >= 32 &&
+           hipb_count(d->feat_s0) >= pix * 32 && ((uintptr_t)d->feat_s0->ptr & 15) == 0;
+}
+
 /* The device part of sam_decode for P prompts whose tokens are in qpe /
  * qry: the two-way transformer, the hypernetwork and IoU heads (raw IoU
  * outputs in sv), the upscaling and the logits. Host-synchronisation
@@ -556,8 +569,8 @@ static void dec_kernels(struct sam_model *m, int P)
     }
     else {
         /* Output upscaling: ConvT 256 -> 64 + feat_s1, LayerNorm2d, GELU,
-         * ConvT 64 -> 32 + feat_s0, GELU (the kin buffer holds the first
-         * GEMM), then the logits. */
+         * ConvT 64 -> 32 + feat_s0, GELU (in one launch where the operands
+         * allow it; the kin buffer holds the first GEMM), then the logits. */
         gemm(m, (int)(P * T), 256, SAM_DIM, mat(d->keys, 0, SAM_DIM),
              mat(d->up0w, 0, 256), 0, mat(d->kin, 0, 256), 1, 1, NULL, NULL,
              0, 1.0f, ACT_NONE);
@@ -565,11 +578,20 @@ static void dec_kernels(struct sam_model *m, int P)
                       ACT_NONE);
         layernorm(m, P * 4 * T, 64, d->u1, d->u1, d->up1w, d->up1b, LN2D_EPS,
                   ACT_GELU);
-        gemm(m, (int)(P * 4 * T), 128, 64, mat(d->u1, 0, 64),
-             mat(d->up3w, 0, 128), 0, mat(d->g2, 0, 128), 1, 1, NULL, NULL, 0,
-             1.0f, ACT_NONE);
-        convt_scatter(m, d->g2, d->u2, d->up3b, d->feat_s0, P, 2 * G, 2 * G,
-                      32, ACT_GELU);
+        if (hipb_failed())
+            return;
+        if (upscale2_ok(m, d)) {
+            hipb_run_begin(m->hip);
+            err = launch_upscale2_split(d->u1->ptr, d->up3w->ptr, d->up3w->dtype, d->up3b->ptr,
+                                        d->feat_s0->ptr, d->u2->ptr, 2 * G, P,
+                                        m->hip->cu_count, m->hip->stream);
+            hipb_run_end(m->hip, err, "upscale2", 2.0 * P * 4 * T * 64.0 * 128);
+        }
+        else {
+            gemm(m, (int)(P * 4 * T), 128, 64, mat(d->u1, 0, 64), mat(d->up3w, 0, 128), 0,
+                 mat(d->g2, 0, 128), 1, 1, NULL, NULL, 0, 1.0f, ACT_NONE);
+            convt_scatter(m, d->g2, d->u2, d->up3b, d->feat_s0, P, 2 * G, 2 * G, 32, ACT_GELU);
+        }
         mask_logits(m, d->u2, d->hyper, d->lowres, P, (int)(16 * T));
     }
 }

@@ -310,6 +310,12 @@ int launch_t2i_fused(const float *keys, const void *pk16, const void *U16,
                      int wv_dt, const float *bv, float *o, int T, int P,
                      int nsplit, void *stream);
 
+/* Exact path: u2 [P][4 G2^2][32] from u1 [P][G2^2][64] through the second
+ * transposed convolution (W [64][32 x 4], float or half), bias, map feat
+ * [4 G2^2][32] and GELU; 16-byte aligned rows. */
+int launch_upscale2_split(const float *u1, const void *W, int dt, const float *b3,
+                          const float *feat, float *u2, int G2, int P, int cus,
+                          void *stream);
 /* The decoder's IoU head (head 0, token 1, 4 raw outputs into iou [P][4])
  * and hypernetwork MLPs (heads 1..3, tokens 3..5, into hyper [P][3][32])
  * on qry [P][8][256]: three Linear layers each, weights of element type
