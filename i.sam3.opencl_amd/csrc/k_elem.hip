@@ -208,6 +208,59 @@ __global__ __launch_bounds__(256) void k_layernorm_w(
     }
 }
 
+/* The decoder's image keys after an image -> token block, rows of 256, one
+ * wave per row: x = X (+ add[row % T]), Y = LayerNorm(x), and with pe Y2 = Y +
+ * pe[row % T]: the residual with the shared source tokens, norm4 and the next
+ * block's keys + PE in one pass over memory instead of three launches that
+ * each read and write the map (32 prompts at 72 x 72, layer 0: 97 us against
+ * 220).
+ * Bound by memory. The arithmetic is k_layernorm_w's. */
+__global__ __launch_bounds__(256) void k_keys_norm(const float *__restrict__ X,
+                                                   const float *__restrict__ add,
+                                                   const float *__restrict__ g,
+                                                   const float *__restrict__ bt, float eps,
+                                                   const float *__restrict__ pe, float *Y,
+                                                   float *__restrict__ Y2, long rows, int T)
+{
+    const int l = threadIdx.x & 63;
+    const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+
+    if (r >= rows)
+        return;
+    const long at = r * 256 + 4 * l, sh = r % T * 256 + 4 * l;
+    f32x4 v = *(const f32x4 *)(X + at);
+    const f32x4 gv = *(const f32x4 *)(g + 4 * l), bv = *(const f32x4 *)(bt + 4 * l);
+    f32x4 pv = {};
+
+    if (add)
+        v += *(const f32x4 *)(add + sh);
+    if (pe)
+        pv = *(const f32x4 *)(pe + sh);
+    const float mean = wave_sum_rows((v.x + v.y) + (v.z + v.w)) / 256.0f;
+    const f32x4 dv = v - mean;
+    const float var =
+        wave_sum_rows(fmaf(dv.x, dv.x, fmaf(dv.y, dv.y, fmaf(dv.z, dv.z, dv.w * dv.w)))) / 256.0f;
+    const float rs = 1.0f / sqrtf(var + eps);
+    f32x4 o;
+
+    for (int e = 0; e < 4; e++)
+        o[e] = fmaf((v[e] - mean) * rs, gv[e], bv[e]);
+    *(f32x4 *)(Y + at) = o;
+    if (pe)
+        *(f32x4 *)(Y2 + at) = o + pv;
+}
+
+extern "C" int launch_keys_norm(const float *X, const float *add, const float *g, const float *b,
+                                float eps, const float *pe, float *Y, float *Y2, long rows, int T,
+                                void *stream)
+{
+    if (rows < 1 || (rows + 3) / 4 > 0x7fffffffL || T < 1)
+        return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL(k_keys_norm, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
+                       (hipStream_t)stream, X, add, g, b, eps, pe, Y, Y2, rows, T);
+    return hipGetLastError();
+}
+
 /* Narrow rows (C = 4 LPR floats, LPR = 8, 16 or 32 lanes per row): 256 / LPR
  * rows per workgroup, a lane holds one float4 of its row, the sums close
  * with butterflies inside the lane group. No window partition. */

@@ -208,7 +208,8 @@ void sam_dec_prepare(struct sam_model *m)
     hipb_release(&nm);
 }
 
-void t2i_attention(struct sam_model *m, int P, const struct sam_attn_w *a)
+/* t2i_attention; have_kin: kin holds keys + PE already (fp32 path). */
+static void t2i_run(struct sam_model *m, int P, const struct sam_attn_w *a, int have_kin)
 {
     struct sam_decoder *d = dec_of(m, "t2i_attention");
     const long T = (long)m->grid * m->grid, n = (long)P * NTOK * SAM_DIM;
@@ -267,7 +268,8 @@ void t2i_attention(struct sam_model *m, int P, const struct sam_attn_w *a)
                ACT_NONE, 1);
         return;
     }
-    add_bcast(m, d->kin, d->keys, d->pe_img, P * T * SAM_DIM, T * SAM_DIM);
+    if (!have_kin)
+        add_bcast(m, d->kin, d->keys, d->pe_img, P * T * SAM_DIM, T * SAM_DIM);
     linear(m, P * NTOK, SAM_DIM, 128, d->qin, 0, a->qw, a->qb, d->sq, 0,
            ACT_NONE, 0);
     linear(m, (int)(P * T), SAM_DIM, 128, d->kin, 0, a->kw, a->kb, d->bk, 0,
@@ -280,18 +282,35 @@ void t2i_attention(struct sam_model *m, int P, const struct sam_attn_w *a)
            ACT_NONE, 1);
 }
 
-void i2t_attention(struct sam_model *m, int layer, int P)
+void t2i_attention(struct sam_model *m, int P, const struct sam_attn_w *a)
+{
+    t2i_run(m, P, a, 0);
+}
+
+/* norm4's operands are as launch_keys_norm reads them (its other buffers are
+ * sam_dec_init's own). */
+static int keys_norm_ok(const struct sam_dec_layer *L)
+{
+    return L->n4w && L->n4b && L->n4w->dtype == HIPB_F32 && L->n4b->dtype == HIPB_F32 &&
+           hipb_count(L->n4w) >= SAM_DIM && hipb_count(L->n4b) >= SAM_DIM &&
+           (((uintptr_t)L->n4w->ptr | (uintptr_t)L->n4b->ptr) & 15) == 0;
+}
+
+/* i2t_attention; on the fp32 path with want_kin also kin = keys + PE of the
+ * updated keys. Returns whether kin was written. */
+static int i2t_run(struct sam_model *m, int layer, int P, int want_kin)
 {
     struct sam_decoder *d = dec_of(m, "i2t_attention");
     const long T = (long)m->grid * m->grid, n = (long)P * NTOK * SAM_DIM;
     const struct sam_dec_layer *L;
+    int fused, err;
 
     if (!d)
-        return;
+        return 0;
     if (P < 1 || P > d->batch || layer < 0 || layer > 1) {
         hipb_fatal("i2t_attention: layer %d, %d prompts for a batch of %d",
                    layer, P, d->batch);
-        return;
+        return 0;
     }
     L = &d->layers[layer];
     add_bcast(m, d->qin, d->qry, d->qpe, n, n);
@@ -301,14 +320,13 @@ void i2t_attention(struct sam_model *m, int layer, int P)
          * on the fly in layer 1, so kin is not read). */
         struct hipb_backend *be = m->hip;
         const float s = 1.4426950408889634f / sqrtf(16.0f);
-        int err;
 
         linear(m, P * NTOK, SAM_DIM, 128, d->qin, 0, L->i2t.kw, L->i2t.kb,
                d->sk, 0, ACT_NONE, 0);
         linear(m, P * NTOK, SAM_DIM, 128, d->qry, 0, L->i2t.vw, L->i2t.vb,
                d->sv, 0, ACT_NONE, 0);
         if (hipb_failed())
-            return;
+            return 0;
         hipb_run_begin(be);
         err = launch_i2t_fold(d->sk->ptr, d->sv->ptr, layer,
                               layer ? L->i2t.qw->ptr : NULL,
@@ -329,8 +347,9 @@ void i2t_attention(struct sam_model *m, int layer, int P)
                                be->stream);
         hipb_run_end(be, err, "i2t_fused",
                      4.0 * P * T * 64.0 * ((layer ? 256 : 128) + SAM_DIM));
-        return;
+        return 0;
     }
+    fused = keys_norm_ok(L);
     if (layer == 0) {
         linear(m, P * NTOK, SAM_DIM, 128, d->qin, 0, L->i2t.kw, L->i2t.kb,
                d->sk, 0, ACT_NONE, 0);
@@ -340,7 +359,8 @@ void i2t_attention(struct sam_model *m, int layer, int P)
             NTOK * 128, d->bo);
         linear(m, (int)(P * T), 128, SAM_DIM, d->bo, 0, L->i2t.ow, L->i2t.ob,
                d->keys, 0, ACT_NONE, 0);
-        add_bcast(m, d->keys, d->keys, d->src, P * T * SAM_DIM, T * SAM_DIM);
+        if (!fused)
+            add_bcast(m, d->keys, d->keys, d->src, P * T * SAM_DIM, T * SAM_DIM);
     }
     else {
         linear(m, (int)(P * T), SAM_DIM, 128, d->kin, 0, L->i2t.qw,
@@ -354,8 +374,23 @@ void i2t_attention(struct sam_model *m, int layer, int P)
         linear(m, (int)(P * T), 128, SAM_DIM, d->bo, 0, L->i2t.ow, L->i2t.ob,
                d->keys, 0, ACT_NONE, 1);
     }
-    layernorm(m, P * T, SAM_DIM, d->keys, d->keys, L->n4w, L->n4b, DEC_EPS,
-              ACT_NONE);
+    if (hipb_failed())
+        return 0;
+    if (!fused) {
+        layernorm(m, P * T, SAM_DIM, d->keys, d->keys, L->n4w, L->n4b, DEC_EPS, ACT_NONE);
+        return 0;
+    }
+    hipb_run_begin(m->hip);
+    err = launch_keys_norm(d->keys->ptr, layer ? NULL : d->src->ptr, L->n4w->ptr, L->n4b->ptr,
+                           DEC_EPS, want_kin ? d->pe_img->ptr : NULL, d->keys->ptr, d->kin->ptr,
+                           P * T, (int)T, m->hip->stream);
+    hipb_run_end(m->hip, err, "keys_norm", 0.0);
+    return want_kin;
+}
+
+void i2t_attention(struct sam_model *m, int layer, int P)
+{
+    i2t_run(m, layer, P, 0);
 }
 
 /* Prompt-token self attention (sam3_model.c:1274-1286 for layer 0, no
@@ -466,7 +501,7 @@ static void dec_kernels(struct sam_model *m, int P)
     const int G = m->grid;
     const long T = (long)G * G, n = (long)P * NTOK * SAM_DIM;
     const struct sam_dec_layer *L0 = &d->layers[0], *L1 = &d->layers[1];
-    int i, err;
+    int i, err, kin;
 
     /* Layer 0: self attention, token -> image attention on the shared
      * image keys (stride 0), token MLP, image -> token attention. */
@@ -483,20 +518,20 @@ static void dec_kernels(struct sam_model *m, int P)
     token_mlp(m, P, L0);
     layernorm(m, P * NTOK, SAM_DIM, d->qry, d->qry, L0->n3w, L0->n3b,
               DEC_EPS, ACT_NONE);
-    i2t_attention(m, 0, P);
+    kin = i2t_run(m, 0, P, 1);
 
     /* Layer 1. */
     self_attention(m, 1, P);
-    t2i_attention(m, P, &L1->t2i);
+    t2i_run(m, P, &L1->t2i, kin);
     layernorm(m, P * NTOK, SAM_DIM, d->qry, d->qry, L1->n2w, L1->n2b,
               DEC_EPS, ACT_NONE);
     token_mlp(m, P, L1);
     layernorm(m, P * NTOK, SAM_DIM, d->qry, d->qry, L1->n3w, L1->n3b,
               DEC_EPS, ACT_NONE);
-    i2t_attention(m, 1, P);
+    kin = i2t_run(m, 1, P, 1);
 
     /* Final token -> image attention. */
-    t2i_attention(m, P, &d->final_t2i);
+    t2i_run(m, P, &d->final_t2i, kin);
     layernorm(m, P * NTOK, SAM_DIM, d->qry, d->qry, d->nfw, d->nfb, DEC_EPS,
               ACT_NONE);
 

@@ -86,6 +86,12 @@ int launch_layernorm(const float *X, void *Y, int ydt, const float *g,
                      const float *b, long rows, int C, float eps, int act,
                      int H, int ws, int nwx, void *stream);
 
+/* Rows of 256, 16-byte aligned: Y = LayerNorm(X (+ add[row % T])), and with pe
+ * Y2 = Y + pe[row % T]; Y may alias X. */
+int launch_keys_norm(const float *X, const float *add, const float *g, const float *b,
+                     float eps, const float *pe, float *Y, float *Y2, long rows, int T,
+                     void *stream);
+
 int launch_softmax_rows(float *S, long rows, int L, void *stream);
 /* softmax_ext: causal mask or box bias, then the row softmax; rows =
  * heads x Nq, heads from h0 (dy / dx NULL for no bias). */

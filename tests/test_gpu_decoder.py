@@ -298,3 +298,20 @@ def test_decode_half_weights(hip, orc, weights):
     finally:
         d.free()
         b.free()
+
+
+@pytest.mark.parametrize("G,P", [(15, 1), (15, 3), (9, 2)])
+def test_decode_odd_grid(hip, be, orc, weights, G, P):
+    """Odd grids: token counts that no tile, row group or wave of the image
+    token kernels divides, prompts starting inside them."""
+    d = Dec(hip, be, orc, weights, G, P, 60 + G)
+    try:
+        pts = np.random.default_rng(G).uniform(0, 14 * G, (P, 2)).astype(np.float32)
+        iou = d.dec.decode(pts)
+        oiou, olow, _, _ = orc.sam_decode(d.dw, pts, d.prep, d.s0, d.s1)
+        tol = TOL[be.precision]
+        assert report("decode odd G=%d P=%d %s" % (G, P, be.precision), d.dec.lowres(P),
+                      olow) <= tol
+        assert np.abs(iou - oiou).max() <= 4 * tol
+    finally:
+        d.free()
