@@ -271,6 +271,46 @@ k_mask_post(const float *__restrict__ lowres, const int *__restrict__ sel, int L
     }
 }
 
+/* Up to 256 plane numbers by value, so that they travel with the launch. */
+struct mask_sel {
+    int v[256];
+};
+
+/* sel[i0 + i] and the empty statistics of masks i0 .. i0 + n - 1. */
+__global__ __launch_bounds__(256) void k_mask_init(mask_sel s, int n, int i0,
+                                                   int *__restrict__ sel,
+                                                   int *__restrict__ stats)
+{
+    const int i = threadIdx.x;
+
+    if (i >= n)
+        return;
+    int *st = stats + 6 * (i0 + i);
+
+    sel[i0 + i] = s.v[i];
+    st[0] = st[1] = 0;
+    st[2] = st[3] = 0x7fffffff;
+    st[4] = st[5] = -1;
+}
+
+/* The masks' plane numbers (host) and empty statistics into device memory,
+ * without a transfer that the host would wait for (about 10 us each). */
+extern "C" int launch_mask_init(const int *hsel, int n, int *sel, int *stats, void *stream)
+{
+    for (int i0 = 0; i0 < n; i0 += 256) {
+        const int c = n - i0 < 256 ? n - i0 : 256;
+        mask_sel s;
+
+        for (int i = 0; i < c; i++)
+            s.v[i] = hsel[i0 + i];
+        for (int i = c; i < 256; i++)
+            s.v[i] = 0;
+        hipLaunchKernelGGL(k_mask_init, dim3(1), dim3(256), 0, (hipStream_t)stream, s, c, i0, sel,
+                           stats);
+    }
+    return hipGetLastError();
+}
+
 extern "C" int launch_mask_post(const float *lowres, const int *sel, int n,
                                 int L, int out_h, int out_w, float offset,
                                 unsigned char *mask, int *stats, void *stream)

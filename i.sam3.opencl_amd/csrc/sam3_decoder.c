@@ -873,16 +873,11 @@ void sam_postprocess(struct sam_model *m, int n, const int *sel, int out_h,
             return;
         d->mask_cap = need;
     }
-    for (i = 0; i < n; i++) {
-        stats[6 * i + 0] = 0;
-        stats[6 * i + 1] = 0;
-        stats[6 * i + 2] = 0x7fffffff;
-        stats[6 * i + 3] = 0x7fffffff;
-        stats[6 * i + 4] = -1;
-        stats[6 * i + 5] = -1;
-    }
-    hipb_write(m->hip, d->sel, 0, sel, n * sizeof(int));
-    hipb_write(m->hip, d->stats, 0, stats, 6 * n * sizeof(int));
+    hipb_run_begin(m->hip);
+    err = launch_mask_init(sel, n, d->sel->ptr, d->stats->ptr, m->hip->stream);
+    hipb_run_end(m->hip, err, "mask_init", 0.0);
+    if (hipb_failed())
+        return;
     hipb_run_begin(m->hip);
     err = launch_mask_post(d->lowres->ptr, d->sel->ptr, n, L, out_h, out_w,
                            offset, d->mask->ptr, d->stats->ptr,

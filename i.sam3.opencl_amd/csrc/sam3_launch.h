@@ -252,6 +252,9 @@ int launch_convt_scatter(const float *G, float *out, const float *bias,
 /* Low-resolution logits out [P][3][npix] = hyper [P][3][32] . U [P][npix][32]. */
 int launch_mask_logits(const float *U, const float *hyper, float *out, int P,
                        int npix, void *stream);
+/* sel[0 .. n) from the host's hsel, and the empty statistics [n][6] that
+ * launch_mask_post adds to. */
+int launch_mask_init(const int *hsel, int n, int *sel, int *stats, void *stream);
 /* Bilinear resize of n selected L x L logit planes to out_h x out_w
  * binary masks, with per-mask counts and bounding boxes accumulated into
  * stats [n][6] (initialised by the caller). */

@@ -315,3 +315,21 @@ def test_decode_odd_grid(hip, be, orc, weights, G, P):
         assert np.abs(iou - oiou).max() <= 4 * tol
     finally:
         d.free()
+
+
+def test_postprocess_many_planes(hip, be, orc, weights):
+    """More planes than one launch carries plane numbers (300 > 256), each
+    selected from three."""
+    G = 4
+    d = Dec(hip, be, orc, weights, G, 100, 61)
+    try:
+        L = 4 * G
+        low = np.random.default_rng(62).standard_normal((300, L, L)).astype(np.float32)
+        sel = np.random.default_rng(63).integers(0, 300, 300).astype(np.int32)
+        be.write(d.dec.buf("lowres"), 0, low)
+        stats = d.dec.postprocess(sel, 21, 33, 0.3, False)
+        _, mask, want = orc.postprocess(low, sel, 21, 33, 0.3, False)
+        assert np.array_equal(stats, want)
+        assert np.array_equal(d.dec.read_mask(299, 21, 33, 0, 0, 32, 20), mask[299])
+    finally:
+        d.free()
