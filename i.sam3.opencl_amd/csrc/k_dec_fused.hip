@@ -67,13 +67,12 @@ __device__ __forceinline__ int yt_row(int kappa)
  * score term). Row r of Wt is (h, t) = (r / 8, r % 8). The token -> image
  * attention uses the same fold for its queries (sk = projected queries,
  * Wq = the key projection, no bq or Wo). */
+template <int DT>
 __global__ __launch_bounds__(256) void k_i2t_fold(const float *__restrict__ sk,
                                                   const float *__restrict__ sv,
-                                                  int layer, const void *Wq,
-                                                  int wq_dt,
+                                                  int layer, const void *Wq, int wq_dt,
                                                   const float *__restrict__ bq,
-                                                  const void *Wo, int wo_dt,
-                                                  float s,
+                                                  const void *Wo, int wo_dt, float s,
                                                   uint16_t *__restrict__ Wt16,
                                                   float *__restrict__ bt,
                                                   uint16_t *__restrict__ YT16,
@@ -99,7 +98,7 @@ __global__ __launch_bounds__(256) void k_i2t_fold(const float *__restrict__ sk,
         float w[16];
 
         for (int c = 0; c < 16; c++)
-            w[c] = wld(Wq, wq_dt, (long)(16 * h + c) * 256 + t);
+            w[c] = wld(Wq, DT >= 0 ? DT : wq_dt, (long)(16 * h + c) * 256 + t);
         for (int tk = 0; tk < 8; tk++) {
             float acc = 0.0f;
 
@@ -137,13 +136,18 @@ __global__ __launch_bounds__(256) void k_i2t_fold(const float *__restrict__ sk,
         float wo[16];
 
         for (int c = 0; c < 16; c++)
-            wo[c] = wld(Wo, wo_dt, (long)t * 128 + 16 * h + c);
-        for (int tk = 0; tk < 8; tk++) {
-            float acc = 0.0f;
+            wo[c] = wld(Wo, DT >= 0 ? DT : wo_dt, (long)t * 128 + 16 * h + c);
+        /* Tokens 0..3 and 4..7 land in four consecutive columns each. */
+        for (int q = 0; q < 2; q++) {
+            float y[4];
 
-            for (int c = 0; c < 16; c++)
-                acc = fmaf(wo[c], vs[tk][c], acc);
-            yt[yt_row(8 * h + tk)] = f2bf(acc);
+            for (int tk = 0; tk < 4; tk++) {
+                y[tk] = 0.0f;
+                for (int c = 0; c < 16; c++)
+                    y[tk] = fmaf(wo[c], vs[4 * q + tk][c], y[tk]);
+            }
+            *(u32x2 *)(yt + yt_row(8 * h + 4 * q)) =
+                (u32x2){pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
         }
     }
 }
@@ -156,9 +160,14 @@ extern "C" int launch_i2t_fold(const float *sk, const float *sv, int layer,
 {
     if (P < 1 || (layer && !Wq) || (!layer && !Wo) || (!layer && Kc16))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_i2t_fold, dim3(P, 8), dim3(256), 0, (hipStream_t)stream,
-                       sk, sv, layer, Wq, wq_dt, bq, Wo, wo_dt, s,
-                       (uint16_t *)Wt16, bt, (uint16_t *)YT16, (uint16_t *)Kc16);
+    /* bf16 weights (what precision=bf16 uploads) with the type known, so that
+     * their loads go out together; any other by wld's branch. */
+    auto kern = (!Wq || wq_dt == DT_BF16) && (!Wo || wo_dt == DT_BF16) ? k_i2t_fold<DT_BF16>
+                                                                       : k_i2t_fold<-1>;
+
+    hipLaunchKernelGGL(kern, dim3(P, 8), dim3(256), 0, (hipStream_t)stream, sk, sv, layer, Wq,
+                       wq_dt, bq, Wo, wo_dt, s, (uint16_t *)Wt16, bt, (uint16_t *)YT16,
+                       (uint16_t *)Kc16);
     return hipGetLastError();
 }
 
@@ -1045,83 +1054,116 @@ __global__ __launch_bounds__(256, 2) void k_t2i_fused(
     }
 }
 
-/* Z [P][64][256] from the nsplit partial records: thread per (p, row, d). */
-__global__ __launch_bounds__(256) void k_t2i_merge(const float *__restrict__ part,
-                                                   float *__restrict__ Z, int P,
-                                                   int nsplit)
+/* o [P][8][128] from the nsplit partial records: workgroup (p, h) merges rows
+ * 8 h .. + 7 into Z (thread = column, the records' rows read whole), left in
+ * LDS, then o[p][i][16 h + c] = Wv[16 h + c] . Z[8 h + i] + bv: eight lanes per
+ * Wv row (row_dot8's loads), threads 0..127 the first four tokens, the rest
+ * the others. One launch; with the merge and the products apart and Wv staged
+ * element by element 13 + 19 us at 64 prompts, now 9.6. */
+#define T2I_MAX_SPLIT 1024 /* two per CU at most are asked for */
+
+template <int DT>
+__global__ __launch_bounds__(256) void k_t2i_end(const float *__restrict__ part, const void *Wv,
+                                                 const float *__restrict__ bv,
+                                                 float *__restrict__ o, int P, int nsplit)
 {
-    const long gid = (long)blockIdx.x * 256 + threadIdx.x;
-
-    if (gid >= (long)P * FOLD_ROWS * 256)
-        return;
-    const int d = (int)(gid & 255);
-    const long pr = gid >> 8; /* p * 64 + row */
-    const int p = (int)(pr / FOLD_ROWS), row = (int)(pr % FOLD_ROWS);
-    const float *ml = part + (long)P * nsplit * FOLD_ROWS * 256;
-    float M = -INFINITY;
-
-    for (int s = 0; s < nsplit; s++)
-        M = fmaxf(M, ml[(((long)p * nsplit + s) * FOLD_ROWS + row) * 2]);
-    float num = 0.0f, den = 0.0f;
-
-    for (int s = 0; s < nsplit; s++) {
-        const long rec = ((long)p * nsplit + s) * FOLD_ROWS + row;
-        const float ms = ml[rec * 2];
-        const float wgt = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-
-        num = fmaf(wgt, part[rec * 256 + d], num);
-        den = fmaf(wgt, ml[rec * 2 + 1], den);
-    }
-    Z[gid] = num / den;
-}
-
-/* o [P][8][128]: o[p][i][16 h + c] = Wv[16 h + c] . Z[p][8 h + i] + bv.
- * Workgroup (p, h): Z rows 8 h .. + 7 and Wv rows 16 h .. + 15 staged in
- * LDS (Wv rows padded to 257 floats), thread (i, c) one dot product. */
-__global__ __launch_bounds__(128) void k_t2i_unfold(const float *__restrict__ Z,
-                                                    const void *Wv, int wv_dt,
-                                                    const float *__restrict__ bv,
-                                                    float *__restrict__ o, int P)
-{
-    __shared__ float zs[8][256], ws[16][257];
+    constexpr int E = DT == DT_F32 ? 4 : 8, N = 256 / (8 * E);
+    __shared__ __attribute__((aligned(16))) float zs[8][256];
+    __shared__ float wgt[8 * T2I_MAX_SPLIT], den[8];
     const int p = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
-    const float *zr = Z + ((long)p * FOLD_ROWS + 8 * h) * 256;
+    const int q = t & 7, c = (t >> 3) & 15, i0 = 4 * (t >> 7);
+    const float *ml = part + (long)P * nsplit * FOLD_ROWS * 256;
+    const u32x4 *wr = (const u32x4 *)((const char *)Wv +
+                                      (long)(16 * h + c) * 256 * (DT == DT_F32 ? 4 : 2));
+    u32x4 wv[N];
 
-    for (int x = t; x < 8 * 256; x += 128)
-        zs[x / 256][x % 256] = zr[x];
-    for (int x = t; x < 16 * 256; x += 128)
-        ws[x / 256][x % 256] = wld(Wv, wv_dt, (long)16 * h * 256 + x);
+    for (int i = 0; i < N; i++)
+        wv[i] = wr[8 * i + q];
+    {
+        /* The 8 rows' split weights, 32 lanes a row, then their sum. */
+        const int i = t >> 5, l = t & 31;
+        const float *mr = ml + ((long)p * nsplit * FOLD_ROWS + 8 * h + i) * 2;
+        float M = -INFINITY, d = 0.0f;
+
+        for (int s = l; s < nsplit; s += 32)
+            M = fmaxf(M, mr[(long)s * FOLD_ROWS * 2]);
+        for (int x = 16; x > 0; x >>= 1)
+            M = fmaxf(M, __shfl_xor(M, x, 64));
+        for (int s = l; s < nsplit; s += 32) {
+            const float ms = mr[(long)s * FOLD_ROWS * 2];
+            const float w = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
+
+            wgt[i * nsplit + s] = w;
+            d = fmaf(w, mr[(long)s * FOLD_ROWS * 2 + 1], d);
+        }
+        for (int x = 16; x > 0; x >>= 1)
+            d += __shfl_xor(d, x, 64);
+        if (l == 0)
+            den[i] = d;
+    }
     __syncthreads();
-    const int i = t / 16, c = t % 16;
-    float acc = bv[16 * h + c];
+    for (int i = 0; i < 8; i++) {
+        const float *pr = part + ((long)p * nsplit * FOLD_ROWS + 8 * h + i) * 256 + t;
+        float num = 0.0f;
 
-    for (int d = 0; d < 256; d++)
-        acc = fmaf(ws[c][d], zs[i][d], acc);
-    o[((long)p * 8 + i) * 128 + 16 * h + c] = acc;
+#pragma unroll 8
+        for (int s = 0; s < nsplit; s++)
+            num = fmaf(wgt[i * nsplit + s], pr[(long)s * FOLD_ROWS * 256], num);
+        zs[i][t] = num / den[i];
+    }
+    __syncthreads();
+    float acc[4] = {};
+
+    for (int i = 0; i < N; i++)
+        for (int e = 0; e < 4; e++) {
+            const uint32_t u = wv[i][e];
+            const int d = E * (8 * i + q) + (DT == DT_F32 ? e : 2 * e);
+
+            for (int k = 0; k < 4; k++)
+                if (DT == DT_F32)
+                    acc[k] = fmaf(__builtin_bit_cast(float, u), zs[i0 + k][d], acc[k]);
+                else {
+                    const uint16_t lo = (uint16_t)u, hi = (uint16_t)(u >> 16);
+
+                    acc[k] = fmaf(DT == DT_BF16 ? bf2f(lo) : h2f(lo), zs[i0 + k][d], acc[k]);
+                    acc[k] = fmaf(DT == DT_BF16 ? bf2f(hi) : h2f(hi), zs[i0 + k][d + 1], acc[k]);
+                }
+        }
+    for (int k = 0; k < 4; k++) {
+        float v = acc[k];
+
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        if (q == k)
+            o[((long)p * 8 + i0 + k) * 128 + 16 * h + c] = v + bv[16 * h + c];
+    }
 }
 
 extern "C" int launch_t2i_fused(const float *keys, const void *pk16,
                                 const void *U16, const void *Qc16, float *part,
-                                float *Z, const void *Wv, int wv_dt,
+                                const void *Wv, int wv_dt,
                                 const float *bv, float *o, int T, int P,
                                 int nsplit, void *stream)
 {
     const int nblk = (T + 63) / 64;
-    const long n = (long)P * FOLD_ROWS * 256;
 
     if (P < 1 || T < 1 || nsplit < 1 || nsplit > nblk ||
-        (long)P * nsplit > 0x7fffffffL || !pk16 || !Qc16 ||
+        nsplit > T2I_MAX_SPLIT || (long)P * nsplit > 0x7fffffffL || !pk16 || !Qc16 ||
         (((uintptr_t)keys | (uintptr_t)pk16 | (uintptr_t)U16 | (uintptr_t)Qc16 |
-          (uintptr_t)part) & 15))
+          (uintptr_t)part | (uintptr_t)Wv) & 15))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_t2i_fused, dim3((unsigned)((P * nsplit + 7) / 8 * 8)),
                        dim3(256), 0, (hipStream_t)stream, keys,
                        (const uint16_t *)pk16, (const uint16_t *)U16,
                        (const uint16_t *)Qc16, part, T, P, nsplit);
-    hipLaunchKernelGGL(k_t2i_merge, dim3((unsigned)((n + 255) / 256)), dim3(256),
-                       0, (hipStream_t)stream, part, Z, P, nsplit);
-    hipLaunchKernelGGL(k_t2i_unfold, dim3(P, 8), dim3(128), 0, (hipStream_t)stream,
-                       Z, Wv, wv_dt, bv, o, P);
+    {
+        auto kern = wv_dt == DT_F32 ? k_t2i_end<DT_F32>
+                                    : wv_dt == DT_F16 ? k_t2i_end<DT_F16> : k_t2i_end<DT_BF16>;
+
+        hipLaunchKernelGGL(kern, dim3(P, 8), dim3(256), 0, (hipStream_t)stream, part, Wv, bv, o,
+                           P, nsplit);
+    }
     return hipGetLastError();
 }
 

@@ -112,7 +112,6 @@ void sam_dec_init(struct sam_model *m, struct sam_decoder *d, int batch)
                                      "upscaling weights 2");
         d->t2i_part = dalloc(m, (2L * m->hip->cu_count + P) * 64 * 258,
                              "token -> image partials");
-        d->t2i_z = dalloc(m, P * 64 * SAM_DIM, "token -> image key sums");
         d->fold_c = hipb_alloc_typed(m->hip, P * 64 * 16, HIPB_BF16,
                                      "folded token rows");
         d->pe_q1 = hipb_alloc_typed(m->hip, T * 128, HIPB_BF16,
@@ -147,7 +146,7 @@ void sam_dec_free(struct sam_model *m)
                         &d->bk, &d->bv, &d->bo, &d->u1, &d->g2, &d->u2,
                         &d->hyper, &d->lowres, &d->mask, &d->sel, &d->stats,
                         &d->fold_w, &d->fold_b, &d->fold_y, &d->up_w1t,
-                        &d->up_w2t, &d->t2i_part, &d->t2i_z, &d->fold_c,
+                        &d->up_w2t, &d->t2i_part, &d->fold_c,
                         &d->pe_q1, &d->pe_k1, &d->pe_kf};
 
     if (m->hip)
@@ -259,8 +258,7 @@ static void t2i_run(struct sam_model *m, int P, const struct sam_attn_w *a, int 
         hipb_run_end(be, err, "t2i_fold", 0.0);
         hipb_run_begin(be);
         err = launch_t2i_fused(d->keys->ptr, pk->ptr, d->fold_w->ptr,
-                               d->fold_c->ptr, d->t2i_part->ptr,
-                               d->t2i_z->ptr, a->vw->ptr, a->vw->dtype,
+                               d->fold_c->ptr, d->t2i_part->ptr, a->vw->ptr, a->vw->dtype,
                                a->vb->ptr, d->so->ptr, (int)T, P, nsplit,
                                be->stream);
         hipb_run_end(be, err, "t2i_fused", 4.0 * P * 64.0 * T * SAM_DIM);

@@ -313,9 +313,9 @@ int launch_upscale_fused(const float *keys, const void *W1T16,
  * part as pk16 [T][128] bf16 (PE through the key projection, no bias)
  * against Qc16 (the fold's compact rows s q_{i,h}), nsplit key splits
  * with partials in part (P nsplit 64 258 floats), merged into Z [P][64]
- * [256], then o [P][8][128] = Wv Z + bv per head. */
+ * [256] on the chip, then o [P][8][128] = Wv Z + bv per head. */
 int launch_t2i_fused(const float *keys, const void *pk16, const void *U16,
-                     const void *Qc16, float *part, float *Z, const void *Wv,
+                     const void *Qc16, float *part, const void *Wv,
                      int wv_dt, const float *bv, float *o, int T, int P,
                      int nsplit, void *stream);
 

@@ -453,9 +453,8 @@ struct sam_decoder {
      * transposes [256][256] and [128][64]. */
     hipb_mem up_w1t, up_w2t;
     /* precision=bf16: token -> image attention key-split partials
-     * ((2 CUs + batch) records of 64 rows x 258 floats) and the merged
-     * weighted key sums Z [batch][64][256]. */
-    hipb_mem t2i_part, t2i_z;
+     * ((2 CUs + batch) records of 64 rows x 258 floats). */
+    hipb_mem t2i_part;
     /* precision=bf16: the folds' compact per-head token rows (s k_{t,h},
      * or s q_{i,h} for token -> image) [batch][64][16] bf16, and the dense
      * PE through the layer-1 image-query, layer-1 key and final key
