@@ -1065,11 +1065,35 @@ static void attention_region(struct sam_model *m, const struct vit_block *blk,
         return;
     }
 
-    layernorm(m, T, E, m->x, m->xn, blk->n1w, blk->n1b, ENC_EPS, ACT_NONE);
-    if (blk->window) {
-        window_partition(m, m->xn, m->xw, m->grid, E, g.s, g.nwx);
+    if (blk->window > 0 && !unfused && E % 256 == 0 && E <= 4096) {
+        /* LayerNorm straight into window-partitioned rows, the same bits:
+         * the partition's own pass read and wrote every window row once
+         * more (50 x 50 grid, window 24, E = 1024, half weights: the block
+         * 602 us with it, 586 without). Only at the widths of the
+         * wave-per-row kernel, which maps rows itself; narrower rows keep
+         * their several-rows-per-workgroup LayerNorm and the partition. */
+        int err;
+
+        if (!buf_ok("vit_attention", "x", m->x, (size_t)T * E, HIPB_F32) ||
+            !buf_ok("vit_attention", "window tokens", m->xw, (size_t)rows * E, HIPB_F32) ||
+            !buf_ok("vit_attention", "n1w", blk->n1w, (size_t)E, HIPB_F32) ||
+            !buf_ok("vit_attention", "n1b", blk->n1b, (size_t)E, HIPB_F32))
+            return;
+        hipb_run_begin(b);
+        err = launch_layernorm(m->x->ptr, m->xw->ptr, HIPB_F32, blk->n1w->ptr, blk->n1b->ptr, T,
+                               E, ENC_EPS, ACT_NONE, m->grid, g.s, g.nwx, b->stream);
+        hipb_run_end(b, err, "layernorm", 0.0);
         A = m->xw;
     }
+    else {
+        layernorm(m, T, E, m->x, m->xn, blk->n1w, blk->n1b, ENC_EPS, ACT_NONE);
+        if (blk->window) {
+            window_partition(m, m->xn, m->xw, m->grid, E, g.s, g.nwx);
+            A = m->xw;
+        }
+    }
+    if (hipb_failed())
+        return;
     linear(m, (int)rows, E, 3 * E, A, 0, blk->qkvw, blk->qkvb, m->qkv, 0,
            ACT_NONE, 0);
     if (hipb_failed())

@@ -311,6 +311,35 @@ def test_vit_attention_small(hip, be, orc, grid, ws, unfused):
                   (grid, ws, unfused, be.precision), got, want) <= TOL[be.precision]
 
 
+@pytest.mark.parametrize("E,grid,ws", [(256, 10, 4), (256, 6, 6), (256, 5, 8),
+                                       (512, 7, 1), (1024, 7, 3), (192, 10, 4)])
+def test_window_rows_bit_exact(hip, be, orc, E, grid, ws):
+    """The float paths' window rows (LayerNorm straight into them at widths
+    of whole 256s): the bits of LayerNorm and window_partition apart, the
+    padding of ragged grids zero over a work buffer of other values."""
+    if be.precision == "bf16":
+        pytest.skip("bf16 rows go to a buffer of their own")
+    x, n1w, n1b, w, b = block_inputs(E + grid, grid, E)
+    nwx = -(-grid // ws)
+    n = nwx * nwx * ws * ws * E
+    blk = hip.VitBlock()
+    blk.n1w, blk.n1b = be.upload(n1w), be.upload(n1b)
+    blk.qkvw, blk.qkvb = be.upload_weight(w), be.upload(b)
+    blk.window = ws
+    m = hip.Model(be, grid=grid, embed=E, heads=E // 64, blocks=[blk])
+    m.m.rope_win = be.upload(orc.rope_table(ws))
+    be.write(m.m.x, 0, x)
+    rows, outs = [], []
+    for unfused in (False, True):
+        be.write(m.m.xw, 0, np.full(n, 7.0, np.float32))
+        hip.vit_attention(m, blk, unfused)
+        rows.append(be.read(m.m.xw, n))
+        outs.append(be.read(m.m.attn, n))
+    m.free()
+    assert np.array_equal(rows[0].view(np.uint32), rows[1].view(np.uint32))
+    assert rel_l2(outs[0], outs[1]) <= TOL[be.precision]
+
+
 _FULL_REGION = {}
 
 
