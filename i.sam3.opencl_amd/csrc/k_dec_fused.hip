@@ -845,8 +845,8 @@ extern "C" int launch_upscale_fused(const float *keys, const void *W1T16,
  * keys x 32 rows, rows = lanes; PK straight from global memory, 256 bytes
  * per key instead of PE's 1 KB), the online softmax, and Z^T += keys^T
  * P^T (256 x 32). The two streams of a row tile merge through LDS; each
- * split leaves (Z, m, l) partials for k_t2i_merge; k_t2i_unfold applies
- * Wv and bv. */
+ * split leaves (Z, m, l) partials; k_t2i_end merges them and applies Wv
+ * and bv. */
 
 /* Byte offset of keys^T element (dim d, key k) in a [256][64] bf16 tile:
  * rows of 128 B, 16-byte chunk k / 8 at chunk (k / 8) ^ ((d >> 1) & 7). */

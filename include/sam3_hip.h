@@ -104,9 +104,10 @@ struct hipb_backend {
  * device_opt: NULL, "auto", "gpu" or a device ordinal "0".."N-1";
  * platform_opt: NULL, "" or a substring of "HIP" / "AMD" (anything else
  * matches no device); profile_opt: NULL, "auto" or "dgpu";
- * precision_opt: NULL or "fp32" (exact path, f32 MFMA), "fp16" (weight
- * matrices stored as half, float arithmetic, as the reference) or
- * "bf16" (bf16 MFMA with f32 accumulation for attention and the GEMMs).
+ * precision_opt: NULL or "fp32" (exact path: fp32 operands, f32
+ * accumulation), "fp16" (weight matrices stored as half, float
+ * arithmetic, as the reference) or "bf16" (bf16 MFMA with f32
+ * accumulation for attention and the GEMMs).
  * Fatal if no device matches. I_SAM3_OPENCL_PROFILE in the environment
  * switches on per-kernel timing, as in the reference. */
 void hipb_init(struct hipb_backend *b, const char *device_opt,
@@ -259,7 +260,8 @@ struct opnd bmat(hipb_mem buf, long off, int ld, long s0, long s1); /* ops.h:49 
 /* Batched C = act(alpha * A * op(B) + bias) + R (sam3_ops.h:51-54,
  * contract sam3_kernels.cl:57-69). A and C are float (C may be bf16 and
  * A bf16 with precision=bf16); B may be half or bf16 weights. R may
- * alias C. */
+ * alias C. Float products of large matrices use a workspace of the backend
+ * that grows on demand, except while the caller captures the stream. */
 void gemm(struct sam_model *m, int M, int N, int K, struct opnd A,
           struct opnd B, int transb, struct opnd C, int nb, int nb1,
           hipb_mem bias, hipb_mem R, long roff, float alpha, int act);
@@ -341,7 +343,8 @@ void mha_noalloc(struct sam_model *m, int P, int Nq, int Nk, int dint,
  * operands of the reference's QK^T and PV calls (sam3_model.c:1004-1011)
  * apply unchanged. rope (NULL for none) rotates Q and K rows at position
  * i % npos of the unit. With precision=bf16 the product runs on bf16
- * MFMA with f32 accumulation; otherwise on f32 MFMA. Replaces the
+ * MFMA with f32 accumulation; otherwise it is a float product (f32 MFMA,
+ * or operands split exactly into bf16 pieces for larger problems). Replaces the
  * gemm -> softmax_rows -> gemm loop of sam3_model.c:1000-1013. */
 void attn_fused(struct sam_model *m, int N, int nb, int nb1, struct opnd Q,
                 struct opnd K, struct opnd V, struct opnd O, hipb_mem rope,
