@@ -547,6 +547,8 @@ extern "C" int launch_gemm(const gemm_desc *d, void *ws, size_t ws_bytes, void *
         if (r != -1)
             return r;
     }
+    if (d->win_ws > 0)
+        return hipErrorInvalidValue; /* row map: packed exact path only */
     if (d->mode == MODE_BF16 && d->transb && d->nb == 1 && d->K % 64 == 0 &&
         avec && bvec && (long)grid.x * grid.y <= 64 &&
         ((uintptr_t)d->A & 15) == 0 && ((uintptr_t)d->B & 15) == 0) {

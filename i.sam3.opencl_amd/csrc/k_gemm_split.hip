@@ -326,13 +326,23 @@ struct frag_src {
     long ld;
     int rows, K, kmajor; /* kmajor: element (r, k) at k ld + r, else r ld + k */
     char *dst;
+    int win_H, win_ws, win_nwx, win_m0; /* gemm_desc's (A only; win_ws 0: rows as they lie) */
 };
+
+/* Window-partition position of grid token t (k_window_unpartition_add's). */
+__device__ __forceinline__ long win_row(int t, int H, int ws, int nwx)
+{
+    const int y = t / H, x = t - y * H, wy = y / ws, wx = x / ws;
+
+    return ((long)wy * nwx + wx) * ws * ws + (y - wy * ws) * ws + (x - wx * ws);
+}
 
 /* 32 rows x 64 k per 256-thread workgroup: eight lanes read 256 contiguous
  * bytes of a row (or, k-major, 32 lanes 128 contiguous bytes of a k), the
  * pieces go through LDS (chunk position xored with the k octet against bank
  * conflicts) and leave as contiguous fragments. */
-template <int DT, int NP> __device__ __forceinline__ void pack_block(const frag_src &f, int blk, char *S)
+template <int DT, int NP, bool WIN>
+__device__ __forceinline__ void pack_block(const frag_src &f, int blk, char *S)
 {
     const int t = threadIdx.x, nks = GS_STEPS(f.K), nkc = nks / 4;
     const int rb = blk / nkc, kc = blk % nkc;
@@ -341,7 +351,9 @@ template <int DT, int NP> __device__ __forceinline__ void pack_block(const frag_
     f32x4 x[2] = {};
 
     if (row < f.rows) {
-        const long i0 = f.kmajor ? (long)k0 * f.ld + row : (long)row * f.ld + k0;
+        const long srow =
+            WIN ? win_row(f.win_m0 + row, f.win_H, f.win_ws, f.win_nwx) : row;
+        const long i0 = f.kmajor ? (long)k0 * f.ld + row : srow * f.ld + k0;
 
         if (!f.kmajor && k0 + 8 <= f.K) {
             if constexpr (DT == DT_F32) {
@@ -386,15 +398,16 @@ template <int DT, int NP> __device__ __forceinline__ void pack_block(const frag_
     }
 }
 
-template <int BDT>
+/* WIN: A's rows are taken from their windows. */
+template <int BDT, bool WIN>
 __global__ __launch_bounds__(256) void k_split_pack(frag_src a, frag_src b, int ablocks)
 {
     __shared__ __attribute__((aligned(16))) char S[4 * 3 * 1024];
 
     if ((int)blockIdx.x < ablocks)
-        pack_block<DT_F32, 3>(a, blockIdx.x, S);
+        pack_block<DT_F32, 3, WIN>(a, blockIdx.x, S);
     else
-        pack_block<BDT, BDT == DT_F32 ? 3 : 2>(b, blockIdx.x - ablocks, S);
+        pack_block<BDT, BDT == DT_F32 ? 3 : 2, false>(b, blockIdx.x - ablocks, S);
 }
 
 /* Asynchronous 16-byte global -> LDS copy: lane i reads base + voff_i and
@@ -420,7 +433,7 @@ __device__ __forceinline__ void gs_vmwait0()
  * is even; copies past the end repeat the last step into a slot that no one
  * reads): with a branch in it the compiler kept a second copy of the
  * accumulators, 128 moves per step (145 against 180 TFLOP/s). */
-template <int BM, int BN, int WM, int WN, int BDT>
+template <int BM, int BN, int WM, int WN, int BDT, bool WIN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void
 k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
 {
@@ -558,7 +571,11 @@ k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
                     if (m >= d.M || n >= d.N)
                         continue;
                     if (!(fabsf(v) < __builtin_inff()))
-                        v = dot_seq<BDT>((const float *)d.A + d.aoff + (long)m * d.lda,
+                        v = dot_seq<BDT>((const float *)d.A + d.aoff +
+                                             (WIN ? win_row(d.win_m0 + m, d.win_H, d.win_ws,
+                                                            d.win_nwx)
+                                                  : (long)m) *
+                                                 d.lda,
                                          (const char *)d.B +
                                              (BDT == DT_F32 ? 4 : 2) *
                                                  (d.boff + (d.transb ? (long)n * d.ldb : (long)n)),
@@ -704,10 +721,11 @@ static int gs_chunk(const gemm_desc *d)
 
 /* Packing pays when what it saves, 4.6e-15 s per product (125 against 175
  * TFLOP/s), exceeds its 2.2e-12 s per element and a launch: at equal sides
- * about 1000 x 1000. */
+ * about 1000 x 1000. A product over the tokens of windows replaces one over
+ * all window rows, so it is packed where that was. */
 extern "C" size_t gemm_split_ws(const gemm_desc *d)
 {
-    const double M = d->M, N = d->N, K = d->K;
+    const double wr = (double)d->win_nwx * d->win_ws, M = d->win_ws > 0 ? wr * wr : d->M, N = d->N, K = d->K;
 
     if (!gs_aligned(d) || d->nb != 1 || gs_small(d) ||
         (M + N) * K * 2.2e-12 + 4e-6 > M * N * K * 4.6e-15)
@@ -759,16 +777,19 @@ static int launch_packed(const gemm_desc *d, void *ws, hipStream_t s)
     const int chunk = gs_chunk(d), bblocks = (int)((d->N + 31L) / 32 * (nks / 4));
     char *pb = (char *)ws, *pa = pb + (d->N + 31L) / 32 * nks * NPB * 1024;
     const frag_src fb = {(const char *)d->B + (BDT == DT_F32 ? 4 : 2) * d->boff, d->ldb, d->N,
-                         d->K, !d->transb, pb};
+                         d->K, !d->transb, pb, 0, 0, 0, 0};
 
     for (int m0 = 0; m0 < d->M; m0 += chunk) {
         gemm_desc c = *d;
 
         c.M = d->M - m0 < chunk ? d->M - m0 : chunk;
-        c.aoff += (long)m0 * d->lda;
+        c.win_m0 = m0;
+        if (d->win_ws == 0)
+            c.aoff += (long)m0 * d->lda;
         c.coff += (long)m0 * d->ldc;
         c.roff += (long)m0 * d->ldc;
-        const frag_src fa = {(const float *)d->A + c.aoff, d->lda, c.M, d->K, 0, pa};
+        const frag_src fa = {(const float *)d->A + c.aoff, d->lda, c.M, d->K, 0, pa,
+                             c.win_H, c.win_ws, c.win_nwx, c.win_m0};
         const long ablocks = (c.M + 31L) / 32 * (nks / 4);
         const int cfg = gs_pick(&c);
         const long grid = (gs_tiles(&c, gs_cfg[cfg].bm, gs_cfg[cfg].bn) + GS_NXCD - 1) /
@@ -777,13 +798,21 @@ static int launch_packed(const gemm_desc *d, void *ws, hipStream_t s)
         if (ablocks + bblocks > 0x7fffffffL || grid > 0x7fffffffL)
             return hipErrorInvalidConfiguration;
         /* The weights are split once, with the first chunk. */
-        hipLaunchKernelGGL((k_split_pack<BDT>),
-                           dim3((unsigned)(ablocks + (m0 ? 0 : bblocks))), dim3(256), 0, s, fa,
-                           fb, (int)ablocks);
+        const dim3 pgrid((unsigned)(ablocks + (m0 ? 0 : bblocks)));
+
+        if (d->win_ws > 0)
+            hipLaunchKernelGGL((k_split_pack<BDT, true>), pgrid, dim3(256), 0, s, fa, fb,
+                               (int)ablocks);
+        else
+            hipLaunchKernelGGL((k_split_pack<BDT, false>), pgrid, dim3(256), 0, s, fa, fb,
+                               (int)ablocks);
 #define GS_FRAG(I, BM, BN, WM, WN)                                                              \
-    if (cfg == I)                                                                              \
-    hipLaunchKernelGGL((k_gemm_frag<BM, BN, WM, WN, BDT>), dim3((unsigned)grid),               \
-                       dim3((BM / WM) * (BN / WN) * 64), 0, s, c, pa, pb)
+    if (cfg == I && d->win_ws > 0)                                                             \
+        hipLaunchKernelGGL((k_gemm_frag<BM, BN, WM, WN, BDT, true>), dim3((unsigned)grid),     \
+                           dim3((BM / WM) * (BN / WN) * 64), 0, s, c, pa, pb);                 \
+    else if (cfg == I)                                                                         \
+        hipLaunchKernelGGL((k_gemm_frag<BM, BN, WM, WN, BDT, false>), dim3((unsigned)grid),    \
+                           dim3((BM / WM) * (BN / WN) * 64), 0, s, c, pa, pb)
         GS_FRAG(0, 256, 256, 64, 64);
         GS_FRAG(1, 256, 128, 64, 64);
         GS_FRAG(2, 128, 128, 64, 32);
@@ -841,6 +870,8 @@ extern "C" int launch_gemm_split(const gemm_desc *d, void *ws, size_t ws_bytes, 
 
     if (!gs_aligned(d))
         return -1;
+    if (d->win_ws > 0 && !(need && ws && ws_bytes >= need))
+        return -1; /* row map: packed operands only */
     if (gs_small(d))
         return d->bdt == DT_F32 ? launch_small<DT_F32>(d, s) : launch_small<DT_F16>(d, s);
     if (need && ws && ws_bytes >= need)

@@ -54,6 +54,10 @@ struct gemm_desc {
      * are its grid token (padding rows are dropped): the projection's
      * window_unpartition_add fused into the store. */
     int unpart_H, unpart_ws, unpart_nwx;
+    /* Packed exact path only: with win_ws > 0, row m of the product (row
+     * win_m0 + m of a chunked one) is a token of an H x H grid and A's row
+     * is its window-partition position (nwx windows per side). */
+    int win_H, win_ws, win_nwx, win_m0;
     /* NT kernel only: with pack_N > 0 the product is a QKV projection
      * (N = 3 pack_E columns, q | k | v thirds of 64-wide heads; rows are
      * units of pack_N tokens, pack_N % 64 == 0) and the store writes the

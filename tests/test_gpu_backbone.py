@@ -81,6 +81,16 @@ def test_vit_block_full_size(hip, be, orc, ws):
                   want) <= TOL[be.precision]
 
 
+@pytest.mark.parametrize("grid,ws", [(49, 24), (50, 14), (40, 32)])
+def test_vit_block_ragged_windows(hip, be, orc, grid, ws):
+    """Grids that the windows do not divide, at a width whose projection runs
+    on packed operands on the float paths: its rows are the tokens, read from
+    their windows."""
+    got, want = run_block(hip, be, orc, grid, 1024, 16, 64, ws, 95 + grid)
+    assert report("vit_block ragged grid=%d ws=%d %s" % (grid, ws, be.precision), got,
+                  want) <= TOL[be.precision]
+
+
 def trunk(hip, be, orc, grid, ps, E, heads, mlp, windows, seed, pe_f32=False):
     img, pe_w, pos, lnpw, lnpb, blocks = bc.trunk_case(seed, grid, ps, E, mlp,
                                                        windows)
