@@ -577,37 +577,6 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
                         st.l);
 }
 
-/* Asynchronous 16-byte global -> LDS copy (global_load_lds_dwordx4):
- * lane i of the wave writes lds_base + 16 i (lds_base wave-uniform, via
- * M0). Issued as inline assembly so that the compiler does not treat the
- * copy as a store that later LDS reads of the other slot must wait for:
- * the kernel waits for it itself (s_waitcnt vmcnt(0)) before the barrier
- * that hands the slot to the readers. */
-__device__ __forceinline__ void g2lds16(const void *g, void *lds_base)
-{
-    /* The low 32 bits of a flat LDS address are the LDS offset. */
-    const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_base);
-
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(lds), "v"(g)
-                 : "memory", "m0");
-}
-
-/* The same copy with a wave-uniform 64-bit base in SGPRs and a 32-bit
- * per-lane byte offset (the saddr form): no per-lane address arithmetic
- * when only the base moves from block to block. `lds` must be
- * wave-uniform. */
-__device__ __forceinline__ void g2lds16_s(const void *base, unsigned voff, unsigned lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory", "m0");
-}
-
 /* ------------------------------------------------------------ fp32 path, split operands */
 
 /* The exact path of larger problems: K, V and Q, and the weights P, as three
@@ -814,7 +783,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_split(attn_desc d, const char *
         const unsigned to = __builtin_amdgcn_readfirstlane(lds + BLK * buf);
 
         for (int i = 0; i < CPW; i++)
-            g2lds16_s(b + 1024 * i, voff, to + 1024u * i);
+            g2lds16(b + 1024 * i, voff, to + 1024u * i);
     };
     bf16x8 q[NS][3];
     exact_state st;
@@ -1356,8 +1325,8 @@ __device__ __forceinline__ void attn_tile(const Desc &d, const uint16_t *__restr
         const uint16_t *kb_ = Ku + (long)kb * 64 * 64, *vb_ = Vu + kb * 64;
 
         for (int j = 0; j < 2; j++) {
-            g2lds16_s(kb_, koff[j], lds_k + 8192u * slot + 1024u * j);
-            g2lds16_s(vb_, voff[j], lds_v + 8192u * slot + 1024u * j);
+            g2lds16(kb_, koff[j], lds_k + 8192u * slot + 1024u * j);
+            g2lds16(vb_, voff[j], lds_v + 8192u * slot + 1024u * j);
         }
     };
     /* The first block of the plain instance: K's two copies before V's,
@@ -1369,9 +1338,9 @@ __device__ __forceinline__ void attn_tile(const Desc &d, const uint16_t *__restr
             const uint16_t *kb_ = Ku + (long)kb * 64 * 64, *vb_ = Vu + kb * 64;
 
             for (int j = 0; j < 2; j++)
-                g2lds16_s(kb_, koff[j], lds_k + 8192u * slot + 1024u * j);
+                g2lds16(kb_, koff[j], lds_k + 8192u * slot + 1024u * j);
             for (int j = 0; j < 2; j++)
-                g2lds16_s(vb_, voff[j], lds_v + 8192u * slot + 1024u * j);
+                g2lds16(vb_, voff[j], lds_v + 8192u * slot + 1024u * j);
         }
         else
             load_block(kb, slot);
@@ -1395,7 +1364,7 @@ __device__ __forceinline__ void attn_tile(const Desc &d, const uint16_t *__restr
             const int row = 32 * w + 8 * j + (l >> 3), chunk = (l & 7) ^ ((row >> 1) & 7);
             const int qrow = tile * 128 + row < Np ? tile * 128 + row : Np - 1;
 
-            g2lds16_s(Qu, 2u * ((unsigned)qrow * 64u + 8u * chunk), qlds + 1024u * j);
+            g2lds16(Qu, 2u * ((unsigned)qrow * 64u + 8u * chunk), qlds + 1024u * j);
         }
         load_first(kb0, 0);
         /* The Q copies landed (the block's four may still be in flight). */
@@ -1997,9 +1966,9 @@ __global__ __launch_bounds__(64 * NG * WPG) void k_attn_bf16_grp(attn_desc d,
     auto load_block = [&](int kb, int area) {
         for (int j = 0; j < CPW; j++) {
             if (isk[j])
-                g2lds16_s(Ku + (long)kb * 64 * 64, goffk[j], lds_g + 16384u * area + ldso[j]);
+                g2lds16(Ku + (long)kb * 64 * 64, goffk[j], lds_g + 16384u * area + ldso[j]);
             else
-                g2lds16_s(Vu + kb * 64, goffv[j], lds_g + 16384u * area + ldso[j]);
+                g2lds16(Vu + kb * 64, goffv[j], lds_g + 16384u * area + ldso[j]);
         }
     };
     unsigned kro[4], vro[4];

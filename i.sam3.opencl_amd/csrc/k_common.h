@@ -82,6 +82,24 @@ template <int NP> __device__ __forceinline__ void split4(const f32x4 x, u32x2 (&
     }
 }
 
+/* Asynchronous 16-byte global -> LDS copy (global_load_lds_dwordx4, saddr
+ * form): lane i of the wave reads base + voff_i and writes lds + 16 i (base
+ * and lds wave-uniform, lds via M0). The s_nop is the wait state that the
+ * hardware needs between a scalar write of M0 and an LDS load that reads it:
+ * inside inline assembly the compiler does not add it. Inline assembly so
+ * that the compiler does not treat the copy as a store that later LDS reads
+ * of another slot must wait for: the kernel waits itself (s_waitcnt
+ * vmcnt(0)) before the barrier that hands the slot to its readers. */
+__device__ __forceinline__ void g2lds16(const void *base, unsigned voff, unsigned lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(voff), "s"(base)
+                 : "memory", "m0");
+}
+
 /* Element load of any storage type as float. */
 template <typename T> __device__ __forceinline__ float ld_f(const T *p);
 template <> __device__ __forceinline__ float ld_f<float>(const float *p)

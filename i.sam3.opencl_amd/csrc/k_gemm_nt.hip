@@ -38,21 +38,6 @@ __device__ __forceinline__ int nt_swz(int row, int chunk)
     return 8 * (chunk ^ ((row >> 1) & 7));
 }
 
-/* Asynchronous 16-byte global -> LDS copy (global_load_lds_dwordx4, saddr
- * form): lane i of the wave reads base + voff_i and writes lds + 16 i
- * (base and lds wave-uniform, lds via M0). Inline assembly so the compiler
- * does not wait for it before unrelated LDS reads; the kernel waits
- * itself (s_waitcnt vmcnt(0)) before the barrier that publishes the slot.
- */
-__device__ __forceinline__ void nt_g2lds16_s(const void *base, unsigned voff, unsigned lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory", "m0");
-}
-
 /* Store of a 128 x 128 tile of a QKV projection as packed attention
  * operands (gemm_desc pack_*), from the float tile E [128][132] in LDS:
  * the tile's columns are two 64-wide heads of one third. Wave w takes
@@ -243,7 +228,7 @@ k_gemm_nt(gemm_desc d)
             /* Whether copy j is of A or of B is the same for the wave. */
             const bool isa = 8 * (wu * LPW + j) < BM;
 
-            nt_g2lds16_s((isa ? Ab : Bb) + 128L * ks, goff[j],
+            g2lds16((isa ? Ab : Bb) + 128L * ks, goff[j],
                          lds0 + (unsigned)SLOT_BYTES * slot + 1024u * j);
         }
     };
@@ -549,7 +534,7 @@ k_gemm_nt2(gemm_desc d)
     auto load_stage = [&](int ks, int slot) {
 #pragma unroll
         for (int j = 0; j < LPW; j++)
-            nt_g2lds16_s((8 * (wu * LPW + j) < BM ? Ab : Bb) + 128L * ks, goff[j],
+            g2lds16((8 * (wu * LPW + j) < BM ? Ab : Bb) + 128L * ks, goff[j],
                          lds0 + (unsigned)SLOT * slot + 1024u * j);
     };
     /* Fragment byte offsets per K step s: A rows wm WM + 32 i + l32, B

@@ -410,18 +410,6 @@ __global__ __launch_bounds__(256) void k_split_pack(frag_src a, frag_src b, int 
         pack_block<BDT, BDT == DT_F32 ? 3 : 2, false>(b, blockIdx.x - ablocks, S);
 }
 
-/* Asynchronous 16-byte global -> LDS copy: lane i reads base + voff_i and
- * writes lds + 16 i (base and lds wave-uniform). The kernel waits for it
- * itself before the barrier that publishes the slot. */
-__device__ __forceinline__ void gs_g2lds16(const void *base, unsigned voff, unsigned lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "global_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds), "v"(voff), "s"(base)
-                 : "memory", "m0");
-}
-
 __device__ __forceinline__ void gs_vmwait0()
 {
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
@@ -484,7 +472,7 @@ k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
 
 #pragma unroll
         for (int i = 0; i < CPW; i++)
-            gs_g2lds16(src[i] + kc * step[i], voff, lds[i] + (unsigned)SLOT * slot);
+            g2lds16(src[i] + kc * step[i], voff, lds[i] + (unsigned)SLOT * slot);
     };
     f32x16 acc[NA][NB];
 #pragma unroll
