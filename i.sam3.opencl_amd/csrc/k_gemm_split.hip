@@ -25,9 +25,11 @@
  * before).
  *
  * A non-finite operand (or one that rounds past the largest bf16) makes its
- * pieces, and so every output it enters, NaN; an output that comes out
- * non-finite is formed again from the float operands by fused multiply-adds
- * in k order, so infinities and NaN travel as in k_gemm_f32.
+ * pieces, and so every output it enters, NaN. A 32 x 32 block with a
+ * non-finite output is formed again from the float operands by the f32 MFMA
+ * (block_f32) and those outputs taken from there, so infinities and NaN
+ * travel as in k_gemm_f32 and a product full of NaN costs what the f32 unit
+ * costs, not a serial sum per output.
  *
  * LDS holds MFMA fragments: per 32 rows, 16 k and piece 1 KiB of 64 chunks
  * of 16 bytes (8 k of one row), chunk 32 (k half) + row, so that a fragment
@@ -52,19 +54,83 @@ __device__ __forceinline__ int frag_off(int r, int q)
     return 16 * (32 * h + (r ^ (4 * h))) + 8 * (q & 1);
 }
 
-/* One output formed from the float operands (non-finite results): a row of
- * A against elements of B bstep apart. */
+/* A 32 x 32 block of the product by the f32 MFMA from the float operands:
+ * lane l's row of A and column of B are l % 32 of the block's; a lane half
+ * takes four consecutive k of every eight (K % 4 == 0: in or out together). */
 template <int BDT>
-__device__ __noinline__ float dot_seq(const float *a, const void *b, long bstep, int K)
+__device__ __noinline__ f32x16 block_f32(const float *a, const void *b, long bstep, int K)
 {
-    float s = 0.0f;
+    const int h = (threadIdx.x & 63) >> 5;
+    f32x16 acc = {};
 
-    for (int k = 0; k < K; k++)
-        s = fmaf(a[k],
-                 BDT == DT_F32 ? ((const float *)b)[k * bstep]
-                               : h2f(((const uint16_t *)b)[k * bstep]),
-                 s);
-    return s;
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 8) {
+        const int k = k0 + 4 * h;
+        f32x4 x = {}, y = {};
+
+        if (k < K) {
+            x = *(const f32x4 *)(a + k);
+            for (int e = 0; e < 4; e++)
+                y[e] = BDT == DT_F32 ? ((const float *)b)[(k + e) * bstep]
+                                     : h2f(((const uint16_t *)b)[(k + e) * bstep]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+/* Epilogue (store_one, sam3_kernels.cl:306-319) of a wave's 32 NA x 32 NB
+ * part of C from (m0, n0), 32 lanes to 128 contiguous bytes of a row: act(alpha
+ * v + bias) + R, the non-finite v taken from block_f32. arow(m), bcol(n): row
+ * m of A, column n of B; C and R at the matrix's element 0. */
+template <int BDT, int NA, int NB, class ROW, class COL>
+__device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[NA][NB], int m0,
+                                             int n0, float *C, const float *R, ROW arow, COL bcol)
+{
+    const int l = threadIdx.x & 63, h = l >> 5, l32 = l & 31;
+
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const int n = n0 + 32 * j + l32;
+        float bn = d.bias && n < d.N ? d.bias[n] : 0.0f;
+
+        /* The load is waited for here, once: at its first use, in a branch
+         * per result, the wait came back in every branch and took in the
+         * store of the one before (1 us per tile). */
+        asm volatile("" : "+v"(bn));
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            const int mb = m0 + 32 * i;
+            unsigned long long bad = 0;
+
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                bad |= __ballot(!(fabsf(acc[i][j][r]) < __builtin_inff()));
+            if (bad) {
+                const f32x16 x = block_f32<BDT>(arow(min(mb + l32, d.M - 1)),
+                                                bcol(min(n, d.N - 1)), d.transb ? 1L : d.ldb, d.K);
+
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (!(fabsf(acc[i][j][r]) < __builtin_inff()))
+                        acc[i][j][r] = x[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = mb + 8 * (r >> 2) + 4 * h + (r & 3);
+                float v = acc[i][j][r];
+
+                if (m >= d.M || n >= d.N)
+                    continue;
+                v = act_k(d.alpha * v + bn, d.act);
+                if (R)
+                    v += R[(long)m * d.ldc + n];
+                C[(long)m * d.ldc + n] = v;
+            }
+        }
+    }
 }
 
 /* Operands split while they are staged: a workgroup owns a BM x BN tile of
@@ -111,6 +177,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
     const int nk = (d.K + GS_K - 1) / GS_K;
     f32x16 acc[NA][NB];
     f32x4 ra[LA], rb[LB];
+    u32x2 hb[LB]; /* B's quads as loaded (half N x K operand) */
     const float *pa[LA];
     long ob[LB];
 
@@ -146,15 +213,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
             if constexpr (TRANSB) {
                 if constexpr (BDT == DT_F32)
                     rb[i] = in ? *(const f32x4 *)((const float *)d.B + ob[i] + k0) : (f32x4){};
-                else {
-                    const u32x2 v =
-                        in ? *(const u32x2 *)((const uint16_t *)d.B + ob[i] + k0) : (u32x2){};
-
-                    for (int e = 0; e < 2; e++) {
-                        rb[i][2 * e] = h2f((uint16_t)(v[e] & 0xffffu));
-                        rb[i][2 * e + 1] = h2f((uint16_t)(v[e] >> 16));
-                    }
-                }
+                else
+                    hb[i] = in ? *(const u32x2 *)((const uint16_t *)d.B + ob[i] + k0) : (u32x2){};
             }
             else {
                 const int q = (t + T * i) / BN;
@@ -191,6 +251,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
             char *p = s + ABYTES + (row >> 5) * NPB * 1024 + frag_off(row & 31, q);
             u32x2 v[NPB];
 
+            /* Converted here, not where they are loaded: there the compiler
+             * may convert at once and wait for the load (37 against 47 us,
+             * 4298 x 321 x 888). */
+            if constexpr (TRANSB && BDT == DT_F16)
+                for (int e = 0; e < 4; e++)
+                    rb[i][e] = h2f((uint16_t)(hb[i][e >> 1] >> (16 * (e & 1))));
             split4<NPB>(rb[i], v);
             for (int e = 0; e < NPB; e++)
                 *(u32x2 *)(p + 1024 * e) = v[e];
@@ -237,6 +303,12 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
         constexpr int s = decltype(slot)::value;
 
         __syncthreads();
+        /* Nothing of the staging moves up between the products of the step
+         * before: its wait for the loads would come with it (344 x 2919 x
+         * 1732: 70 -> 63 us, half B 56 -> 47). Not with a K x N half B, whose
+         * single-element loads gain by moving (50 x 3179 x 3232: 124 -> 112). */
+        if constexpr (BDT == DT_F32 || TRANSB)
+            __builtin_amdgcn_sched_barrier(0);
         stage(s ^ 1);
         load(ks + 2, whole);
         products(s);
@@ -267,41 +339,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
         products(ks & 1);
     }
 
-    /* Epilogue (store_one, sam3_kernels.cl:306-319): 32 lanes store 128
-     * contiguous bytes of a row. */
-    {
-        const long cbase = d.coff + z0 * d.sc0 + z1 * d.sc1;
-        const long rbase = d.roff + z0 * d.sc0 + z1 * d.sc1;
-        float *C = (float *)d.C + cbase;
-        const float *R = d.R ? (const float *)d.R + rbase : nullptr;
-
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            const int n = n0 + wn * WN + 32 * j + l32;
-            const float bn = d.bias && n < d.N ? d.bias[n] : 0.0f;
-
-#pragma unroll
-            for (int i = 0; i < NA; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int m = m0 + wm * WM + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    float v = acc[i][j][r];
-
-                    if (m >= d.M || n >= d.N)
-                        continue;
-                    if (!(fabsf(v) < __builtin_inff()))
-                        v = dot_seq<BDT>((const float *)d.A + abase + (long)m * d.lda,
-                                         (const char *)d.B +
-                                             (BDT == DT_F32 ? 4 : 2) *
-                                                 (bbase + (TRANSB ? (long)n * d.ldb : (long)n)),
-                                         TRANSB ? 1 : d.ldb, d.K);
-                    v = act_k(d.alpha * v + bn, d.act);
-                    if (R)
-                        v += R[(long)m * d.ldc + n];
-                    C[(long)m * d.ldc + n] = v;
-                }
-        }
-    }
+    store_blocks<BDT, NA, NB>(
+        d, acc, m0 + wm * WM, n0 + wn * WN, (float *)d.C + d.coff + z0 * d.sc0 + z1 * d.sc1,
+        d.R ? (const float *)d.R + d.roff + z0 * d.sc0 + z1 * d.sc1 : nullptr,
+        [&](int m) { return (const float *)d.A + abase + (long)m * d.lda; },
+        [&](int n) {
+            return (const char *)d.B +
+                   (BDT == DT_F32 ? 4 : 2) * (bbase + n * (TRANSB ? (long)d.ldb : 1L));
+        });
 }
 
 /* ------------------------------------------------------------ packed */
@@ -432,7 +477,7 @@ k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
     constexpr int CPW = (FR + NW - 1) / NW;                    /* copies per wave */
     constexpr int SLOT = FR * 1024;
     __shared__ __attribute__((aligned(16))) char S[NSLOT * SLOT];
-    const int t = threadIdx.x, l = t & 63, h = l >> 5, l32 = l & 31;
+    const int t = threadIdx.x, l = t & 63;
     const int wu = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wu / (BN / WN), wn = wu % (BN / WN);
     const int tn = (d.N + BN - 1) / BN, tm = (d.M + BM - 1) / BM;
@@ -540,41 +585,17 @@ k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
     }
     /* No copy may land after the workgroup's LDS is given back. */
     gs_vmwait0();
-    {
-        float *C = (float *)d.C + d.coff;
-        const float *R = d.R ? (const float *)d.R + d.roff : nullptr;
-
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            const int n = n0 + wn * WN + 32 * j + l32;
-            const float bn = d.bias && n < d.N ? d.bias[n] : 0.0f;
-
-#pragma unroll
-            for (int i = 0; i < NA; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int m = m0 + wm * WM + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    float v = acc[i][j][r];
-
-                    if (m >= d.M || n >= d.N)
-                        continue;
-                    if (!(fabsf(v) < __builtin_inff()))
-                        v = dot_seq<BDT>((const float *)d.A + d.aoff +
-                                             (WIN ? win_row(d.win_m0 + m, d.win_H, d.win_ws,
-                                                            d.win_nwx)
-                                                  : (long)m) *
-                                                 d.lda,
-                                         (const char *)d.B +
-                                             (BDT == DT_F32 ? 4 : 2) *
-                                                 (d.boff + (d.transb ? (long)n * d.ldb : (long)n)),
-                                         d.transb ? 1 : d.ldb, d.K);
-                    v = act_k(d.alpha * v + bn, d.act);
-                    if (R)
-                        v += R[(long)m * d.ldc + n];
-                    C[(long)m * d.ldc + n] = v;
-                }
-        }
-    }
+    store_blocks<BDT, NA, NB>(
+        d, acc, m0 + wm * WM, n0 + wn * WN, (float *)d.C + d.coff,
+        d.R ? (const float *)d.R + d.roff : nullptr,
+        [&](int m) {
+            return (const float *)d.A + d.aoff +
+                   (WIN ? win_row(d.win_m0 + m, d.win_H, d.win_ws, d.win_nwx) : (long)m) * d.lda;
+        },
+        [&](int n) {
+            return (const char *)d.B +
+                   (BDT == DT_F32 ? 4 : 2) * (d.boff + n * (d.transb ? (long)d.ldb : 1L));
+        });
 }
 
 /* ------------------------------------------------------------ small */

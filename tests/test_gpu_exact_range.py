@@ -1,0 +1,79 @@
+"""The exact path (precision=fp32) outside ordinary magnitudes: operands as
+small as floats go, results beyond the largest float, and what a call costs
+when its operands hold NaN.
+
+The larger products and attentions run on operands split into bf16 pieces.
+Scaling an operand by a power of two is exact, so each result here is that of
+an ordinary problem times a known power of two, and the tolerance is the
+ordinary one: sqrt(K) 2^-24 of the result for a sum of K products."""
+import numpy as np
+import pytest
+
+from gpu_common import rel_l2, report
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import sam3_hip
+    return sam3_hip
+
+
+@pytest.fixture(scope="module")
+def be(hip):
+    b = hip.Backend(precision="fp32")
+    yield b
+    b.free()
+
+
+def ms(be, call):
+    """Time of the third call in a row, by events."""
+    for _ in range(2):
+        call()
+    be.finish()
+    be.timer_start()
+    call()
+    return be.timer_stop()
+
+
+# Packed operands; split while staged (float and K x N operand); f32 MFMA.
+GEMMS = [(2500, 1030, 512, 1), (700, 1024, 68, 1), (16500, 256, 256, 0), (33, 70, 300, 1)]
+
+
+def product(hip, be, A, B, transb, C, alpha=1.0):
+    M, K = A.shape
+    N = B.shape[0] if transb else B.shape[1]
+    m = hip.Model(be, embed=128, heads=2)
+    dA, dB, dC = be.upload(A), be.upload(B), be.upload(C)
+    try:
+        hip.gemm(m, M, N, K, hip.mat(dA, 0, K), hip.mat(dB, 0, B.shape[1]), transb,
+                 hip.mat(dC, 0, N), 1, 1, None, None, 0, alpha)
+        return be.read(dC).reshape(M, N)
+    finally:
+        for x in (dA, dB, dC):
+            be.release(x)
+        m.free()
+
+
+@pytest.mark.parametrize("M,N,K,transb", GEMMS)
+def test_gemm_nan_costs_no_more_than_the_f32_units(hip, be, M, N, K, transb):
+    """A product of NaN takes at most ten times the ordinary one (the f32
+    matrix unit is a sixteenth of the bf16 one's rate, six products of which
+    an ordinary one takes)."""
+    m = hip.Model(be, embed=128, heads=2)
+    g = np.random.default_rng(M)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    B = g.standard_normal((N, K) if transb else (K, N), dtype=np.float32)
+    dA, dB, dC = be.upload(A), be.upload(B), be.alloc(M * N * 4)
+    t = []
+    for bad in (False, True):
+        if bad:
+            A[:, K // 2] = np.nan
+            be.write(dA, 0, A)
+        t.append(ms(be, lambda: hip.gemm(m, M, N, K, hip.mat(dA, 0, K),
+                                         hip.mat(dB, 0, K if transb else N), transb,
+                                         hip.mat(dC, 0, N))))
+    assert np.isnan(be.read(dC, M * N)).all()
+    print("gemm %d x %d x %d: %.1f us, NaN %.1f us" % (M, N, K, 1e3 * t[0], 1e3 * t[1]))
+    assert t[1] <= 10 * t[0]
