@@ -9,23 +9,27 @@
  * with k_gemm_f32.
  *
  * The split. The f32 MFMA peaks at 157 TFLOP/s, the bf16 MFMA at sixteen
- * times that. A float is exactly the sum of three bf16 values (8 + 8 + 8
- * mantissa bits, each piece the rounding of what is left): x = x0 + x1 + x2,
- * |x1| <= 2^-8 |x|, |x2| <= 2^-16 |x|, roundings to nearest, so the pieces'
- * signs are unbiased. Of the nine products of two split values the six of
- * order 2^-16 and above are formed on the bf16 MFMA with f32 accumulation;
- * the three dropped ones are below 2^-24 of the product (2^-27 in the mean),
- * less than the rounding of one f32 fused multiply-add. A half is exactly
- * two pieces (five products). The range is the float's: bf16 has its
- * exponents. Rounding the accumulator six times per 16 k instead of once per
- * two, the result is no further from the 64-bit product than the f32 MFMA's
- * in k_gemm_f32: relative error 1.1e-7 against 1.4e-7 at K = 64, 2.4e-7
- * against 2.9e-7 at 256, 4.9e-7 against 5.7e-7 at 1024, 1.0e-6 against 1.15e-6
- * at 4096; the small kernel's split sums 1.5e-7 (256) and 2.9e-7 (2048, 8.1e-7
+ * times that. A float x in bf16 pieces: x0 the rounding of x to bf16, x1 that
+ * of x - x0, x2 what is left, 8 + 8 + 8 mantissa bits: |x1| <= 2^-8 |x|, |x2| <=
+ * 2^-16 |x|, roundings to nearest, so the pieces' signs are unbiased. bf16
+ * has the float's exponents, so the lowest piece of a float below 2^-109 would
+ * fall out of its range: floats are scaled by 2^24 first (SPLIT_SCALE),
+ * which leaves every bit of every float, subnormals too, at 2^-125 or above,
+ * and the sums are scaled back. So three pieces are exactly the float for
+ * every |x| < 2^103; larger ones overflow (below). Of the nine products of
+ * two split values the six of order 2^-16 and above are formed on the bf16
+ * MFMA with f32 accumulation; the three dropped ones are below 2^-24 of the
+ * product (2^-27 in the mean), less than the rounding of one f32 fused
+ * multiply-add. A half is exactly two pieces (five products), unscaled.
+ * Rounding the accumulator six times per 16 k instead of once per two, the
+ * result is no further from the 64-bit product than the f32 MFMA's in
+ * k_gemm_f32: relative error 1.1e-7 against 1.4e-7 at K = 64, 2.4e-7 against
+ * 2.9e-7 at 256, 4.9e-7 against 5.7e-7 at 1024, 1.0e-6 against 1.15e-6 at
+ * 4096; the small kernel's split sums 1.5e-7 (256) and 2.9e-7 (2048, 8.1e-7
  * before).
  *
- * A non-finite operand (or one that rounds past the largest bf16) makes its
- * pieces, and so every output it enters, NaN. A 32 x 32 block with a
+ * A non-finite operand, or one past 2^103, makes its pieces, and so every
+ * output it enters, NaN; a sum past 2^80 overflows. A 32 x 32 block with a
  * non-finite output is formed again from the float operands by the f32 MFMA
  * (block_f32) and those outputs taken from there, so infinities and NaN
  * travel as in k_gemm_f32 and a product full of NaN costs what the f32 unit
@@ -53,6 +57,10 @@ __device__ __forceinline__ int frag_off(int r, int q)
 
     return 16 * (32 * h + (r ^ (4 * h))) + 8 * (q & 1);
 }
+
+/* Scale of the split floats; the sums carry it once per float operand. */
+#define SPLIT_SCALE 0x1p24f
+template <int BDT> constexpr float split_unscale = BDT == DT_F32 ? 0x1p-48f : 0x1p-24f;
 
 /* A 32 x 32 block of the product by the f32 MFMA from the float operands:
  * lane l's row of A and column of B are l % 32 of the block's; a lane half
@@ -83,7 +91,8 @@ __device__ __noinline__ f32x16 block_f32(const float *a, const void *b, long bst
 
 /* Epilogue (store_one, sam3_kernels.cl:306-319) of a wave's 32 NA x 32 NB
  * part of C from (m0, n0), 32 lanes to 128 contiguous bytes of a row: act(alpha
- * v + bias) + R, the non-finite v taken from block_f32. arow(m), bcol(n): row
+ * v + bias) + R of the sums scaled back, the non-finite v taken from
+ * block_f32. arow(m), bcol(n): row
  * m of A, column n of B; C and R at the matrix's element 0. */
 template <int BDT, int NA, int NB, class ROW, class COL>
 __device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[NA][NB], int m0,
@@ -106,8 +115,10 @@ __device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[N
             unsigned long long bad = 0;
 
 #pragma unroll
-            for (int r = 0; r < 16; r++)
+            for (int r = 0; r < 16; r++) {
+                acc[i][j][r] *= split_unscale<BDT>;
                 bad |= __ballot(!(fabsf(acc[i][j][r]) < __builtin_inff()));
+            }
             if (bad) {
                 const f32x16 x = block_f32<BDT>(arow(min(mb + l32, d.M - 1)),
                                                 bcol(min(n, d.N - 1)), d.transb ? 1L : d.ldb, d.K);
@@ -240,7 +251,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
             char *p = s + (row >> 5) * 3072 + frag_off(row & 31, t & 3);
             u32x2 v[3];
 
-            split4<3>(ra[i], v);
+            split4<3>(ra[i] * SPLIT_SCALE, v);
             for (int e = 0; e < 3; e++)
                 *(u32x2 *)(p + 1024 * e) = v[e];
         }
@@ -257,7 +268,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
             if constexpr (TRANSB && BDT == DT_F16)
                 for (int e = 0; e < 4; e++)
                     rb[i][e] = h2f((uint16_t)(hb[i][e >> 1] >> (16 * (e & 1))));
-            split4<NPB>(rb[i], v);
+            split4<NPB>(BDT == DT_F32 ? rb[i] * SPLIT_SCALE : rb[i], v);
             for (int e = 0; e < NPB; e++)
                 *(u32x2 *)(p + 1024 * e) = v[e];
         }
@@ -423,9 +434,10 @@ __device__ __forceinline__ void pack_block(const frag_src &f, int blk, char *S)
                 }
     }
     u32x2 lo[NP], hi[NP];
+    const float scale = DT == DT_F32 ? SPLIT_SCALE : 1.0f;
 
-    split4<NP>(x[0], lo);
-    split4<NP>(x[1], hi);
+    split4<NP>(x[0] * scale, lo);
+    split4<NP>(x[1] * scale, hi);
     for (int p = 0; p < NP; p++) {
         const int c = (32 * (k8 & 1) + r) ^ k8;
 

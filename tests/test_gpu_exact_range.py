@@ -77,3 +77,48 @@ def test_gemm_nan_costs_no_more_than_the_f32_units(hip, be, M, N, K, transb):
     assert np.isnan(be.read(dC, M * N)).all()
     print("gemm %d x %d x %d: %.1f us, NaN %.1f us" % (M, N, K, 1e3 * t[0], 1e3 * t[1]))
     assert t[1] <= 10 * t[0]
+
+
+@pytest.mark.parametrize("ea,eb", [
+    (-118, 100),   # low pieces of A below bf16's range
+    (-140, 110),   # A subnormal
+    (110, -138),   # the other way round
+    (-60, -60),    # small results
+    (90, 30),      # results past the split's range, formed by the f32 unit
+    (105, 10),     # an operand past it
+])
+@pytest.mark.parametrize("M,N,K,transb", GEMMS)
+def test_gemm_magnitudes(hip, be, M, N, K, transb, ea, eb):
+    """A 2^ea times B 2^eb: the ordinary product times 2^(ea + eb). Subnormal
+    operands are first rounded to what the float type holds. A residual of the
+    result's size, bias none."""
+    g = np.random.default_rng(M + 200 + ea)
+    A = np.ldexp(g.standard_normal((M, K), dtype=np.float32), ea).astype(np.float32)
+    B = np.ldexp(g.standard_normal((N, K) if transb else (K, N), dtype=np.float32),
+                 eb).astype(np.float32)
+    got = product(hip, be, A, B, transb, np.zeros((M, N), np.float32))
+    rows = np.unique(np.concatenate([np.arange(40) % M, [M - 1], g.integers(0, M, 60)]))
+    want = np.ldexp(A[rows].astype(np.float64), -ea) @ np.ldexp(
+        (B.T if transb else B).astype(np.float64), -eb)
+    r = rel_l2(np.ldexp(got[rows].astype(np.float64), -ea - eb), want)
+    print("2^%d x 2^%d, %d x %d x %d: rel-L2 %.2e" % (ea, eb, M, N, K, r))
+    assert r <= (np.sqrt(K) + 2) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("M,N,K,transb", GEMMS)
+def test_gemm_wide_rows(hip, be, M, N, K, transb):
+    """Rows of A that span the float's range (2^-140 to 2^60, B the other way
+    round, so that every product counts): each result within sqrt(K) 2^-24 of
+    the size of its products."""
+    g = np.random.default_rng(K)
+    e = g.integers(-140, 60, K)
+    A = np.ldexp(g.standard_normal((M, K), dtype=np.float32), e).astype(np.float32)
+    B = g.standard_normal((N, K), dtype=np.float32)
+    B = np.ldexp(B, np.minimum(-e - 20, 100)).astype(np.float32)
+    got = product(hip, be, A, np.ascontiguousarray(B if transb else B.T), transb,
+                  np.zeros((M, N), np.float32))
+    a, b = A[:64].astype(np.float64), B.astype(np.float64)
+    size = np.sqrt((a * a) @ (b * b).T)
+    err = np.abs(got[:64] - a @ b.T) / size
+    print("wide rows %d x %d x %d: %.2e" % (M, N, K, err.max()))
+    assert np.sqrt((err ** 2).mean()) <= (np.sqrt(K) + 2) * 2.0 ** -24
