@@ -1309,8 +1309,8 @@ extern "C" int launch_dec_heads(const float *qry, const void *const w0[4],
  * against 96 MFMAs. 32 prompts at 72 x 72: 209 us against 346 for the product
  * and its scatter.
  *
- * Non-finite tokens or weights make their products NaN; such a product is
- * formed again from the floats in k order. */
+ * Non-finite tokens or weights make their products NaN; a block with such a
+ * product is formed again from the floats by the f32 MFMA. */
 template <int DT>
 __global__ __launch_bounds__(256, 3) void
 k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
@@ -1383,6 +1383,27 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
                             wf[pairs[q][1]], x[s][pairs[q][0]], acc[dd], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int dd = 0; dd < 4; dd++) {
+            unsigned long long bad = 0;
+
+            for (int r = 0; r < 16; r++)
+                bad |= __ballot(!(fabsf(acc[dd][r]) < INFINITY));
+            if (bad) {
+                /* The block by the f32 MFMA from the floats (two k a step, one
+                 * per lane half), its non-finite elements from there. */
+                const int n = 4 * (16 * ((l32 >> 2) & 1) + 4 * (l32 >> 3) + (l32 & 3)) + dd;
+                f32x16 g = {};
+
+#pragma unroll 1
+                for (int k = 0; k < 64; k += 2)
+                    g = __builtin_amdgcn_mfma_f32_32x32x2f32(weight(k + h, n), xr[k - 7 * h], g,
+                                                             0, 0, 0);
+                for (int r = 0; r < 16; r++)
+                    if (!(fabsf(acc[dd][r]) < INFINITY))
+                        acc[dd][r] = g[r];
+            }
+        }
         if (m >= T4)
             continue;
 #pragma unroll
@@ -1398,16 +1419,8 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
                 f32x4 v;
 
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float g = acc[dd][4 * a + e];
-
-                    if (!(fabsf(g) < INFINITY)) {
-                        g = 0.0f;
-                        for (int k = 0; k < 64; k++)
-                            g = fmaf(xr[k - 8 * h], weight(k, 4 * (16 * h + 4 * a + e) + dd), g);
-                    }
-                    v[e] = act_k(g + b[e] + f[e], ACT_GELU_K);
-                }
+                for (int e = 0; e < 4; e++)
+                    v[e] = act_k(acc[dd][4 * a + e] + b[e] + f[e], ACT_GELU_K);
                 *(f32x4 *)(o + 4 * a) = v;
             }
         }

@@ -122,3 +122,44 @@ def test_gemm_wide_rows(hip, be, M, N, K, transb):
     err = np.abs(got[:64] - a @ b.T) / size
     print("wide rows %d x %d x %d: %.2e" % (M, N, K, err.max()))
     assert np.sqrt((err ** 2).mean()) <= (np.sqrt(K) + 2) * 2.0 ** -24
+
+
+def decoder(hip, be, G, P, emb, w, s0):
+    """lowres of P prompts on a G x G image, and the time of its second
+    upscaling (ms)."""
+    model = hip.Model(be, embed=1024, heads=16)
+    model.m.grid = G
+    dec = hip.Decoder(model, w, P, img=14 * G)
+    try:
+        g = np.random.default_rng(3)
+        dec.set_image(emb, s0, g.standard_normal((4 * G * G, 64)).astype(np.float32))
+        pts = g.uniform(0, 14 * G, (P, 2)).astype(np.float32)
+        dec.decode(pts)
+        hip.prof_reset()
+        be.set_profile(True)
+        try:
+            dec.decode(pts)
+        finally:
+            be.set_profile(False)
+        t = [r for r in hip.prof_table() if r[0] == "upscale2"]
+        return dec.lowres(P).copy(), t[0][1]
+    finally:
+        dec.free()
+        model.free()
+
+
+@pytest.mark.parametrize("G,P", [(36, 4), (9, 3)])
+def test_upscaling_nan_cost(hip, be, G, P):
+    """A decode of a NaN image spends at most five times the ordinary time in
+    the second upscaling: its products on the f32 unit beside the same GELUs."""
+    g = np.random.default_rng(G)
+    w = hip.random_decoder_weights(7)
+    emb = g.standard_normal((G * G, 256)).astype(np.float32)
+    s0 = g.standard_normal((16 * G * G, 32)).astype(np.float32)
+    low, t = decoder(hip, be, G, P, emb, w, s0)
+    assert np.isfinite(low).all()
+    emb[G] = np.nan
+    low, tn = decoder(hip, be, G, P, emb, w, s0)
+    assert np.isnan(low).all()
+    print("upscaling G=%d P=%d: %.1f us, NaN %.1f us" % (G, P, 1e3 * t, 1e3 * tn))
+    assert tn <= 5 * t
