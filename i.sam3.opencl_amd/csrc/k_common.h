@@ -63,8 +63,16 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, p);
 }
 
+/* Scale of a float before split4: the lowest bit of any float, subnormals
+ * too, is then at 2^-125 or above, inside bf16's range; |x| >= 2^103
+ * overflows. split_unscale takes it back from a product of a float with an
+ * operand of type DT (halves, two pieces, are not scaled). */
+#define SPLIT_SCALE 0x1p24f
+template <int DT> constexpr float split_unscale = DT == DT_F32 ? 0x1p-48f : 0x1p-24f;
+
 /* Four floats as NP bf16 pieces of four, each the rounding (to nearest) of
- * what the pieces before it leave: three are exactly the float. */
+ * what the pieces before it leave: three are exactly the float for 2^-109 <=
+ * |x| < 2^127, so for every float once scaled by SPLIT_SCALE. */
 template <int NP> __device__ __forceinline__ void split4(const f32x4 x, u32x2 (&p)[NP])
 {
     f32x4 r = x;

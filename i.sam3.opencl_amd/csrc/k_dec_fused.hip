@@ -1296,7 +1296,8 @@ extern "C" int launch_dec_heads(const float *qry, const void *const w0[4],
  * GB of it for 32 prompts at 72 x 72, and a launch).
  *
  * Product on operands split into bf16 pieces (k_gemm_split.hip: three per
- * float, two per half weight, piece pairs down to 2^-16), transposed: weight
+ * float, scaled by SPLIT_SCALE, two per half weight, piece pairs down to
+ * 2^-16), transposed: weight
  * rows are the A operand, tokens the B operand, so a lane holds one token,
  * and with the weight rows of a 32-row block in the order row 8 a + 4 b + e =
  * channel 16 b + 4 a + e (block = dd) it holds 16 consecutive channels of
@@ -1327,6 +1328,7 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
         return DT == DT_F32 ? ((const float *)W)[k * 128 + n]
                             : h2f(((const uint16_t *)W)[k * 128 + n]);
     };
+    const float wscale = DT == DT_F32 ? SPLIT_SCALE : 1.0f;
 
     for (int i = t; i < 1024; i += 256) {
         /* Column n, k octet o: eight loads, lanes along n. */
@@ -1340,8 +1342,8 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
             x[e] = weight(8 * o + e, n);
             y[e] = weight(8 * o + 4 + e, n);
         }
-        split4<NP>(x, lo);
-        split4<NP>(y, hi);
+        split4<NP>(x * wscale, lo);
+        split4<NP>(y * wscale, hi);
         for (int e = 0; e < NP; e++)
             *(u32x4 *)(q + 1024 * e) = (u32x4){lo[e].x, lo[e].y, hi[e].x, hi[e].y};
     }
@@ -1361,8 +1363,8 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
         for (int s = 0; s < 4; s++) {
             u32x2 lo[3], hi[3];
 
-            split4<3>(*(const f32x4 *)(xr + 16 * s), lo);
-            split4<3>(*(const f32x4 *)(xr + 16 * s + 4), hi);
+            split4<3>(*(const f32x4 *)(xr + 16 * s) * SPLIT_SCALE, lo);
+            split4<3>(*(const f32x4 *)(xr + 16 * s + 4) * SPLIT_SCALE, hi);
             for (int e = 0; e < 3; e++)
                 x[s][e] =
                     __builtin_bit_cast(bf16x8, (u32x4){lo[e].x, lo[e].y, hi[e].x, hi[e].y});
@@ -1387,8 +1389,10 @@ k_upscale2_split(const float *__restrict__ u1, const void *__restrict__ W,
         for (int dd = 0; dd < 4; dd++) {
             unsigned long long bad = 0;
 
-            for (int r = 0; r < 16; r++)
+            for (int r = 0; r < 16; r++) {
+                acc[dd][r] *= split_unscale<DT>;
                 bad |= __ballot(!(fabsf(acc[dd][r]) < INFINITY));
+            }
             if (bad) {
                 /* The block by the f32 MFMA from the floats (two k a step, one
                  * per lane half), its non-finite elements from there. */

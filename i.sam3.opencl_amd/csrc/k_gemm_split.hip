@@ -58,10 +58,6 @@ __device__ __forceinline__ int frag_off(int r, int q)
     return 16 * (32 * h + (r ^ (4 * h))) + 8 * (q & 1);
 }
 
-/* Scale of the split floats; the sums carry it once per float operand. */
-#define SPLIT_SCALE 0x1p24f
-template <int BDT> constexpr float split_unscale = BDT == DT_F32 ? 0x1p-48f : 0x1p-24f;
-
 /* A 32 x 32 block of the product by the f32 MFMA from the float operands:
  * lane l's row of A and column of B are l % 32 of the block's; a lane half
  * takes four consecutive k of every eight (K % 4 == 0: in or out together). */

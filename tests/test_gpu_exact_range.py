@@ -163,3 +163,23 @@ def test_upscaling_nan_cost(hip, be, G, P):
     assert np.isnan(low).all()
     print("upscaling G=%d P=%d: %.1f us, NaN %.1f us" % (G, P, 1e3 * t, 1e3 * tn))
     assert tn <= 5 * t
+
+
+def test_upscaling_small_weights(hip, be):
+    """The second upscaling's weights times 2^-118, its bias and map zero: the
+    logits are those of weights times 2^-60 (where GELU is linear too and the
+    pieces are ordinary) times 2^-58, within the rounding of the 64 products."""
+    G, P = 9, 2
+    g = np.random.default_rng(5)
+    emb = g.standard_normal((G * G, 256)).astype(np.float32)
+    s0 = np.zeros((16 * G * G, 32), np.float32)
+    out = []
+    for e in (-60, -118):
+        w = dict(hip.random_decoder_weights(7))
+        w["up3w"] = np.ldexp(w["up3w"], e).astype(np.float32)
+        w["up3b"] = np.zeros_like(w["up3b"])
+        low, _ = decoder(hip, be, G, P, emb, w, s0)
+        out.append(np.ldexp(low.astype(np.float64), -e))
+    r = rel_l2(out[1], out[0])
+    print("upscaling weights 2^-118: rel-L2 %.2e" % r)
+    assert np.abs(out[0]).max() > 0 and r <= 8 * 2.0 ** -24
