@@ -141,8 +141,12 @@ __device__ __forceinline__ bool split_merge(float *__restrict__ part, unsigned *
                 asm volatile("" : "+v"(ch[j][0]), "+v"(ch[j][1]), "+v"(ch[j][2]),
                              "+v"(ch[j][3]), "+v"(ch[j][4]), "+v"(ch[j][5]), "+v"(ch[j][6]),
                              "+v"(ch[j][7]), "+v"(ch[j][8])::"memory");
+                /* (A repeated record with weight 0 would make an infinite sum
+                 * NaN.) */
+                if (s0 + j >= n)
+                    break;
                 const f32x4 ml = __builtin_bit_cast(f32x4, ch[j][8]);
-                const bool take = ml[1] > 0.0f && s0 + j < n;
+                const bool take = ml[1] > 0.0f;
                 const float Mn = take ? fmaxf(M, ml[0]) : M;
                 const float c = take ? __builtin_amdgcn_exp2f(M - Mn) : 1.0f;
                 const float wt = take ? __builtin_amdgcn_exp2f(ml[0] - Mn) : 0.0f;

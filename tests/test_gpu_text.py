@@ -270,3 +270,35 @@ def test_split_operands(hip, be, orc, nq, nk, heads, hd, form, bad):
         assert np.allclose(got[:, :2 * hd][fin], want[:, :2 * hd][fin], rtol=1e-4, atol=1e-4)
         got, want = got[:, cols], want[:, cols]
     assert report("split operands %s %s" % (form, be.precision), got, want) <= TOL[be.precision]
+
+
+@pytest.mark.parametrize("nq,nk,heads,hd,W", [
+    (201, 5184, 8, 32, 72),    # many splits, bias rows
+    (700, 3000, 4, 64, 0),     # few splits
+    (40, 6400, 2, 64, 0),      # one query tile, two merge levels
+])
+def test_split_keys_non_finite(hip, be, nq, nk, heads, hd, W):
+    """One NaN in a key reaches every query of its head, whichever key split
+    holds it, and one infinity in a value every query's channel; the other
+    heads and channels are untouched."""
+    g = np.random.default_rng(nq)
+    Q = g.standard_normal((nq, heads * hd)).astype(np.float32)
+    K, V = (g.standard_normal((nk, heads * hd)).astype(np.float32) for _ in range(2))
+    kw = {}
+    if W:
+        kw = dict(dy=g.standard_normal((nq, nk // W, heads)).astype(np.float32),
+                  dx=g.standard_normal((nq, W, heads)).astype(np.float32), W=W)
+    want = _run(hip, be, Q, K, V, heads, hd, **kw)
+    for key in (3, nk // 2, nk - 1):
+        k, v = K.copy(), V.copy()
+        k[key, 5] = np.nan
+        got = _run(hip, be, Q, k, V, heads, hd, **kw)
+        assert np.isnan(got[:, :hd]).all()
+        assert np.array_equal(got[:, hd:], want[:, hd:])
+        if be.precision == "bf16":
+            continue
+        v[key, 6] = -np.inf
+        got = _run(hip, be, Q, K, v, heads, hd, **kw)
+        assert np.array_equal(got[:, 6], np.full(nq, -np.inf, np.float32)), key
+        cols = np.arange(heads * hd) != 6
+        assert report("split keys, one infinity", got[:, cols], want[:, cols]) <= TOL["fp32"]
