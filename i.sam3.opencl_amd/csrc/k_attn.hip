@@ -601,9 +601,10 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
  * 32: 5184 x 5184 276 -> 163. The error against 64 bits is lower at every size
  * measured (5184 keys: 1.15e-6 against 1.34e-6).
  *
- * A non-finite operand makes every result it enters NaN; a query whose
- * result comes out non-finite is formed again from the float operands
- * (exact_row_seq), so infinities and NaN travel as in k_attn_f32. */
+ * A non-finite operand makes every result it enters NaN; a wave with such a
+ * query forms its part again from the float operands on the f32 MFMA
+ * (attn_wave_f32) and takes those queries from there, so infinities and NaN
+ * travel as in k_attn_f32, at a few times its cost. */
 
 /* Bytes of a key block's fragments: K [HD / 16][3], then V^T [HD / 32][2]
  * [3], 1 KiB each. */
@@ -685,68 +686,82 @@ __global__ __launch_bounds__(256) void k_kv_split(attn_desc d, char *__restrict_
     }
 }
 
-/* Columns 8 g + 4 h .. + 3 (g < HD / 8) of query qi's result from the float
- * operands, one key after another (non-finite results). */
+/* A wave's 32 queries over key blocks kb0 .. kb1 - 1 from the float operands
+ * on the f32 MFMA, k_attn_f32's arithmetic without its staging (for queries
+ * whose result came out non-finite): q the lane's query row (query qi), K
+ * and V row 0 of the unit's; o0, o1 (16 each), m, l into out. Operands are
+ * read eight channels at a time, HD / 2 of them by a lane half. The
+ * registers are kept below k_attn_split's. */
 template <int HD, bool EXT>
-__device__ __noinline__ void exact_row_seq(attn_desc d, long unit, int qi, const float *brow,
-                                           int bH, float *o)
+__device__ __forceinline__ void attn_wave_f32(const float *q, const float *K, int ldk, const float *V,
+                                           int ldv, int Nk, const float2 *rope, int npos,
+                                           float scale, int causal, const float *brow, int bH,
+                                           int bW, int qi, int kb0, int kb1, float *out)
 {
-    /* A score is the same number in both passes, however large. */
-#pragma clang fp contract(off)
-    const int h = (threadIdx.x & 63) >> 5;
-    const long b0 = unit / d.nb1, b1 = unit % d.nb1;
-    const float *q = (const float *)d.Q + d.qoff + b0 * d.sq0 + b1 * d.sq1 + (long)qi * d.ldq;
-    const float *K = (const float *)d.K + d.koff + b0 * d.sk0 + b1 * d.sk1;
-    const float *V = (const float *)d.V + d.voff + b0 * d.sv0 + b1 * d.sv1;
-    const float2 *cs = HD == 64 ? (const float2 *)d.rope : nullptr;
-    float mx = -INFINITY, l = 0.0f;
+    const int l = threadIdx.x & 63, h = l >> 5, l32 = l & 31;
+    attn_desc d; /* what exact_softmax reads of it */
+    auto load8 = [&](const float *row, int pos, float (&x)[8]) {
+        for (int e = 0; e < 8; e++)
+            x[e] = row[e];
+        if (HD == 64 && rope)
+            for (int j = 0; j < 4; j++) {
+                const float a = x[2 * j], b = x[2 * j + 1];
+                const float2 r = rope[pos + j];
 
-    for (int e = 0; e < HD / 2; e++)
-        o[e] = 0.0f;
-    for (int pass = 0; pass < 2; pass++)
-        for (int key = 0; key < d.Nk; key++) {
-            const float *k = K + (long)key * d.ldk;
-            float s = 0.0f;
-
-            for (int j = 0; j < HD / 2; j++) {
-                float qa = q[2 * j], qb = q[2 * j + 1], ka = k[2 * j], kb = k[2 * j + 1];
-
-                if (cs) {
-                    const float2 rq = cs[(long)(qi % d.npos) * 32 + j];
-                    const float2 rk = cs[(long)(key % d.npos) * 32 + j];
-                    const float a = qa, c = ka;
-
-                    qa = fmaf(a, rq.x, -(qb * rq.y));
-                    qb = fmaf(a, rq.y, qb * rq.x);
-                    ka = fmaf(c, rk.x, -(kb * rk.y));
-                    kb = fmaf(c, rk.y, kb * rk.x);
-                }
-                s = fmaf(qb, kb, fmaf(qa, ka, s));
+                x[2 * j] = fmaf(a, r.x, -(b * r.y));
+                x[2 * j + 1] = fmaf(a, r.y, b * r.x);
             }
-            if (EXT && brow) {
-                const float b = d.bW > 0 ? brow[key / d.bW] + brow[bH + key % d.bW] : brow[key];
+    };
+    exact_state st;
 
-                s = (s * d.scale + b) * LOG2E_F;
-            }
-            else
-                s *= d.scale * LOG2E_F;
-            if (EXT && d.causal && key > qi)
-                s = -INFINITY;
-            if (pass == 0)
-                mx = fmaxf(mx, s);
-            else {
-                const float p = __builtin_amdgcn_exp2f(s - (mx == -INFINITY ? 0.0f : mx));
+    d.Nk = Nk;
+    d.scale = scale;
+    d.causal = causal;
+    d.bW = bW;
+    st.o0 = st.o1 = (f32x16){};
+    st.m = st.l = 0.0f;
+#pragma unroll 1
+    for (int kb = kb0; kb < kb1; kb++) {
+        /* Keys past Nk repeat the last one; their weights are zero. */
+        const int key = min(kb * 32 + l32, Nk - 1);
+        const int kp = HD == 64 && rope ? key % npos * 32 : 0;
+        const int qp = HD == 64 && rope ? qi % npos * 32 : 0;
+        f32x16 s = {};
 
-                l += p;
-                for (int e = 0; e < HD / 2; e++)
-                    o[e] = fmaf(p, V[(long)key * d.ldv + 8 * (e >> 2) + 4 * h + (e & 3)], o[e]);
-            }
+#pragma unroll 1
+        for (int c = HD / 2 * h; c < HD / 2 * (h + 1); c += 8) {
+            float x[8], y[8];
+
+            load8(K + (long)key * ldk + c, kp + c / 2, x);
+            load8(q + c, qp + c / 2, y);
+            for (int e = 0; e < 8; e++)
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], s, 0, 0, 0);
         }
-    o[HD / 2] = l;
+        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int kv = kb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+            const float *v = V + (long)min(kv, Nk - 1) * ldv + l32;
+
+            st.o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv < Nk ? v[0] : 0.0f, s[i], st.o0, 0, 0,
+                                                         0);
+            if (HD == 64)
+                st.o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv < Nk ? v[32] : 0.0f, s[i], st.o1,
+                                                             0, 0, 0);
+            if ((i & 3) == 3)
+                __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (int r = 0; r < 16; r++) {
+        out[r] = st.o0[r];
+        out[16 + r] = st.o1[r];
+    }
+    out[32] = st.m;
+    out[33] = st.l + __shfl_xor(st.l, 32, 64);
 }
 
 template <int HD, bool EXT, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void k_attn_split(attn_desc d, const char *__restrict__ kv,
+__global__ __launch_bounds__(256, HD == 32 ? 4 : 2) void k_attn_split(attn_desc d, const char *__restrict__ kv,
                                                        float *__restrict__ part,
                                                        unsigned *__restrict__ cnt, int nsplit)
 {
@@ -885,37 +900,40 @@ __global__ __launch_bounds__(256, 2) void k_attn_split(attn_desc d, const char *
     __builtin_amdgcn_s_setprio(0);
 
     st.l += __shfl_xor(st.l, 32, 64);
-    auto finite = [&]() {
+    {
+        /* A query with a non-finite result in either lane half. */
         float sum = st.l;
 
         for (int r = 0; r < 16; r++)
             sum += (st.o0[r] - st.o0[r]) + (HD == 64 ? st.o1[r] - st.o1[r] : 0.0f);
-        return fabsf(sum) < INFINITY;
-    };
+        const unsigned long long b = __ballot(qi < N && !(fabsf(sum) < INFINITY));
 
-    if constexpr (SPLIT) {
-        /* A split that is not finite outweighs the others in the merge. */
-        if (!finite()) {
-            st.m = 1e30f;
-            st.l = INFINITY;
+        if (b) {
+            float o[34];
+
+            attn_wave_f32<HD, EXT>(
+                (const float *)d.Q + d.qoff + b0 * d.sq0 + b1 * d.sq1 + (long)min(qi, N - 1) * d.ldq,
+                (const float *)d.K + d.koff + b0 * d.sk0 + b1 * d.sk1, d.ldk,
+                (const float *)d.V + d.voff + b0 * d.sv0 + b1 * d.sv1, d.ldv, Nk,
+                (const float2 *)d.rope, d.npos, d.scale, d.causal, brow, bH, d.bW,
+                min(qi, N - 1), kb0, kb1, o);
+            if ((b | b >> 32) >> l32 & 1) {
+                for (int r = 0; r < 16; r++) {
+                    st.o0[r] = o[r];
+                    if (HD == 64)
+                        st.o1[r] = o[16 + r];
+                }
+                st.m = o[32];
+                st.l = o[33];
+            }
         }
+    }
+    if constexpr (SPLIT)
         if (!split_merge<HD == 64>(part, cnt, item, nsplit, sp, !idle, st.o0, st.o1, st.m, st.l))
             return;
-    }
-    if (qi >= N)
-        return;
-    if (!finite()) {
-        float o[HD / 2 + 1];
-
-        exact_row_seq<HD, EXT>(d, unit, qi, brow, bH, o);
-        st.l = o[HD / 2];
-        for (int r = 0; r < 16; r++) {
-            st.o0[r] = o[r];
-            if (HD == 64)
-                st.o1[r] = o[HD / 4 + r];
-        }
-    }
-    exact_store<HD>(d, d.ooff + b0 * d.so0 + b1 * d.so1 + (long)qi * d.ldo, st.o0, st.o1, st.l);
+    if (qi < N)
+        exact_store<HD>(d, d.ooff + b0 * d.so0 + b1 * d.so1 + (long)qi * d.ldo, st.o0, st.o1,
+                        st.l);
 }
 
 /* ------------------------------------------------------------ packing */

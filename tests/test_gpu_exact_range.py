@@ -183,3 +183,42 @@ def test_upscaling_small_weights(hip, be):
     r = rel_l2(out[1], out[0])
     print("upscaling weights 2^-118: rel-L2 %.2e" % r)
     assert np.abs(out[0]).max() > 0 and r <= 8 * 2.0 ** -24
+
+
+def attention(hip, be, Q, K, V, heads, hd, causal=False):
+    """attend of Nq queries over Nk keys, and its time (ms)."""
+    D = heads * hd
+    m = hip.Model(be, embed=128, heads=2)
+    dq, dk, dv = be.upload(Q), be.upload(K), be.upload(V)
+    do = be.alloc(Q.size * 4)
+    try:
+        t = ms(be, lambda: hip.attend(m, Q.shape[0], K.shape[0], heads, hd, dq, D, dk, D, dv, D,
+                                      do, D, causal, None, None, 0))
+        return be.read(do).reshape(Q.shape), t
+    finally:
+        for x in (dq, dk, dv, do):
+            be.release(x)
+        m.free()
+
+
+def normal(g, n, D, e=0):
+    return np.ldexp(g.standard_normal((n, D), dtype=np.float32), e).astype(np.float32)
+
+
+# Split operands, one split and several; the f32 MFMA kernel.
+ATTENTIONS = [(1601, 1601, 16, 64, False), (1000, 2000, 6, 64, False), (1300, 1300, 16, 32, False),
+              (1500, 1500, 12, 64, True), (201, 700, 8, 32, False)]
+
+
+@pytest.mark.parametrize("nq,nk,heads,hd,causal", ATTENTIONS)
+def test_attention_nan_cost(hip, be, nq, nk, heads, hd, causal):
+    """An attention of NaN takes at most ten times the ordinary one."""
+    g = np.random.default_rng(nq)
+    q, k, v = (normal(g, n, heads * hd) for n in (nq, nk, nk))
+    _, t = attention(hip, be, q, k, v, heads, hd, causal)
+    k[0] = np.nan
+    got, tn = attention(hip, be, q, k, v, heads, hd, causal)
+    assert np.isnan(got).all()
+    print("attention %d x %d, %d x %d: %.1f us, NaN %.1f us" % (nq, nk, heads, hd, 1e3 * t,
+                                                                1e3 * tn))
+    assert tn <= 10 * t
