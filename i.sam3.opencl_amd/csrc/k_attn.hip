@@ -259,17 +259,17 @@ struct exact_state {
  * max (its cross-lane exchange, the rescale of O and l) only for blocks
  * whose in-lane maxima it cannot clear; O / l does not depend on m. */
 template <int HD, bool EXT>
-__device__ __forceinline__ f32x16 exact_softmax(const attn_desc &d, f32x16 s, int kb, bool first,
-                                                int qi, const float *brow, int bH,
+__device__ __forceinline__ f32x16 exact_softmax(const attn_desc &d, float scale, f32x16 s, int kb,
+                                                bool first, int qi, const float *brow, int bH,
                                                 exact_state &st)
 {
     const int h = (threadIdx.x & 63) >> 5, Nk = d.Nk;
-    const float sc2 = d.scale * LOG2E_F;
+    const float sc2 = scale * LOG2E_F;
     float rs = 0.0f, mx = -INFINITY;
 
     if (EXT && brow) {
         for (int r = 0; r < 16; r++)
-            s[r] *= d.scale;
+            s[r] *= scale;
         if (d.bW > 0) {
             const int yb = kb * 32 / d.bW, xb = kb * 32 - yb * d.bW;
 
@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
     };
     /* The block's weights, then O^T += V^T P^T from buffer buf. */
     auto soft_pv = [&](f32x16 s, int kb, int buf) {
-        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
+        s = exact_softmax<HD, EXT>(d, d.scale, s, kb, kb == kb0, qi, brow, bH, st);
         /* The exponentials issued before the P V MFMAs: left to the
          * scheduler, which weighs the code after the key loop too, each
          * MFMA could follow the exponential it reads and wait for it
@@ -583,9 +583,10 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
 
 /* ------------------------------------------------------------ fp32 path, split operands */
 
-/* The exact path of larger problems: K, V and Q, and the weights P, as three
- * bf16 pieces each (exactly the float, split4), six piece products per
- * product on v_mfma_f32_32x32x16_bf16 with f32 accumulation, the three below
+/* The exact path of larger problems: K, V and Q, scaled by SPLIT_SCALE, as
+ * three bf16 pieces each (exactly the float, split4), and the weights P too
+ * (what falls out of bf16's range is below 2^-133 of weights whose sum is
+ * 2^-64 at least), six piece products per product on v_mfma_f32_32x32x16_bf16 with f32 accumulation, the three below
  * 2^-24 of it dropped: what the f32 MFMA of k_attn_f32 forms at a sixteenth
  * of the rate. K (rotated) and V^T are split once per call by
  * k_kv_split into MFMA fragments, which this kernel copies HBM -> LDS
@@ -601,8 +602,8 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
  * 32: 5184 x 5184 276 -> 163. The error against 64 bits is lower at every size
  * measured (5184 keys: 1.15e-6 against 1.34e-6).
  *
- * A non-finite operand makes every result it enters NaN; a wave with such a
- * query forms its part again from the float operands on the f32 MFMA
+ * A non-finite operand, or one past 2^103, makes every result it enters NaN,
+ * a score past 2^80 is infinite; a wave with such a query forms its part again from the float operands on the f32 MFMA
  * (attn_wave_f32) and takes those queries from there, so infinities and NaN
  * travel as in k_attn_f32, at a few times its cost. */
 
@@ -652,8 +653,8 @@ __global__ __launch_bounds__(256) void k_kv_split(attn_desc d, char *__restrict_
             }
         }
         for (int e = 0; e < 8; e++) {
-            Ks[kr][dc + e] = k[e];
-            Vs[kr][dc + e] = v[e];
+            Ks[kr][dc + e] = k[e] * SPLIT_SCALE;
+            Vs[kr][dc + e] = v[e] * SPLIT_SCALE;
         }
     }
     __syncthreads();
@@ -715,7 +716,6 @@ __device__ __forceinline__ void attn_wave_f32(const float *q, const float *K, in
     exact_state st;
 
     d.Nk = Nk;
-    d.scale = scale;
     d.causal = causal;
     d.bW = bW;
     st.o0 = st.o1 = (f32x16){};
@@ -737,7 +737,7 @@ __device__ __forceinline__ void attn_wave_f32(const float *q, const float *K, in
             for (int e = 0; e < 8; e++)
                 s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], s, 0, 0, 0);
         }
-        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
+        s = exact_softmax<HD, EXT>(d, scale, s, kb, kb == kb0, qi, brow, bH, st);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int kv = kb * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
@@ -806,6 +806,7 @@ __global__ __launch_bounds__(256, HD == 32 ? 4 : 2) void k_attn_split(attn_desc 
     };
     bf16x8 q[NS][3];
     exact_state st;
+    const float scale = d.scale * split_unscale<DT_F32>; /* of scores from scaled Q and K */
 
     load(kb0, 0);
     /* Q: the lane's channels 16 s + 8 h .. + 7 of query qi, rotated, split. */
@@ -833,8 +834,8 @@ __global__ __launch_bounds__(256, HD == 32 ? 4 : 2) void k_attn_split(attn_desc 
         }
         u32x2 lo[3], hi[3];
 
-        split4<3>((f32x4){x[0], x[1], x[2], x[3]}, lo);
-        split4<3>((f32x4){x[4], x[5], x[6], x[7]}, hi);
+        split4<3>((f32x4){x[0], x[1], x[2], x[3]} * SPLIT_SCALE, lo);
+        split4<3>((f32x4){x[4], x[5], x[6], x[7]} * SPLIT_SCALE, hi);
         for (int p = 0; p < 3; p++)
             q[s][p] = __builtin_bit_cast(bf16x8, (u32x4){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
     }
@@ -866,7 +867,7 @@ __global__ __launch_bounds__(256, HD == 32 ? 4 : 2) void k_attn_split(attn_desc 
                 s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[pairs[p][0]], q[i][pairs[p][1]], s,
                                                             0, 0, 0);
         }
-        s = exact_softmax<HD, EXT>(d, s, kb, kb == kb0, qi, brow, bH, st);
+        s = exact_softmax<HD, EXT>(d, scale, s, kb, kb == kb0, qi, brow, bH, st);
         bf16x8 pf[2][3];
 
 #pragma unroll
@@ -901,12 +902,20 @@ __global__ __launch_bounds__(256, HD == 32 ? 4 : 2) void k_attn_split(attn_desc 
 
     st.l += __shfl_xor(st.l, 32, 64);
     {
-        /* A query with a non-finite result in either lane half. */
+        /* A query with a non-finite result in either lane half, or without
+         * weight though it sees a key of the split (scores below -2^80 have
+         * overflowed). */
         float sum = st.l;
 
-        for (int r = 0; r < 16; r++)
+        for (int r = 0; r < 16; r++) {
+            st.o0[r] *= 1.0f / SPLIT_SCALE;
+            if (HD == 64)
+                st.o1[r] *= 1.0f / SPLIT_SCALE;
             sum += (st.o0[r] - st.o0[r]) + (HD == 64 ? st.o1[r] - st.o1[r] : 0.0f);
-        const unsigned long long b = __ballot(qi < N && !(fabsf(sum) < INFINITY));
+        }
+        const bool sees = !(EXT && d.causal) || kb0 * 32 <= qi;
+        const unsigned long long b =
+            __ballot(qi < N && (!(fabsf(sum) < INFINITY) || (st.l == 0.0f && sees)));
 
         if (b) {
             float o[34];
@@ -2339,7 +2348,8 @@ extern "C" size_t attn_split_ws(const attn_desc *d)
     const double ops = 4.0 * d->nb * (double)d->N * d->Nk * d->hd;
     const double keys = (double)d->nb * d->Nk * d->hd;
 
-    if (d->nb > 65535 || ops * 4.0e-15 < keys * 5.0e-12 + 5e-6)
+    /* The scores' scale carries 2^-48 (SPLIT_SCALE squared) and stays normal. */
+    if (!(fabsf(d->scale) >= 0x1p-60f) || d->nb > 65535 || ops * 4.0e-15 < keys * 5.0e-12 + 5e-6)
         return 0;
     return (size_t)d->nb * (((size_t)d->Nk + 31) / 32) * KVS_BLOCK((size_t)d->hd);
 }

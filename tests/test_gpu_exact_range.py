@@ -222,3 +222,62 @@ def test_attention_nan_cost(hip, be, nq, nk, heads, hd, causal):
     print("attention %d x %d, %d x %d: %.1f us, NaN %.1f us" % (nq, nk, heads, hd, 1e3 * t,
                                                                 1e3 * tn))
     assert tn <= 10 * t
+
+
+def softmax_rows64(q, k, v, heads, hd, causal, rows):
+    """Sampled queries in 64 bits."""
+    out = np.empty((len(rows), heads * hd))
+    for h in range(heads):
+        c = slice(h * hd, (h + 1) * hd)
+        s = q[rows][:, c].astype(np.float64) @ k[:, c].astype(np.float64).T / np.sqrt(hd)
+        if causal:
+            s[np.arange(k.shape[0])[None] > rows[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, c] = p / p.sum(1, keepdims=True) @ v[:, c].astype(np.float64)
+    return out
+
+
+@pytest.mark.parametrize("eq,ek,ev", [
+    (118, -118, 0),     # low pieces of K below bf16's range
+    (-122, 122, 0),     # Q small, K past the range that splits
+    (0, 0, -118),       # small values
+    (110, -110, 100),   # Q and V past the split's range
+])
+@pytest.mark.parametrize("nq,nk,heads,hd,causal", ATTENTIONS)
+def test_attention_magnitudes(hip, be, nq, nk, heads, hd, causal, eq, ek, ev):
+    """Queries, keys and values times powers of two: the ordinary attention
+    (queries times 2^(eq + ek), which the scores carry) times 2^ev. Scores are
+    sums of hd products (their error, times the score's size of about 4, enters
+    the weights) and outputs of nk: 4 sqrt(hd) + sqrt(nk) roundings."""
+    g = np.random.default_rng(nq + 200 + ek)
+    q, k, v = (normal(g, n, heads * hd, e) for n, e in ((nq, eq), (nk, ek), (nk, ev)))
+    got, _ = attention(hip, be, q, k, v, heads, hd, causal)
+    rows = np.unique(np.concatenate([np.arange(33), [nq - 1], g.integers(0, nq, 40)]))
+    want = softmax_rows64(q, k, np.ldexp(v.astype(np.float64), -ev), heads, hd, causal, rows)
+    r = rel_l2(np.ldexp(got[rows].astype(np.float64), -ev), want)
+    print("attention 2^%d 2^%d 2^%d, %d x %d x %d: rel-L2 %.2e" % (eq, ek, ev, nq, nk, hd, r))
+    assert r <= (4 * np.sqrt(hd) + np.sqrt(nk)) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("nq,nk,heads,hd,causal", ATTENTIONS)
+def test_attention_scores_past_the_split_range(hip, be, nq, nk, heads, hd, causal, sign):
+    """Scores of 2^88, all of one sign (below zero they must not turn into a
+    mask): the softmax is one-hot, each output the value row of the largest
+    score."""
+    g = np.random.default_rng(nq)
+    q = np.abs(normal(g, nq, heads * hd, 45)) + np.float32(2.0 ** 44)
+    k = sign * (np.abs(normal(g, nk, heads * hd, 40)) + np.float32(2.0 ** 39))
+    v = normal(g, nk, heads * hd)
+    got, _ = attention(hip, be, q, k.astype(np.float32), v, heads, hd, causal)
+    rows = np.arange(0, nq, 37)
+    for h in range(heads):
+        c = slice(h * hd, (h + 1) * hd)
+        s = q[rows][:, c].astype(np.float64) @ k[:, c].astype(np.float64).T
+        if causal:
+            s[np.arange(nk)[None] > rows[:, None]] = -np.inf
+        top = np.sort(s, 1)[:, -2:]
+        # Clear of the scores' own rounding (hd terms of 2^-24 each).
+        sure = np.diff(top)[:, 0] > hd * 2.0 ** -23 * np.abs(top[:, 1])
+        assert sure.sum() > len(rows) // 2
+        assert np.array_equal(got[rows][sure][:, c], v[s.argmax(1)][sure][:, c])
