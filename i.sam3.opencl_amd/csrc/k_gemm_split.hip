@@ -109,20 +109,21 @@ __device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[N
         for (int i = 0; i < NA; i++) {
             const int mb = m0 + 32 * i;
             unsigned long long bad = 0;
+            float alpha = d.alpha * split_unscale<BDT>;
 
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                acc[i][j][r] *= split_unscale<BDT>;
+            for (int r = 0; r < 16; r++)
                 bad |= __ballot(!(fabsf(acc[i][j][r]) < __builtin_inff()));
-            }
             if (bad) {
                 const f32x16 x = block_f32<BDT>(arow(min(mb + l32, d.M - 1)),
                                                 bcol(min(n, d.N - 1)), d.transb ? 1L : d.ldb, d.K);
 
 #pragma unroll
                 for (int r = 0; r < 16; r++)
-                    if (!(fabsf(acc[i][j][r]) < __builtin_inff()))
-                        acc[i][j][r] = x[r];
+                    acc[i][j][r] = fabsf(acc[i][j][r]) < __builtin_inff()
+                                       ? acc[i][j][r] * split_unscale<BDT>
+                                       : x[r];
+                alpha = d.alpha;
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -131,7 +132,7 @@ __device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[N
 
                 if (m >= d.M || n >= d.N)
                     continue;
-                v = act_k(d.alpha * v + bn, d.act);
+                v = act_k(alpha * v + bn, d.act);
                 if (R)
                     v += R[(long)m * d.ldc + n];
                 C[(long)m * d.ldc + n] = v;
@@ -475,7 +476,7 @@ __device__ __forceinline__ void gs_vmwait0()
  * reads): with a branch in it the compiler kept a second copy of the
  * accumulators, 128 moves per step (145 against 180 TFLOP/s). */
 template <int BM, int BN, int WM, int WN, int BDT, bool WIN>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, BM * BN >= 256 * 128 ? 4 : 1) void
 k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
 {
     constexpr int NW = (BM / WM) * (BN / WN), NSLOT = 2;
@@ -705,6 +706,9 @@ static int gs_aligned(const gemm_desc *d)
 {
     const long a = d->aoff | d->sa0 | d->sa1 | d->lda, b = d->boff | d->sb0 | d->sb1 | d->ldb;
 
+    /* alpha carries the scale of the pieces (2^-48) and stays normal. */
+    if (d->alpha != 0.0f && !(fabsf(d->alpha) >= 0x1p-60f))
+        return 0;
     if (d->mode != MODE_F32 || d->adt != DT_F32 || d->cdt != DT_F32 || d->bdt == DT_BF16 ||
         d->unpart_ws > 0 || d->pack_N > 0 || d->K < 4 || d->K % 4 || a % 4 ||
         ((uintptr_t)d->A & 15))
