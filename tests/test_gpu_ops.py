@@ -501,3 +501,37 @@ def test_gemm_small_bf16(hip, be16, orc, M, N, K, act, abf, cbf):
     if cbf:
         tol = tol + 2.0 ** -8 * np.abs(want)
     assert np.all(np.abs(got - want) <= tol)
+
+
+def us(be, call):
+    """The fastest of five launches in a row, by events."""
+    call()
+    best = 1e9
+    for _ in range(5):
+        be.finish()
+        be.timer_start()
+        call()
+        best = min(best, 1e3 * be.timer_stop())
+    return best
+
+
+@pytest.mark.parametrize("M,N,K,transb,nb", [(16, 16, 16, 0, 1000), (64, 64, 64, 0, 1000),
+                                             (16, 64, 32, 0, 777)])
+def test_gemm_many_tiny_products(hip, be, M, N, K, transb, nb):
+    """A thousand products of a tile each cost at most three times one (they
+    fit the chip at once), and are right."""
+    m = model(hip, be)
+    g = rng(M + nb)
+    A = g.standard_normal((nb, M, K), dtype=np.float32)
+    B = g.standard_normal((nb, K, N), dtype=np.float32)
+    dA, dB, dC = be.upload(A), be.upload(B), be.alloc(nb * M * N * 4)
+
+    def run(n):
+        hip.gemm(m, M, N, K, hip.bmat(dA, 0, K, M * K, 0), hip.bmat(dB, 0, N, K * N, 0), transb,
+                 hip.bmat(dC, 0, N, M * N, 0), n, 1)
+
+    one, many = us(be, lambda: run(1)), us(be, lambda: run(nb))
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert rel_l2(be.read(dC).reshape(nb, M, N), want) <= (np.sqrt(K) + 2) * 2.0 ** -24
+    print("%d x %d x %d: one %.1f us, %d %.1f us" % (M, N, K, one, nb, many))
+    assert many <= 3 * one
