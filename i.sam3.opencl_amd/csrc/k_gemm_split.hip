@@ -728,14 +728,22 @@ static long gs_tiles(const gemm_desc *d, int bm, int bn)
     return (long)((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn);
 }
 
-/* Small: at most one 64 x 64 tile per two CUs (of one batch: the kernel, and
- * so the bits, do not depend on how many are in a call), where a staged tile's K loop
+/* Small: at most one 64 x 64 tile per two CUs, where a staged tile's K loop
  * is all latency (400 x 1024 x 1024, 112 tiles: 25 us against 30; 1000 x 1024
  * x 1024, 256 tiles: 49 against 31; 1000 x 300 x 4096, 80 tiles: 73 against
- * 137). */
+ * 137). Of a batch only products of up to three tiles or 32 rows or columns:
+ * above that a batch fills the chip and the small kernel, which reads its
+ * operands once per 16 columns, is bound by the caches (576 x 576 x 64: 16
+ * products 34 us against 15, 144 272 against 80; 64 products of 256 x 256 x
+ * 128 40 against 21). A batch is told by its strides, not by how many
+ * products the call holds, so that a call's bits do not depend on that. */
 static int gs_small(const gemm_desc *d)
 {
-    return d->transb && gs_tiles(d, 64, 64) * 2 <= dev_cu_count();
+    const long tiles = gs_tiles(d, 64, 64);
+    const int batch = (d->sa0 | d->sa1 | d->sb0 | d->sb1 | d->sc0 | d->sc1) != 0;
+
+    return d->transb && tiles * 2 <= dev_cu_count() &&
+           !(batch && tiles > 3 && d->M > 32 && d->N > 32);
 }
 
 /* Rows of A per packed chunk: at most 512 MiB of pieces. */

@@ -535,3 +535,33 @@ def test_gemm_many_tiny_products(hip, be, M, N, K, transb, nb):
     assert rel_l2(be.read(dC).reshape(nb, M, N), want) <= (np.sqrt(K) + 2) * 2.0 ** -24
     print("%d x %d x %d: one %.1f us, %d %.1f us" % (M, N, K, one, nb, many))
     assert many <= 3 * one
+
+
+@pytest.mark.parametrize("n,K,nb", [(576, 64, 144), (196, 64, 256), (256, 128, 64)])
+def test_gemm_batch_costs_what_its_size_does(hip, be, n, K, nb):
+    """A batch of Q K^T sized products takes at most 1.8 times one product
+    with as many operations and results, and each product's bits do not
+    depend on how many the call holds."""
+    m = model(hip, be)
+    g = rng(n + nb)
+    A = g.standard_normal((nb, n, K), dtype=np.float32)
+    B = g.standard_normal((nb, n, K), dtype=np.float32)
+    dA, dB, dC = be.upload(A), be.upload(B), be.alloc(nb * n * n * 4)
+
+    def run(first, count):
+        hip.gemm(m, n, n, K, hip.bmat(dA, first * n * K, K, n * K, 0),
+                 hip.bmat(dB, first * n * K, K, n * K, 0), 1,
+                 hip.bmat(dC, first * n * n, n, n * n, 0), count, 1)
+
+    batch = us(be, lambda: run(0, nb))
+    got = be.read(dC).reshape(nb, n, n)
+    rows = g.integers(0, n, 20)
+    want = A[:, rows].astype(np.float64) @ B.astype(np.float64).transpose(0, 2, 1)
+    assert rel_l2(got[:, rows], want) <= (np.sqrt(K) + 2) * 2.0 ** -24
+    for first in (0, 3, nb - 1):
+        run(first, 1)
+        assert np.array_equal(be.read(dC, n * n, off=4 * first * n * n).reshape(n, n), got[first])
+    one = us(be, lambda: hip.gemm(m, nb * n, n, K, hip.mat(dA, 0, K), hip.mat(dB, 0, K), 1,
+                                  hip.mat(dC, 0, n)))
+    print("%d x %d x %d x %d: %.1f us, as one product %.1f us" % (nb, n, n, K, batch, one))
+    assert batch <= 1.8 * one
