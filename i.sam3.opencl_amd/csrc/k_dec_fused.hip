@@ -1073,12 +1073,12 @@ __global__ __launch_bounds__(256) void k_t2i_end(const float *__restrict__ part,
     const int p = blockIdx.x, h = blockIdx.y, t = threadIdx.x;
     const int q = t & 7, c = (t >> 3) & 15, i0 = 4 * (t >> 7);
     const float *ml = part + (long)P * nsplit * FOLD_ROWS * 256;
-    const u32x4 *wr = (const u32x4 *)((const char *)Wv +
-                                      (long)(16 * h + c) * 256 * (DT == DT_F32 ? 4 : 2));
+    const char *wr = (const char *)Wv + (long)(16 * h + c) * 256 * (DT == DT_F32 ? 4 : 2) + 16 * q;
     u32x4 wv[N];
 
+    /* 16 bytes each at the element's alignment (any will do for Wv). */
     for (int i = 0; i < N; i++)
-        wv[i] = wr[8 * i + q];
+        __builtin_memcpy(&wv[i], wr + 128 * i, 16);
     {
         /* The 8 rows' split weights, 32 lanes a row, then their sum. */
         const int i = t >> 5, l = t & 31;
@@ -1148,10 +1148,12 @@ extern "C" int launch_t2i_fused(const float *keys, const void *pk16,
 {
     const int nblk = (T + 63) / 64;
 
-    if (P < 1 || T < 1 || nsplit < 1 || nsplit > nblk ||
-        nsplit > T2I_MAX_SPLIT || (long)P * nsplit > 0x7fffffffL || !pk16 || !Qc16 ||
+    if (nsplit > T2I_MAX_SPLIT)
+        nsplit = T2I_MAX_SPLIT;
+    if (P < 1 || T < 1 || nsplit < 1 || nsplit > nblk || (long)P * nsplit > 0x7fffffffL ||
+        !pk16 || !Qc16 ||
         (((uintptr_t)keys | (uintptr_t)pk16 | (uintptr_t)U16 | (uintptr_t)Qc16 |
-          (uintptr_t)part | (uintptr_t)Wv) & 15))
+          (uintptr_t)part) & 15))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_t2i_fused, dim3((unsigned)((P * nsplit + 7) / 8 * 8)),
                        dim3(256), 0, (hipStream_t)stream, keys,

@@ -333,3 +333,45 @@ def test_postprocess_many_planes(hip, be, orc, weights):
         assert np.array_equal(d.dec.read_mask(299, 21, 33, 0, 0, 32, 20), mask[299])
     finally:
         d.free()
+
+
+def test_t2i_unaligned_value_weights(hip, orc, weights):
+    """precision=bf16: the value projection's weights at a byte address that
+    is only the element's, in every element type, give the same tokens as
+    aligned ones."""
+    G, P = 16, 2
+    b = hip.Backend(precision="bf16")
+    d = Dec(hip, b, orc, weights, G, P, 64)
+    try:
+        g = np.random.default_rng(65)
+        qry = g.standard_normal((P, 8, 256)).astype(np.float32)
+        for name, shape in (("qpe", (P, 8, 256)), ("keys", (P, G * G, 256))):
+            b.write(d.dec.buf(name), 0, g.standard_normal(shape).astype(np.float32))
+        a = d.dec.d.layers[1].t2i
+        w = b.read_f32(a.vw).reshape(128, 256)
+        aligned = a.vw
+
+        def tokens(mem):
+            a.vw = mem
+            b.write(d.dec.buf("qry"), 0, qry)
+            hip.t2i_attention(d.model, d.dec, P, a)
+            return b.read_f32(d.dec.buf("qry"), P * 8 * 256).copy()
+
+        want = tokens(aligned)
+        for dt, dtype in ((hip.F32, np.float32), (hip.F16, np.float16), (hip.BF16, None)):
+            bits = (w.view(np.uint32) >> 16).astype(np.uint16) if dtype is None else \
+                w.astype(dtype)
+            size = bits.dtype.itemsize
+            mem = b.alloc(bits.nbytes + 64)
+            b.write(mem, size, np.ascontiguousarray(bits).view(np.uint8))
+            off = hip.HipbBuf(mem.contents.ptr + size, bits.nbytes, dt, b"shifted")
+            got = tokens(hip.Mem(off))
+            a.vw = aligned
+            b.release(mem)
+            if dt == hip.F16:   # small weights lose bits in half
+                assert np.abs(got - want).max() <= 2e-3
+            else:
+                assert np.array_equal(got, want), dt
+    finally:
+        d.free()
+        b.free()
