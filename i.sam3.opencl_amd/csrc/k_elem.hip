@@ -214,8 +214,8 @@ __global__ __launch_bounds__(256) void k_layernorm_w(
  * block's keys + PE in one pass over memory instead of three launches that
  * each read and write the map (32 prompts at 72 x 72, layer 0: 97 us against
  * 220).
- * Bound by memory. The arithmetic is k_layernorm_w's. */
-__global__ __launch_bounds__(256) void k_keys_norm(const float *__restrict__ X,
+ * Bound by memory. The arithmetic is k_layernorm_w's. Y may be X. */
+__global__ __launch_bounds__(256) void k_keys_norm(const float *X,
                                                    const float *__restrict__ add,
                                                    const float *__restrict__ g,
                                                    const float *__restrict__ bt, float eps,
