@@ -620,39 +620,66 @@ void *hipb_scratch(struct hipb_backend *b, size_t n)
     return b->scratch;
 }
 
-/* Workspace of the exact path's GEMM (its split operands): at least n
- * bytes, or NULL (the product then does without) when n is 0, when it cannot
- * be had, or while the caller captures the stream: only the library's own
- * graphs (b->capture), which run on this stream alone, may hold it, and they
- * may not grow it. It grows to at least twice its size and an outgrown one is
- * kept until hipb_free, since a graph may hold its address. */
+/* Workspace of the exact path's products and attention (their split
+ * operands): at least n bytes, or NULL (they then do without) when n is 0 or
+ * past GEMM_WS_MAX, when it cannot be had, or while the caller captures the
+ * stream: only the library's own graphs (b->capture), which run on this stream
+ * alone, may hold it, and they may not grow it. It grows to twice its size, or
+ * to n where that cannot be had; an outgrown one that a graph of the library
+ * was captured with is kept until hipb_free, any other is freed. After a
+ * failed allocation the next GEMM_WS_RETRY requests do without. */
+#define GEMM_WS_MIN ((size_t)32 << 20)
+#define GEMM_WS_MAX ((size_t)8 << 30)
+#define GEMM_WS_RETRY 64
+
 void *hipb_gemm_ws(struct hipb_backend *b, size_t n)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     const int cap = (int)(sizeof(b->gemm_ws) / sizeof(b->gemm_ws[0]));
-    size_t want = n;
+    size_t want = 2 * b->gemm_ws_bytes;
     void *p = NULL;
 
-    if (n == 0)
+    if (n == 0 || n > GEMM_WS_MAX)
         return NULL;
     if (!b->capture &&
         (hipStreamIsCapturing((hipStream_t)b->stream, &st) != hipSuccess ||
          st != hipStreamCaptureStatusNone))
         return NULL;
-    if (b->gemm_ws_count > 0 && n <= b->gemm_ws_bytes)
+    if (b->gemm_ws_count > 0 && n <= b->gemm_ws_bytes) {
+        b->gemm_ws_held |= b->capture;
         return b->gemm_ws[b->gemm_ws_count - 1];
-    if (b->capture || b->gemm_ws_count == cap)
+    }
+    if (b->capture)
         return NULL;
-    if (want < 2 * b->gemm_ws_bytes)
-        want = 2 * b->gemm_ws_bytes;
-    if (want < ((size_t)32 << 20))
-        want = (size_t)32 << 20;
+    if (b->gemm_ws_skip > 0) {
+        b->gemm_ws_skip--;
+        return NULL;
+    }
+    if (b->gemm_ws_count > 0 && !b->gemm_ws_held) {
+        hipStreamSynchronize((hipStream_t)b->stream);
+        hipFree(b->gemm_ws[--b->gemm_ws_count]);
+        b->gemm_ws_bytes = 0;
+    }
+    if (b->gemm_ws_count == cap)
+        return NULL;
+    if (want < GEMM_WS_MIN)
+        want = GEMM_WS_MIN;
+    if (want > GEMM_WS_MAX)
+        want = GEMM_WS_MAX;
+    if (want < n)
+        want = n;
     if (hipMalloc(&p, want) != hipSuccess) {
         (void)hipGetLastError();
-        return NULL;
+        want = n;
+        if (hipMalloc(&p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            b->gemm_ws_skip = GEMM_WS_RETRY;
+            return NULL;
+        }
     }
     b->gemm_ws[b->gemm_ws_count++] = p;
     b->gemm_ws_bytes = want;
+    b->gemm_ws_held = 0;
     return p;
 }
 

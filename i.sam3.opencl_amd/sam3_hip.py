@@ -76,6 +76,8 @@ class HipbBackend(ctypes.Structure):
                 ("gemm_ws", ctypes.c_void_p * 20),
                 ("gemm_ws_count", ctypes.c_int),
                 ("gemm_ws_bytes", ctypes.c_size_t),
+                ("gemm_ws_held", ctypes.c_int),
+                ("gemm_ws_skip", ctypes.c_int),
                 ("capture", ctypes.c_int)]
 
 

@@ -92,11 +92,14 @@ struct hipb_backend {
     void *stage[2];
     void *stage_ev[2];
     int stage_next;
-    /* Workspaces of the exact path's GEMM, each at least twice the one
-     * before; the last is in use, of gemm_ws_bytes. */
+    /* Workspaces of the exact path's products and attention: the last is in
+     * use, of gemm_ws_bytes; the others, and it where gemm_ws_held is set,
+     * are held by graphs of the library. gemm_ws_skip: requests to go before
+     * an allocation that failed is tried again. */
     void *gemm_ws[20];
     int gemm_ws_count;
     size_t gemm_ws_bytes;
+    int gemm_ws_held, gemm_ws_skip;
     int capture; /* the library is capturing a graph of its own */
 };
 
@@ -261,7 +264,8 @@ struct opnd bmat(hipb_mem buf, long off, int ld, long s0, long s1); /* ops.h:49 
  * contract sam3_kernels.cl:57-69). A and C are float (C may be bf16 and
  * A bf16 with precision=bf16); B may be half or bf16 weights. R may
  * alias C. Float products of large matrices use a workspace of the backend
- * that grows on demand, except while the caller captures the stream. */
+ * that grows on demand, up to 8 GiB, except while the caller captures the
+ * stream (the same bits at less speed). */
 void gemm(struct sam_model *m, int M, int N, int K, struct opnd A,
           struct opnd B, int transb, struct opnd C, int nb, int nb1,
           hipb_mem bias, hipb_mem R, long roff, float alpha, int act);
@@ -344,7 +348,9 @@ void mha_noalloc(struct sam_model *m, int P, int Nq, int Nk, int dint,
  * apply unchanged. rope (NULL for none) rotates Q and K rows at position
  * i % npos of the unit. With precision=bf16 the product runs on bf16
  * MFMA with f32 accumulation; otherwise it is a float product (f32 MFMA,
- * or operands split exactly into bf16 pieces for larger problems). Replaces the
+ * or operands split exactly into bf16 pieces for larger problems, in the
+ * backend's workspace; while the caller captures the stream, or without
+ * memory for it, the f32 MFMA: results that differ by rounding). Replaces the
  * gemm -> softmax_rows -> gemm loop of sam3_model.c:1000-1013. */
 void attn_fused(struct sam_model *m, int N, int nb, int nb1, struct opnd Q,
                 struct opnd K, struct opnd V, struct opnd O, hipb_mem rope,
