@@ -261,3 +261,74 @@ def test_trunk_graph_replay(hip, be, orc):
     be.release(out)
     be.release(other)
     m.free()
+
+
+def test_trunk_graph_keeps_its_workspace(hip, orc):
+    """fp32: the captured trunk's products hold the backend's workspace; a
+    larger product outgrows it, and replays (several, with eager work and
+    synchronisations between them) still equal the kernel-by-kernel run bit
+    for bit."""
+    grid, ps, E, heads, mlp = 40, 4, 1024, 16, 1024
+    b = hip.Backend(precision="fp32")
+    img, pe_w, pos, lnpw, lnpb, blocks = bc.trunk_case(97, grid, ps, E, mlp, [0])
+    m = hip.Model(b, grid=grid, embed=E, heads=heads,
+                  blocks=[upload_block(hip, b, w) for w in blocks], mlp=mlp)
+    try:
+        m.m.patch = ps
+        m.m.pe_w = b.upload_weight(pe_w)
+        m.m.pos, m.m.lnpw, m.m.lnpb = b.upload(pos), b.upload(lnpw), b.upload(lnpb)
+        m.m.rope_glob = b.upload(orc.rope_table(grid))
+
+        def run():
+            hip.sam_encode_trunk(m, img)
+            b.finish()
+            return b.read(m.m.x, grid * grid * E).copy()
+
+        eager = run()
+        hip.sam_trunk_graph(m)
+        assert m.m.trunk_exec and b._b.gemm_ws_held and b._b.gemm_ws_count == 1
+        assert np.array_equal(run(), eager)
+        big, w = b.alloc(4 * 12000 * 1024), b.alloc(4 * 8192 * 1024)
+        out = b.alloc(4 * 12000 * 8192)
+        hip.linear(m, 12000, 1024, 8192, big, 0, w, None, out, 0)
+        assert b._b.gemm_ws_count == 2 and not b._b.gemm_ws_held
+        for _ in range(4):
+            assert np.array_equal(run(), eager)
+            hip.linear(m, 12000, 1024, 8192, big, 0, w, None, out, 0)
+            b.finish()
+        assert m.m.trunk_exec
+    finally:
+        m.free()
+        b.free()
+
+
+def test_projection_of_tokens_in_row_chunks(hip, orc):
+    """fp32, a windowed block whose token rows are packed in two chunks (43520
+    of 43681 rows of 2048): the block's output (its MLP adds nothing) equals
+    the projection of all window rows and the unpartition, bit for bit."""
+    grid, E, heads, ws, mlp = 209, 2048, 32, 24, 64
+    b = hip.Backend(precision="fp32")
+    g = np.random.default_rng(98)
+    w = {k: g.uniform(-0.04, 0.04, s).astype(np.float32) for k, s in (
+        ("qkvw", (3 * E, E)), ("qkvb", 3 * E), ("projw", (E, E)), ("projb", E),
+        ("l1w", (mlp, E)), ("l1b", mlp))}
+    w.update(n1w=np.ones(E, np.float32), n1b=np.zeros(E, np.float32),
+             n2w=np.ones(E, np.float32), n2b=np.zeros(E, np.float32),
+             l2w=np.zeros((E, mlp), np.float32), l2b=np.zeros(E, np.float32), window=ws)
+    blk = upload_block(hip, b, w)
+    m = hip.Model(b, grid=grid, embed=E, heads=heads, blocks=[blk], mlp=mlp)
+    try:
+        m.m.rope_win = b.upload(orc.rope_table(ws))
+        x = g.standard_normal((grid * grid, E), dtype=np.float32)
+        b.write(m.m.x, 0, x)
+        hip.vit_block(m, blk)
+        got = b.read(m.m.x, grid * grid * E).copy()
+        b.write(m.m.x, 0, x)
+        hip.vit_attention(m, blk)
+        nwx = -(-grid // ws)
+        hip.linear(m, nwx * nwx * ws * ws, E, E, m.m.attn, 0, blk.projw, blk.projb, m.m.tmp, 0)
+        hip.window_unpartition_add(m, m.m.x, m.m.tmp, grid, E, ws, nwx)
+        assert np.array_equal(got, b.read(m.m.x, grid * grid * E))
+    finally:
+        m.free()
+        b.free()

@@ -28,13 +28,15 @@ def be(hip):
 
 
 def ms(be, call):
-    """Time of the third call in a row, by events."""
-    for _ in range(2):
-        call()
-    be.finish()
-    be.timer_start()
+    """The fastest of five calls, by events."""
     call()
-    return be.timer_stop()
+    best = 1e9
+    for _ in range(5):
+        be.finish()
+        be.timer_start()
+        call()
+        best = min(best, be.timer_stop())
+    return best
 
 
 # Packed operands; split while staged (float and K x N operand); f32 MFMA.
@@ -135,14 +137,16 @@ def decoder(hip, be, G, P, emb, w, s0):
         dec.set_image(emb, s0, g.standard_normal((4 * G * G, 64)).astype(np.float32))
         pts = g.uniform(0, 14 * G, (P, 2)).astype(np.float32)
         dec.decode(pts)
-        hip.prof_reset()
-        be.set_profile(True)
-        try:
-            dec.decode(pts)
-        finally:
-            be.set_profile(False)
-        t = [r for r in hip.prof_table() if r[0] == "upscale2"]
-        return dec.lowres(P).copy(), t[0][1]
+        t = 1e9
+        for _ in range(4):
+            hip.prof_reset()
+            be.set_profile(True)
+            try:
+                dec.decode(pts)
+            finally:
+                be.set_profile(False)
+            t = min([t] + [r[1] for r in hip.prof_table() if r[0] == "upscale2"])
+        return dec.lowres(P).copy(), t
     finally:
         dec.free()
         model.free()

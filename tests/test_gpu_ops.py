@@ -518,7 +518,7 @@ def us(be, call):
 @pytest.mark.parametrize("M,N,K,transb,nb", [(16, 16, 16, 0, 1000), (64, 64, 64, 0, 1000),
                                              (16, 64, 32, 0, 777)])
 def test_gemm_many_tiny_products(hip, be, M, N, K, transb, nb):
-    """A thousand products of a tile each cost at most three times one (they
+    """A thousand products of a tile each cost at most four times one (they
     fit the chip at once), and are right."""
     m = model(hip, be)
     g = rng(M + nb)
@@ -534,7 +534,7 @@ def test_gemm_many_tiny_products(hip, be, M, N, K, transb, nb):
     want = A.astype(np.float64) @ B.astype(np.float64)
     assert rel_l2(be.read(dC).reshape(nb, M, N), want) <= (np.sqrt(K) + 2) * 2.0 ** -24
     print("%d x %d x %d: one %.1f us, %d %.1f us" % (M, N, K, one, nb, many))
-    assert many <= 3 * one
+    assert many <= 4 * one
 
 
 @pytest.mark.parametrize("n,K,nb", [(576, 64, 144), (196, 64, 256), (256, 128, 64)])
@@ -565,3 +565,77 @@ def test_gemm_batch_costs_what_its_size_does(hip, be, n, K, nb):
                                   hip.mat(dC, 0, n)))
     print("%d x %d x %d x %d: %.1f us, as one product %.1f us" % (nb, n, n, K, batch, one))
     assert batch <= 1.8 * one
+
+
+def test_gemm_packed_row_chunks(hip, be):
+    """A product whose rows are packed in two chunks (1280 rows of K = 65536
+    fill the 512 MiB of pieces): rows around the seam and at the end against
+    float64, with bias and residual."""
+    M, N, K = 1400, 1024, 65536
+    m = model(hip, be)
+    g = rng(70)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    B = g.standard_normal((N, K), dtype=np.float32)
+    bias = g.standard_normal(N, dtype=np.float32)
+    C0 = 100 * g.standard_normal((M, N), dtype=np.float32)
+    dA, dB, dv, dC = be.upload(A), be.upload(B), be.upload(bias), be.upload(C0)
+    try:
+        hip.gemm(m, M, N, K, hip.mat(dA, 0, K), hip.mat(dB, 0, K), 1, hip.mat(dC, 0, N), 1, 1,
+                 dv, dC, 0, 0.5)
+        assert be._b.gemm_ws_bytes >= 864 << 20
+        got = be.read(dC).reshape(M, N)
+    finally:
+        for x in (dA, dB, dv, dC):
+            be.release(x)
+    rows = np.array([0, 31, 1247, 1278, 1279, 1280, 1281, 1311, 1312, 1398, 1399])
+    want = 0.5 * (A[rows].astype(np.float64) @ B.T.astype(np.float64)) + bias + C0[rows]
+    assert rel_l2(got[rows] - C0[rows], want - C0[rows]) <= (np.sqrt(K) + 2) * 2.0 ** -24
+
+
+def test_callers_capture(hip, be):
+    """A large product and a large attention while the caller captures the
+    stream: no workspace is used or grown; the product's replays have the eager
+    call's bits, the attention's (f32 MFMA there) agree to rounding. Every
+    replay is checked, eager work and a synchronisation between them."""
+    import ctypes
+    import os
+    rt = ctypes.CDLL(os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib",
+                                  "libamdhip64.so"))
+    vp = ctypes.c_void_p
+    m = hip.Model(be, embed=1024, heads=16)
+    g = rng(71)
+    M, N, K, T = 2500, 1030, 512, 1601
+    A, B = (be.upload(g.standard_normal(s, dtype=np.float32)) for s in ((M, K), (N, K)))
+    qkv = be.upload(g.standard_normal((T, 3072), dtype=np.float32))
+    C, O = be.alloc(M * N * 4), be.alloc(T * 1024 * 4)
+
+    def calls():
+        hip.linear(m, M, K, N, A, 0, B, None, C, 0)
+        hip.attn_fused(m, T, 16, 16, hip.bmat(qkv, 0, 3072, 0, 64),
+                       hip.bmat(qkv, 1024, 3072, 0, 64), hip.bmat(qkv, 2048, 3072, 0, 64),
+                       hip.bmat(O, 0, 1024, 0, 64))
+
+    calls()
+    want = be.read(C).copy(), be.read(O).copy()
+    ws = be._b.gemm_ws_count, be._b.gemm_ws_bytes
+    stream, graph, run = vp(be._b.stream), vp(), vp()
+    assert rt.hipStreamBeginCapture(stream, 2) == 0   # relaxed
+    try:
+        calls()
+    finally:
+        assert rt.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert (be._b.gemm_ws_count, be._b.gemm_ws_bytes) == ws and not be._b.gemm_ws_held
+    assert rt.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    try:
+        for _ in range(4):
+            for x in (C, O):
+                be.write(x, 0, np.zeros(x.contents.bytes // 4, np.float32))
+            assert rt.hipGraphLaunch(run, stream) == 0
+            be.finish()
+            assert np.array_equal(be.read(C), want[0])
+            assert rel_l2(be.read(O), want[1]) <= 2e-6
+            hip.add_bcast(m, C, C, C, M * N, M * N)
+            be.finish()
+    finally:
+        rt.hipGraphExecDestroy(run)
+        rt.hipGraphDestroy(graph)
