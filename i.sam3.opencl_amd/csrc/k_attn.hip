@@ -586,9 +586,9 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
 /* The exact path of larger problems: K, V and Q, scaled by SPLIT_SCALE, as
  * three bf16 pieces each (exactly the float, split4), and the weights P too
  * (what falls out of bf16's range is below 2^-133 of weights whose sum is
- * 2^-64 at least), six piece products per product on v_mfma_f32_32x32x16_bf16 with f32 accumulation, the three below
- * 2^-24 of it dropped: what the f32 MFMA of k_attn_f32 forms at a sixteenth
- * of the rate. K (rotated) and V^T are split once per call by
+ * 2^-64 at least), six piece products per product on
+ * v_mfma_f32_32x32x16_bf16 with f32 accumulation, the three below 2^-24 of it
+ * dropped: what the f32 MFMA of k_attn_f32 forms at a sixteenth of the rate. K (rotated) and V^T are split once per call by
  * k_kv_split into MFMA fragments, which this kernel copies HBM -> LDS
  * asynchronously, a 32-key block ahead; Q is split into registers; the
  * weights come out of exact_softmax, k_attn_f32's, and meet V^T from the
@@ -597,15 +597,16 @@ __global__ __launch_bounds__(256) void k_attn_f32(attn_desc d, float *__restrict
  * Bound by the sum of its MFMA time (48 per 32-key block and wave at head
  * width 64, 1536 cycles) and its VALU time (about 210 instructions, 88 of
  * them splitting the weights), which do not overlap on this chip; three waves
- * per SIMD. 16 heads x 64, packing included, against k_attn_f32: 5184 x 5184
- * 979 -> 519 us (212 TFLOP/s), 2600 x 2600 257 -> 150, 800 x 800 45 -> 37; 8 x
- * 32: 5184 x 5184 276 -> 163. The error against 64 bits is lower at every size
+ * per SIMD (four at head width 32). 16 heads x 64, packing included, against
+ * k_attn_f32: 5184 x 5184 979 -> 519 us (212 TFLOP/s), 2600 x 2600 257 -> 150,
+ * 800 x 800 45 -> 36; 8 x 32: 5184 x 5184 276 -> 163. The error against 64 bits is lower at every size
  * measured (5184 keys: 1.15e-6 against 1.34e-6).
  *
  * A non-finite operand, or one past 2^103, makes every result it enters NaN,
- * a score past 2^80 is infinite; a wave with such a query forms its part again from the float operands on the f32 MFMA
- * (attn_wave_f32) and takes those queries from there, so infinities and NaN
- * travel as in k_attn_f32, at a few times its cost. */
+ * a score past 2^80 is infinite; a wave with such a query forms its part
+ * again from the float operands on the f32 MFMA (attn_wave_f32) and takes
+ * those queries from there, so infinities and NaN travel as in k_attn_f32
+ * (1601 x 1601, 16 heads, one NaN key: 245 us against 78). */
 
 /* Bytes of a key block's fragments: K [HD / 16][3], then V^T [HD / 32][2]
  * [3], 1 KiB each. */

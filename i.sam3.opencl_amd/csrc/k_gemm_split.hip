@@ -151,11 +151,11 @@ __device__ __forceinline__ void store_blocks(const gemm_desc &d, f32x16 (&acc)[N
  * after go out: one barrier per step.
  *
  * Bound by issue: a split costs 22 VALU instructions per four floats, and on
- * this chip VALU and MFMA time add up rather than overlap (128 x 64 tiles:
- * 31 % and 41 % of the SIMD cycles), so it is used where a float meets few
- * columns and splitting it in a pass of its own would cost more: the decoder's
- * image tokens, 331776 x 128 x 256, 215 us against 293 by k_gemm_f32; 165888
- * rows 93 us, 165 with the pass. */
+ * this chip VALU and MFMA time add up rather than overlap (165888 x 128 x
+ * 256: 40 % and 30 % of the SIMD cycles, the rest waits), so it is used where
+ * a float meets few columns and splitting it in a pass of its own would cost
+ * more: the decoder's image tokens, 331776 x 128 x 256, 189 us against 254 by
+ * k_gemm_f32; 165888 rows 87 us, 168 with the pass. */
 template <int BM, int BN, int WM, int WN, int BDT, bool TRANSB>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(gemm_desc d)
 {
@@ -366,15 +366,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 1) void k_gemm_split(ge
 /* ------------------------------------------------------------ packed */
 
 /* Large products split their operands in a pass of their own (k_split_pack:
- * 10 bytes moved per element, 15-60 us for the trunk's), so that the K loop
+ * 10 bytes moved per element, 12-40 us for the trunk's), so that the K loop
  * is MFMAs, fragment reads and asynchronous copies only (k_gemm_frag). At
- * 5184 rows, pass included, against k_gemm_f32: 1024 -> 3072 168 against 311
- * us (194 TFLOP/s), 1024 -> 4096 243 against 454, 4096 -> 1024 287 against 682,
- * 1024 -> 1024 87 against 188; half weights 142, 202, 243 and 75 us. (On a
- * slower machine against the split while staging: 190 / 251, 273 / 323, 295 /
- * 324, 81 / 87 us.) What bounds it now is the MFMA rate under its own power:
- * 186 TFLOP/s of six products are 1120 TFLOP/s of bf16, 77 % of what the
- * platform's 8192^3 bf16 product reaches.
+ * 5184 rows, pass included, against k_gemm_f32 and against the split while
+ * staging: 1024 -> 3072 158 us, 301, 215 (206 TFLOP/s); 1024 -> 4096 232, 446,
+ * 289; 4096 -> 1024 280, 672, 310; 1024 -> 1024 78, 180, 85; half weights 135,
+ * 190, 237 and 68 us. What bounds it is the MFMA rate under its own power: the
+ * MFMA unit is busy 70 % of the cycles, 225 TFLOP/s of six products are 1350
+ * TFLOP/s of bf16, 93 % of what the platform's 8192^3 bf16 product reaches.
  */
 
 /* An operand split once into MFMA fragments: [32-row block][16-k step]
@@ -480,7 +479,9 @@ __device__ __forceinline__ void gs_vmwait0()
  * one of two slots, a step ahead. The loop is one basic block (the step count
  * is even; copies past the end repeat the last step into a slot that no one
  * reads): with a branch in it the compiler kept a second copy of the
- * accumulators, 128 moves per step (145 against 180 TFLOP/s). */
+ * accumulators, 128 moves per step (145 against 180 TFLOP/s). Registers are
+ * kept to what two 256 x 128 workgroups on a CU leave (5184 x 4096 x 1024 with
+ * GELU: 250 us, 259 with one). */
 template <int BM, int BN, int WM, int WN, int BDT, bool WIN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, BM * BN >= 256 * 128 ? 4 : 1) void
 k_gemm_frag(gemm_desc d, const char *pa, const char *pb)
@@ -729,9 +730,9 @@ static long gs_tiles(const gemm_desc *d, int bm, int bn)
 }
 
 /* Small: at most one 64 x 64 tile per two CUs, where a staged tile's K loop
- * is all latency (400 x 1024 x 1024, 112 tiles: 25 us against 30; 1000 x 1024
- * x 1024, 256 tiles: 49 against 31; 1000 x 300 x 4096, 80 tiles: 73 against
- * 137). Of a batch only products of up to three tiles or 32 rows or columns:
+ * is all latency (400 x 1024 x 1024, 112 tiles: 27 us against 28; 1000 x 1024
+ * x 1024, 256 tiles: 49 against 30; 1000 x 300 x 4096, 80 tiles: 75 against
+ * 117). Of a batch only products of up to three tiles or 32 rows or columns:
  * above that a batch fills the chip and the small kernel, which reads its
  * operands once per 16 columns, is bound by the caches (576 x 576 x 64: 16
  * products 34 us against 15, 144 272 against 80; 64 products of 256 x 256 x
@@ -754,10 +755,11 @@ static int gs_chunk(const gemm_desc *d)
     return rows < 256 ? 256 : rows < d->M ? (int)rows : d->M;
 }
 
-/* Packing pays when what it saves, 4.6e-15 s per product (125 against 175
- * TFLOP/s), exceeds its 2.2e-12 s per element and a launch: at equal sides
- * about 1000 x 1000. A product over the tokens of windows replaces one over
- * all window rows, so it is packed where that was. */
+/* Packing pays when what it saves, about 4.6e-15 s per product (125 against
+ * 175 TFLOP/s), exceeds its 2.2e-12 s per element and a launch: 1000 x 1024 x
+ * 1024 30 us staged, 37 packed; 1400 rows 42 and 44; 5184 rows 85 and 78. A
+ * product over the tokens of windows replaces one over all window rows, so
+ * it is packed where that was. */
 extern "C" size_t gemm_split_ws(const gemm_desc *d)
 {
     const double wr = (double)d->win_nwx * d->win_ws, M = d->win_ws > 0 ? wr * wr : d->M, N = d->N, K = d->K;
@@ -861,9 +863,9 @@ static int launch_packed(const gemm_desc *d, void *ws, hipStream_t s)
 template <int BDT, bool TRANSB>
 static int launch_staged(const gemm_desc *d, hipStream_t s)
 {
-    /* 128 x 64 tiles when they give every CU two (165888 x 128 x 256: 93
-     * against 95 us; 5184 x 1024 x 1024: 87 against 94), else 64 x 64 (5184 x
-     * 128 x 256: 11 against 17 us). */
+    /* 128 x 64 tiles when they give every CU two (331776 x 128 x 256: 189 us
+     * against 202; 165888 rows 87 against 90), else 64 x 64 (5184 x 128 x 256:
+     * 11 us against 16). */
     const bool big = gs_tiles(d, 128, 64) * d->nb >= 2L * dev_cu_count();
     const long tiles = big ? gs_tiles(d, 128, 64) : gs_tiles(d, 64, 64);
     const long grid =
